@@ -112,6 +112,7 @@ struct Args {
     const uint8_t* sa;  // swizzled E8M0, [roundup(M,128), ncb*4]
     const uint8_t* sb;
     const void* bias;
+    int bias_code;      // dtype code of bias
     void* out;
     int M, N, K;
     int ncb;               // scale column blocks: ceil(K/32/4)
@@ -290,8 +291,8 @@ __device__ __forceinline__ float bias_at(const void* bias, int n) {
 // array and writes staged data into the other, so the compiler knows they never alias
 // and may interleave the two freely; within an array, per-lane addresses of different
 // buffers differ only by immediates.
-template <int OUT, int BIAS, bool UNIT, int NW, bool SPLIT = false>
-__device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds01, uint8_t* lds23) {
+template <int OUT, bool BIAS, bool UNIT, int NW, bool SPLIT = false>
+__device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds01, uint8_t* lds23, float* lds_bias) {
     constexpr int TBN = 64 * NW;  // tile width along n
     constexpr int PB = TBN / 32;  // staged weight loads per lane per pair of stages
     constexpr int SLOTS = 4 * NW;  // MFMAs per wave per stage
@@ -321,6 +322,9 @@ __device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds01
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
     const int wm = wave & 1, wn = wave >> 1;
     const int half = lane >> 5, r32 = lane & 31;
+
+    uint32_t bias_bits = 0;
+    if constexpr (BIAS) bias_bits = load_bias_bits(p.bias, p.bias_code, n0 + tid, p.N);
 
     const Loader LB = make_loader(p.b + static_cast<int64_t>(n0) * p.K, min(TBN, p.N - n0), p.K, wave, lane, TBN / 4);
     const Loader LA = make_loader(p.a + static_cast<int64_t>(m0) * p.K, min(BM, p.M - m0), p.K, wave, lane);
@@ -457,6 +461,7 @@ __device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds01
         if constexpr (DS) load_dscales(t0 / 2);
         load_pair(LA, XA, (t0 + 2) * BK, kend);
         load_b(t0 + 2);
+        if constexpr (BIAS) lds_bias[tid] = bias_value(bias_bits, p.bias_code);
         store_a(B0{}, B1{});
         store_pair<PB>(LB, XB, buf(B0{}), buf(B1{}));
         store_pair(LA, XA, buf(B2{}) + TILE, buf(B3{}) + TILE);
@@ -508,12 +513,14 @@ __device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds01
     // n = 8*g + 4*half (+0..3) of weight tile i.
     const float alpha = UNIT ? p.tsa[0] * p.tsb[0] : 1.0f;
     // With neither a tensor scale nor a bias the accumulator is the output value.
-    constexpr bool ARITH = UNIT || BIAS >= 0;
-    auto value = [&](float a, int n) {
+    constexpr bool ARITH = UNIT || BIAS;
+    auto value = [&](float a, float b) {
         if constexpr (UNIT) a *= alpha;
-        if constexpr (BIAS >= 0) a += n < p.N ? bias_at<BIAS>(p.bias, n) : 0.0f;
+        if constexpr (BIAS) a += b;
         return a;
     };
+    // the bias of the 4 columns from nl on (nl a multiple of 4)
+    auto bias4 = [&](int nl) { return BIAS ? *reinterpret_cast<const float4*>(lds_bias + nl) : float4{}; };
     if constexpr (OUT != CKH_F32) {
         // 16-bit output: stage the tile in LDS as 256 rows of 512 bytes, the 64-row slab
         // q in buffer q, converting two values per instruction.  Then each wave stores
@@ -521,17 +528,17 @@ __device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds01
         // (NW = 4) or four 256-byte rows (NW = 2).
         auto slab = [&](int q) -> uint8_t* { return (q < 2 ? lds01 : lds23) + (q & 1) * BUF; };
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            uint8_t* rowp = slab(wm * 2 + (j >> 1)) + ((j & 1) * 32 + r32) * EPI_ROW;
+        for (int i = 0; i < NW; ++i) {
 #pragma unroll
-            for (int i = 0; i < NW; ++i) {
+            for (int g = 0; g < 4; ++g) {
+                const int nl = wn * 32 * NW + i * 32 + 8 * g + 4 * half;
+                const float4 b = bias4(nl);
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int nl = wn * 32 * NW + i * 32 + 8 * g + 4 * half;
-                    const int n = n0 + nl;
+                for (int j = 0; j < 4; ++j) {
+                    uint8_t* rowp = slab(wm * 2 + (j >> 1)) + ((j & 1) * 32 + r32) * EPI_ROW;
                     const v16f& a = acc[i][j];
-                    const uint32_t w0 = pack2<OUT, ARITH>(value(a[4 * g], n), value(a[4 * g + 1], n + 1));
-                    const uint32_t w1 = pack2<OUT, ARITH>(value(a[4 * g + 2], n + 2), value(a[4 * g + 3], n + 3));
+                    const uint32_t w0 = pack2<OUT, ARITH>(value(a[4 * g], b.x), value(a[4 * g + 1], b.y));
+                    const uint32_t w1 = pack2<OUT, ARITH>(value(a[4 * g + 2], b.z), value(a[4 * g + 3], b.w));
                     *reinterpret_cast<uint2*>(rowp + nl * 2) = make_uint2(w0, w1);
                 }
             }
@@ -568,9 +575,9 @@ __device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds01
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const int n = n0 + wn * 32 * NW + i * 32 + 8 * g + 4 * half;
-                    float v[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = value(acc[i][j][4 * g + e], n + e);
+                    const float4 b = bias4(n - n0);
+                    const float v[4] = {value(acc[i][j][4 * g], b.x), value(acc[i][j][4 * g + 1], b.y),
+                                        value(acc[i][j][4 * g + 2], b.z), value(acc[i][j][4 * g + 3], b.w)};
                     const int64_t idx = static_cast<int64_t>(m) * p.N + n;
                     if (n + 3 < p.N && (p.N & 3) == 0) {
                         store4<OUT>(p.out, idx, v);
@@ -652,13 +659,14 @@ __device__ __forceinline__ void prefetch_weight(const Args& p, int w) {
 // The dispatcher starts half-tile workgroups on CUs as their last full tile ends, so
 // the tail overlaps the uneven end of the previous round instead of waiting for a
 // second launch.  A grid of one round ends with the weight-prefetch workgroups.
-template <int OUT, int BIAS, bool UNIT>
+template <int OUT, bool BIAS, bool UNIT>
 __global__ __launch_bounds__(NT) void gemm_kernel(Args p) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds01[2 * BUF];
     __shared__ __attribute__((aligned(1024))) uint8_t lds23[2 * BUF];
+    __shared__ __attribute__((aligned(16))) float lds_bias[BIAS ? BN : 4];
     const int b = blockIdx.x;
-    if (b < p.n_full) gemm_tile<OUT, BIAS, UNIT, 4>(p, b, lds01, lds23);
-    else if (b < p.n_full + 2 * p.n_half) gemm_tile<OUT, BIAS, UNIT, 2>(p, b - p.n_full, lds01, lds23);
+    if (b < p.n_full) gemm_tile<OUT, BIAS, UNIT, 4>(p, b, lds01, lds23, lds_bias);
+    else if (b < p.n_full + 2 * p.n_half) gemm_tile<OUT, BIAS, UNIT, 2>(p, b - p.n_full, lds01, lds23, lds_bias);
     else prefetch_weight<UNIT>(p, b - p.n_full - 2 * p.n_half);
 }
 
@@ -669,7 +677,7 @@ template <bool UNIT, int NW>
 __global__ __launch_bounds__(NT) void gemm_split_kernel(Args p) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds01[2 * BUF];
     __shared__ __attribute__((aligned(1024))) uint8_t lds23[2 * BUF];
-    gemm_tile<CKH_F32, -1, UNIT, NW, true>(p, blockIdx.x, lds01, lds23);
+    gemm_tile<CKH_F32, false, UNIT, NW, true>(p, blockIdx.x, lds01, lds23, nullptr);
 }
 
 // Split-K, second launch: thread q adds float4 q % U of unit q / U (U = 4096 NW float4 of a
@@ -1006,19 +1014,15 @@ namespace {
 constexpr int kGemmSlots = 256;
 
 template <bool UNIT>
-void launch_grid(const mx::Args& p, unsigned wgs, int out_code, int bias_code, bool has_bias, hipStream_t st) {
-#define LAUNCH(O, B) hipLaunchKernelGGL((mx::gemm_kernel<O, B, UNIT>), dim3(wgs), dim3(mx::NT), 0, st, p)
-#define BY_BIAS(O)                                                     \
-    do {                                                               \
-        if (!has_bias) LAUNCH(O, -1);                                  \
-        else if (bias_code == CKH_F32) LAUNCH(O, CKH_F32);             \
-        else if (bias_code == CKH_F16) LAUNCH(O, CKH_F16);             \
-        else LAUNCH(O, CKH_BF16);                                      \
+void launch_grid(const mx::Args& p, unsigned wgs, int out_code, bool has_bias, hipStream_t st) {
+#define LAUNCH(O)                                                                                          \
+    do {                                                                                                   \
+        if (has_bias) hipLaunchKernelGGL((mx::gemm_kernel<O, true, UNIT>), dim3(wgs), dim3(mx::NT), 0, st, p); \
+        else hipLaunchKernelGGL((mx::gemm_kernel<O, false, UNIT>), dim3(wgs), dim3(mx::NT), 0, st, p);     \
     } while (0)
-    if (out_code == CKH_BF16) BY_BIAS(CKH_BF16);
-    else if (out_code == CKH_F16) BY_BIAS(CKH_F16);
-    else BY_BIAS(CKH_F32);
-#undef BY_BIAS
+    if (out_code == CKH_BF16) LAUNCH(CKH_BF16);
+    else if (out_code == CKH_F16) LAUNCH(CKH_F16);
+    else LAUNCH(CKH_F32);
 #undef LAUNCH
 }
 
@@ -1207,7 +1211,8 @@ int launch_gemm(mx::Args p, int out_code, int bias_code, bool has_bias, void* wo
     // found no idle CU would run after the tiles, for nothing)
     const int cus = device_cus();
     p.n_pref = wgs < cus ? cus - wgs : 0;
-    launch_grid<UNIT>(p, static_cast<unsigned>(wgs + p.n_pref), out_code, bias_code, has_bias, st);
+    p.bias_code = bias_code;
+    launch_grid<UNIT>(p, static_cast<unsigned>(wgs + p.n_pref), out_code, has_bias, st);
     return check_launch(UNIT ? "scaled_mm_fp8" : "scaled_mm_mxfp8");
 }
 

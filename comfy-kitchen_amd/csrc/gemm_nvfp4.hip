@@ -97,6 +97,7 @@ struct Args {
     const uint8_t* sb;
     const float* alpha;
     const void* bias;
+    int bias_code;  // dtype code of bias
     void* out;
     int M, N, K;  // K in elements
     int ncb;      // scale word columns: ceil(K/16/4)
@@ -219,8 +220,8 @@ __device__ __forceinline__ float bias_at(const void* bias, int n) {
 // NW: 32-column MFMA tiles per wave along n: 4 for 256 x 256 workgroup tiles, 2 for the
 // 256 x 128 column halves of a tile (each wave 128 x 64: 8 MFMAs per substep instead of
 // 16, with 6 of the 8 operand tiles decoded).
-template <int OUT, int BIAS, int NW, bool SPLIT = false>
-__device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds0, uint8_t* lds1) {
+template <int OUT, bool BIAS, int NW, bool SPLIT = false>
+__device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds0, uint8_t* lds1, float* lds_bias) {
     constexpr int TBN = 64 * NW;         // tile width along n
     constexpr int RPW = TBN / 4;         // weight rows loaded per wave
     constexpr int SLOTS = 4 * NW;        // MFMAs per wave per substep
@@ -246,6 +247,9 @@ __device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds0,
     const int wm = wave & 1, wn = wave >> 1;
     const int half = lane >> 5, r32 = lane & 31;
     const int Kb = p.K / 2;
+
+    uint32_t bias_bits = 0;
+    if constexpr (BIAS) bias_bits = load_bias_bits(p.bias, p.bias_code, n0 + tid, p.N);
 
     const Loader LB = make_loader(p.b + static_cast<int64_t>(n0) * Kb, min(TBN, p.N - n0), Kb, wave, lane, RPW);
     const Loader LA = make_loader(p.a + static_cast<int64_t>(m0) * Kb, min(BM, p.M - m0), Kb, wave, lane);
@@ -391,6 +395,7 @@ __device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds0,
     // prologue: groups 0 and 1 in flight, group 0 resident, stage 0 read and decoded
     issue_group(G0{}, gb);
     issue_group(G1{}, gb + 1);
+    if constexpr (BIAS) lds_bias[tid] = bias_value(bias_bits, p.bias_code);
     group_barrier<waitcnt_vm_lgkm0(NLD)>();
     for_each_index([&](auto i_c) { read_part(lds0, S0{}, i_c, R0); }, std::make_integer_sequence<int, NREAD>{});
     for_each_index([&](auto p_c) { decode_part(R0, K0{}, p_c, D0); }, std::make_integer_sequence<int, NDEC>{});
@@ -439,7 +444,9 @@ __device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds0,
     // Epilogue: lane holds out[m][n..n+3] for m = r32-th row of activation tile j and
     // n = 8*gg + 4*half (+0..3) of weight tile i; times alpha, plus bias.
     const float alpha = p.alpha[0];
-    auto value = [&](float a, int n) { return a * alpha + (n < p.N ? bias_at<BIAS>(p.bias, n) : 0.0f); };
+    auto value = [&](float a, float b) { return a * alpha + b; };
+    // the bias of the 4 columns from nl on (nl a multiple of 4), zeros without a bias
+    auto bias4 = [&](int nl) { return BIAS ? *reinterpret_cast<const float4*>(lds_bias + nl) : float4{}; };
     if constexpr (OUT != CKH_F32) {
         // Stage the 16-bit tile in LDS as 256 rows of EPI_ROW bytes (rows 0..127 in
         // buffer 0, 128..255 in buffer 1; the 520-byte pitch spreads a fragment's 32 rows
@@ -447,17 +454,17 @@ __device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds0,
         // one 512-byte row per instruction (full tiles) or two 256-byte rows (half tiles).
         auto row_ptr = [&](int r) -> uint8_t* { return r < 128 ? lds0 + r * EPI_ROW : lds1 + (r - 128) * EPI_ROW; };
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            uint8_t* rowp = row_ptr(wm * 128 + j * 32 + r32);
+        for (int i = 0; i < NW; ++i) {
 #pragma unroll
-            for (int i = 0; i < NW; ++i) {
+            for (int gg = 0; gg < 4; ++gg) {
+                const int nl = wn * 32 * NW + i * 32 + 8 * gg + 4 * half;
+                const float4 b = bias4(nl);
 #pragma unroll
-                for (int gg = 0; gg < 4; ++gg) {
-                    const int nl = wn * 32 * NW + i * 32 + 8 * gg + 4 * half;
-                    const int n = n0 + nl;
+                for (int j = 0; j < 4; ++j) {
+                    uint8_t* rowp = row_ptr(wm * 128 + j * 32 + r32);
                     *reinterpret_cast<uint2*>(rowp + nl * 2) =
-                        make_uint2(pack2<OUT>(value(acc[i][j][4 * gg], n), value(acc[i][j][4 * gg + 1], n + 1)),
-                                   pack2<OUT>(value(acc[i][j][4 * gg + 2], n + 2), value(acc[i][j][4 * gg + 3], n + 3)));
+                        make_uint2(pack2<OUT>(value(acc[i][j][4 * gg], b.x), value(acc[i][j][4 * gg + 1], b.y)),
+                                   pack2<OUT>(value(acc[i][j][4 * gg + 2], b.z), value(acc[i][j][4 * gg + 3], b.w)));
                 }
             }
         }
@@ -492,9 +499,9 @@ __device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds0,
 #pragma unroll
                 for (int gg = 0; gg < 4; ++gg) {
                     const int n = n0 + wn * 32 * NW + i * 32 + 8 * gg + 4 * half;
-                    float v[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = value(acc[i][j][4 * gg + e], n + e);
+                    const float4 b = bias4(n - n0);
+                    const float v[4] = {value(acc[i][j][4 * gg], b.x), value(acc[i][j][4 * gg + 1], b.y),
+                                        value(acc[i][j][4 * gg + 2], b.z), value(acc[i][j][4 * gg + 3], b.w)};
                     const int64_t idx = static_cast<int64_t>(m) * p.N + n;
                     if (n + 3 < p.N && (p.N & 3) == 0) {
                         store4<OUT>(p.out, idx, v);
@@ -509,13 +516,14 @@ __device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds0,
     }
 }
 
-template <int OUT, int BIAS>
+template <int OUT, bool BIAS>
 __global__ __launch_bounds__(NT) void gemm_kernel(Args p) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds0[GBUF];
     __shared__ __attribute__((aligned(1024))) uint8_t lds1[GBUF];
+    __shared__ __attribute__((aligned(16))) float lds_bias[BIAS ? BN : 4];
     const int b = blockIdx.x;
-    if (b < p.n_full) gemm_tile<OUT, BIAS, 4>(p, b, lds0, lds1);
-    else gemm_tile<OUT, BIAS, 2>(p, b - p.n_full, lds0, lds1);
+    if (b < p.n_full) gemm_tile<OUT, BIAS, 4>(p, b, lds0, lds1, lds_bias);
+    else gemm_tile<OUT, BIAS, 2>(p, b - p.n_full, lds0, lds1, lds_bias);
 }
 
 // Split-K, first launch: each workgroup one K range of one 256 x 256 tile (NW = 4) or
@@ -525,7 +533,7 @@ template <int NW>
 __global__ __launch_bounds__(NT) void gemm_split_kernel(Args p) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds0[GBUF];
     __shared__ __attribute__((aligned(1024))) uint8_t lds1[GBUF];
-    gemm_tile<CKH_F32, -1, NW, true>(p, blockIdx.x, lds0, lds1);
+    gemm_tile<CKH_F32, false, NW, true>(p, blockIdx.x, lds0, lds1, nullptr);
 }
 
 // Split-K, second launch: thread q adds float4 q % U of unit q / U (U = 4096 NW float4 of
@@ -1138,18 +1146,15 @@ extern "C" int ckh_scaled_mm_nvfp4(const void* a, const void* b, const void* sa,
     p.n_half = (tail > 0 && tail <= kNvHalfTail) ? tail : 0;
     p.n_full = tiles - p.n_half;
     dim3 grid(static_cast<unsigned>(p.n_full + 2 * p.n_half));
-#define LAUNCH(O, B) hipLaunchKernelGGL((nv::gemm_kernel<O, B>), grid, dim3(nv::NT), 0, st, p)
-#define BY_BIAS(O)                                         \
-    do {                                                   \
-        if (!bias) LAUNCH(O, -1);                          \
-        else if (bias_code == CKH_F32) LAUNCH(O, CKH_F32); \
-        else if (bias_code == CKH_F16) LAUNCH(O, CKH_F16); \
-        else LAUNCH(O, CKH_BF16);                          \
+    p.bias_code = bias_code;
+#define LAUNCH(O)                                                                                       \
+    do {                                                                                                \
+        if (bias) hipLaunchKernelGGL((nv::gemm_kernel<O, true>), grid, dim3(nv::NT), 0, st, p);         \
+        else hipLaunchKernelGGL((nv::gemm_kernel<O, false>), grid, dim3(nv::NT), 0, st, p);             \
     } while (0)
-    if (out_code == CKH_BF16) BY_BIAS(CKH_BF16);
-    else if (out_code == CKH_F16) BY_BIAS(CKH_F16);
-    else BY_BIAS(CKH_F32);
-#undef BY_BIAS
+    if (out_code == CKH_BF16) LAUNCH(CKH_BF16);
+    else if (out_code == CKH_F16) LAUNCH(CKH_F16);
+    else LAUNCH(CKH_F32);
 #undef LAUNCH
     return check_launch("scaled_mm_nvfp4");
 }
