@@ -24,6 +24,7 @@ __version__ = "0.1.0"
 __all__ = [
     "quantize_per_tensor_fp8",
     "dequantize_per_tensor_fp8",
+    "quantize_fp8_dynamic",
     "quantize_nvfp4",
     "quantize_nvfp4_dynamic",
     "dequantize_nvfp4",
@@ -63,6 +64,17 @@ def quantize_per_tensor_fp8(x: torch.Tensor, scale: torch.Tensor,
                             output_type: torch.dtype = torch.float8_e4m3fn) -> torch.Tensor:
     """FP8 quantize with one fp32 scale: fp8(clamp(x * (1/scale), +-max))."""
     return torch.ops.comfy_kitchen.quantize_fp8(x, scale, DTYPE_TO_CODE[output_type])
+
+
+def quantize_fp8_dynamic(x: torch.Tensor, divisor: float = 448.0,
+                         output_type: torch.dtype = torch.float8_e4m3fn) -> tuple[torch.Tensor, torch.Tensor]:
+    """quantize_per_tensor_fp8 with the scale amax(|x|) / divisor (in x's dtype) formed on the
+    device in the same call: returns (codes, 0-dim fp32 scale).
+
+    Not part of the reference's public API: it is the scale=None branch of the FP8 layout's
+    quantize (reference tensor/fp8.py:56-61) with the reduction fused into the quantize
+    launch.  The results equal amax_scale followed by quantize_per_tensor_fp8 bit for bit."""
+    return torch.ops.comfy_kitchen.quantize_fp8_dynamic(x, float(divisor), DTYPE_TO_CODE[output_type])
 
 
 def dequantize_per_tensor_fp8(x: torch.Tensor, scale: torch.Tensor,

@@ -31,6 +31,7 @@ __all__ = [
     "dequantize_mxfp8",
     "dequantize_nvfp4",
     "dequantize_per_tensor_fp8",
+    "quantize_fp8_dynamic",
     "quantize_mxfp8",
     "quantize_nvfp4",
     "quantize_nvfp4_dynamic",
@@ -63,6 +64,7 @@ SIGNATURES: dict[str, tuple] = {
     "ckh_scaled_mm_nvfp4_workspace_bytes": (_i64, [_i64] * 3),
     "ckh_amax_scale": (_i32, [_p, _i64, _i32, _f32, _p, _p, _u64]),
     "ckh_amax_scale_noalloc": (_i32, [_p, _i64, _i32, _f32, _p, _u64]),
+    "ckh_quantize_fp8_dynamic": (_i32, [_p, _f32, _p, _p, _i64, _i32, _i32, _p, _u64]),
     "ckh_quantize_nvfp4_dynamic": (_i32, [_p, _f32, _p, _p, _p, _i64, _i64, _i64, _i64, _f32, _i32, _i32, _p, _u64]),
 }
 ABI_VERSION = 8
@@ -188,6 +190,22 @@ def amax_scale(x: torch.Tensor, divisor: float) -> torch.Tensor:
         _call("ckh_amax_scale", x.data_ptr(), x.numel(), DTYPE_TO_CODE[x.dtype], float(divisor), out.data_ptr(),
               work.data_ptr(), _stream(x))
     return out
+
+
+def quantize_fp8_dynamic(x: torch.Tensor, divisor: float,
+                         output_type: torch.dtype = torch.float8_e4m3fn) -> tuple[torch.Tensor, torch.Tensor]:
+    """quantize_per_tensor_fp8 with the scale amax(|x|) / divisor formed on the device in the
+    same call: (codes, 0-dim fp32 scale), equal to amax_scale + quantize_per_tensor_fp8."""
+    x = x.contiguous()
+    if x.numel() == 0:
+        raise RuntimeError("quantize_fp8_dynamic: empty tensor")
+    out = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
+    scale = torch.empty((), dtype=torch.float32, device=x.device)
+    work = torch.empty(AMAX_WORKSPACE_BYTES // 4, dtype=torch.int32, device=x.device)
+    with _on_device(x):
+        _call("ckh_quantize_fp8_dynamic", x.data_ptr(), float(divisor), scale.data_ptr(), out.data_ptr(), x.numel(),
+              DTYPE_TO_CODE[x.dtype], DTYPE_TO_CODE[output_type], work.data_ptr(), _stream(x))
+    return out.view(output_type), scale
 
 
 # --------------------------------------------------------------------------- MXFP8
@@ -444,6 +462,7 @@ def _build_constraints() -> dict:
                                       output_type=ParamConstraint(dtypes=fp8)),
         "dequantize_per_tensor_fp8": fc(x=ParamConstraint(dtypes=fp8), scale=ParamConstraint(dtypes=floats, devices=frozenset({"cuda", "cpu"})),
                                         output_type=ParamConstraint(dtypes=floats)),
+        "quantize_fp8_dynamic": fc(x=ParamConstraint(dtypes=floats), output_type=ParamConstraint(dtypes=fp8)),
         "quantize_mxfp8": fc(x=ParamConstraint(dtypes=floats, shape_rules=two_d)),
         "dequantize_mxfp8": fc(qx=ParamConstraint(dtypes=frozenset({torch.float8_e4m3fn}),
                                                   shape_rules=two_d + (DivisibleBy(1, 32),)),

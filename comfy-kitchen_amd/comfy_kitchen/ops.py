@@ -51,6 +51,18 @@ def _(x, scale, output_dtype_code):
     return torch.empty_like(x, dtype=DTYPE_CODE_TO_DTYPE[output_dtype_code])
 
 
+@torch.library.custom_op("comfy_kitchen::quantize_fp8_dynamic", mutates_args=())
+def quantize_fp8_dynamic(x: torch.Tensor, divisor: float, output_dtype_code: int) -> tuple[torch.Tensor, torch.Tensor]:
+    return _dispatch("quantize_fp8_dynamic", x=x, divisor=divisor,
+                     output_type=DTYPE_CODE_TO_DTYPE[output_dtype_code])
+
+
+@quantize_fp8_dynamic.register_fake
+def _(x, divisor, output_dtype_code):
+    return (torch.empty_like(x, dtype=DTYPE_CODE_TO_DTYPE[output_dtype_code]),
+            torch.empty((), dtype=torch.float32, device=x.device))
+
+
 # ------------------------------------------------------------------------ NVFP4
 @torch.library.custom_op("comfy_kitchen::quantize_nvfp4", mutates_args=())
 def quantize_nvfp4(x: torch.Tensor, per_tensor_scale: torch.Tensor, epsilon: float,

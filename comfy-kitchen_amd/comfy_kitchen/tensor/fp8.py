@@ -39,8 +39,9 @@ class TensorCoreFP8Layout(QuantizedLayout):
         import comfy_kitchen as ck
 
         if scale is None or (isinstance(scale, str) and scale == "recalculate"):
-            # amax(|x|) / max in x's dtype, as one device-side reduction
-            scale = ck.amax_scale(tensor, torch.finfo(dtype).max)
+            # amax(|x|) / max in x's dtype, reduced on the device in the quantize call
+            qdata, scale = ck.quantize_fp8_dynamic(tensor, torch.finfo(dtype).max, dtype)
+            return qdata, cls.Params(scale=scale, orig_dtype=tensor.dtype, orig_shape=tuple(tensor.shape))
         if not isinstance(scale, torch.Tensor):
             scale = torch.tensor(scale)
         scale = scale.to(device=tensor.device, dtype=torch.float32)

@@ -28,7 +28,13 @@ namespace ckh {
 namespace am {
 
 constexpr int kThreads = 256;
-constexpr int kUnroll = 16;                // 16-byte loads in flight per thread
+constexpr int kUnroll = 16;                // 16-byte loads in flight per thread, large tensors
+// Below kSpreadBlocks workgroups' worth of work at kUnroll loads a thread, the tensor is
+// spread thinner, kUnrollSmall loads a thread: 256 x 3072 bf16 ran on 24 workgroups in 9.5 us
+// and 256 x 5120 on 40 in 9.7 us, waiting out the loads' issue on a few CUs; spread, the
+// NVFP4 dynamic quantize of 256 x 5120 takes 6 us less.
+constexpr int kUnrollSmall = 2;
+constexpr int kSpreadBlocks = 512;
 constexpr int kMaxBlocks = CKH_AMAX_WORKSPACE_BYTES / 4;  // one partial word per workgroup
 
 // |x| bits of 8 packed 16-bit values -> the largest, as fp32 bits
@@ -74,9 +80,9 @@ __device__ __forceinline__ uint32_t block_max(uint32_t m) {
 }
 
 // VEC: x is 16-byte aligned; chunks of 16 bytes, then a scalar tail.  Thread t reads
-// chunks t, t + stride, ... in batches of kUnroll, all of a batch's loads issued before
-// any is used.
-template <int IN, bool VEC>
+// chunks t, t + stride, ... in batches of U, all of a batch's loads issued before any is
+// used.
+template <int IN, bool VEC, int U>
 __global__ __launch_bounds__(kThreads) void amax_kernel(const void* __restrict__ x, int64_t n,
                                                         uint32_t* __restrict__ partial) {
     constexpr int PER = 16 / ElemSize<IN>::value;  // elements per 16-byte chunk
@@ -87,15 +93,15 @@ __global__ __launch_bounds__(kThreads) void amax_kernel(const void* __restrict__
     if constexpr (VEC) {
         const int64_t chunks = n / PER;
         const uint4* p = static_cast<const uint4*>(x);
-        for (int64_t c0 = tid; c0 < chunks; c0 += kUnroll * stride) {
-            uint4 w[kUnroll];
+        for (int64_t c0 = tid; c0 < chunks; c0 += U * stride) {
+            uint4 w[U];
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
+            for (int u = 0; u < U; ++u) {
                 const int64_t c = c0 + u * stride;
                 w[u] = c < chunks ? p[c] : make_uint4(0u, 0u, 0u, 0u);
             }
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) m = max(m, chunk_max<IN>(w[u]));
+            for (int u = 0; u < U; ++u) m = max(m, chunk_max<IN>(w[u]));
         }
         tail_begin = chunks * PER;
     }
@@ -119,20 +125,26 @@ __global__ __launch_bounds__(kThreads) void finalize_kernel(const uint32_t* __re
 int amax_partials(const void* x, int64_t numel, int in_code, uint32_t* partial, hipStream_t st) {
     const int es = in_code == CKH_F32 ? 4 : 2;
     const bool vec = aligned(x, 16);
-    // up to 8 workgroups per CU, each thread with kUnroll 16-byte loads in flight; never
-    // more workgroups than the workspace has partial words
+    // up to 8 workgroups per CU, each thread with kUnroll 16-byte loads in flight (a small
+    // tensor kUnrollSmall, on up to kSpreadBlocks workgroups); never more workgroups than the
+    // workspace has partial words
     const int64_t chunks = cdiv(numel * es, 16);
-    const int blocks = static_cast<int>(
-        std::max<int64_t>(1, std::min<int64_t>(am::kMaxBlocks, cdiv(chunks, am::kThreads * am::kUnroll))));
-#define LAUNCH(I)                                                                                                \
-    do {                                                                                                         \
-        if (vec) hipLaunchKernelGGL((am::amax_kernel<I, true>), dim3(blocks), dim3(am::kThreads), 0, st, x, numel, partial); \
-        else hipLaunchKernelGGL((am::amax_kernel<I, false>), dim3(blocks), dim3(am::kThreads), 0, st, x, numel, partial); \
+    const bool spread = cdiv(chunks, am::kThreads * am::kUnrollSmall) <= am::kSpreadBlocks;
+    const int blocks = static_cast<int>(std::max<int64_t>(
+        1, std::min<int64_t>(am::kMaxBlocks, cdiv(chunks, am::kThreads * (spread ? am::kUnrollSmall : am::kUnroll)))));
+#define LAUNCH_U(I, V, U) \
+    hipLaunchKernelGGL((am::amax_kernel<I, V, U>), dim3(blocks), dim3(am::kThreads), 0, st, x, numel, partial)
+#define LAUNCH(I)                                              \
+    do {                                                       \
+        if (!vec) LAUNCH_U(I, false, 1);                       \
+        else if (spread) LAUNCH_U(I, true, am::kUnrollSmall);  \
+        else LAUNCH_U(I, true, am::kUnroll);                   \
     } while (0)
     if (in_code == CKH_F32) LAUNCH(CKH_F32);
     else if (in_code == CKH_F16) LAUNCH(CKH_F16);
     else LAUNCH(CKH_BF16);
 #undef LAUNCH
+#undef LAUNCH_U
     return blocks;
 }
 

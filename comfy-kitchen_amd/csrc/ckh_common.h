@@ -425,12 +425,9 @@ __device__ __forceinline__ PartialWords<NT> load_partial_words(const uint32_t* _
     return w;
 }
 
-template <int IN, int NT>
-__device__ __forceinline__ float scale_from_partial_words(const PartialWords<NT>& w, float inv_divisor,
-                                                          uint32_t* red) {
-    uint32_t m = w.v[0];
-#pragma unroll
-    for (int i = 1; i < PartialWords<NT>::N; ++i) m = max(m, w.v[i]);
+// The largest m over the NT threads of the workgroup.
+template <int NT>
+__device__ __forceinline__ uint32_t workgroup_max(uint32_t m, uint32_t* red) {
 #pragma unroll
     for (int s = 32; s >= 1; s >>= 1) m = max(m, static_cast<uint32_t>(__shfl_xor(static_cast<int>(m), s, 64)));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
@@ -441,7 +438,16 @@ __device__ __forceinline__ float scale_from_partial_words(const PartialWords<NT>
     uint32_t b = red[0];
 #pragma unroll
     for (int i = 1; i < NT / 64; ++i) b = max(b, red[i]);
-    return scale_of_amax_bits<IN>(b, inv_divisor);
+    return b;
+}
+
+template <int IN, int NT>
+__device__ __forceinline__ float scale_from_partial_words(const PartialWords<NT>& w, float inv_divisor,
+                                                          uint32_t* red) {
+    uint32_t m = w.v[0];
+#pragma unroll
+    for (int i = 1; i < PartialWords<NT>::N; ++i) m = max(m, w.v[i]);
+    return scale_of_amax_bits<IN>(workgroup_max<NT>(m, red), inv_divisor);
 }
 
 }  // namespace ckh

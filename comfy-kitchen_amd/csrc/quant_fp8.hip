@@ -13,6 +13,7 @@
 // (quantize_fp8_pipe_kernel); other quantize calls and every dequantize use 128-thread
 // workgroups with 16 elements per thread, one tile per thread.
 #include "ckh_common.h"
+#include "quant_math.h"
 
 namespace ckh {
 
@@ -159,12 +160,21 @@ __device__ __forceinline__ void quantize_tile(const Raw8<IN>& ra, const Raw8<IN>
 // by wave 0 with the scalar path.  Same-process A/B on C1 against the one-tile-per-lane
 // kernel below: 93.2% vs 90.8% and 91.7% vs 89.6% of the copy floor (16 waves per CU;
 // 8, 12, 24 and 32 measured 87-90%).
+// DYN: the scale is not an input but the layouts' default, amax(|x|) / divisor, formed by
+// every workgroup from the `nparts` partial maxima that amax_partials wrote for this x (DYN 1)
+// or, for an x of at most kWholeAmaxBytes, from all of x (DYN 2); workgroup 0 stores it to
+// *scale_out.  Those words are loaded before the wave's first tile, so that the reduction
+// runs while it is in flight.  (The scale as a launch of its own between the two took
+// 4.5 us a call inside a captured graph.)
 constexpr int kQWavesPerCU = 16;
 
-template <int IN, int OUT>
+template <int IN, int OUT, int DYN>
 __global__ __launch_bounds__(256) void quantize_fp8_pipe_kernel(const void* __restrict__ x,
                                                                 const float* __restrict__ scale,
-                                                                uint8_t* __restrict__ out, int64_t n) {
+                                                                uint8_t* __restrict__ out, int64_t n,
+                                                                const uint32_t* __restrict__ partial,
+                                                                uint32_t nparts, float inv_divisor,
+                                                                float* __restrict__ scale_out) {
     constexpr int ES = ElemSize<IN>::value;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t W = gridDim.x * 4u;
@@ -172,12 +182,23 @@ __global__ __launch_bounds__(256) void quantize_fp8_pipe_kernel(const void* __re
     const uint32_t tiles = static_cast<uint32_t>(n >> 10);
     const char* xb = static_cast<const char*>(x);
     uint32_t t = w0;
-    Raw8<IN> ra{}, rb{};
-    if (t < tiles) {
-        ra = load8_raw<IN>(xb + (static_cast<int64_t>(t) * 1024 + 8 * lane) * ES);
-        rb = load8_raw<IN>(xb + (static_cast<int64_t>(t) * 1024 + 512 + 8 * lane) * ES);
+    PartialWords<256> pw;
+    WholeChunks<256> wc;
+    if constexpr (DYN == 1) pw = load_partial_words<256>(partial, nparts);
+    if constexpr (DYN == 2) wc = load_whole_chunks<256>(x, static_cast<uint32_t>(n) * ES);
+    // (a wave with no tile loads the last one and stores nothing)
+    const int64_t tl = min(t, tiles - 1);
+    Raw8<IN> ra = load8_raw<IN>(xb + (tl * 1024 + 8 * lane) * ES);
+    Raw8<IN> rb = load8_raw<IN>(xb + (tl * 1024 + 512 + 8 * lane) * ES);
+    float sc;
+    if constexpr (DYN == 0) {
+        sc = scale[0];
+    } else {
+        __shared__ uint32_t red[4];
+        if constexpr (DYN == 1) sc = scale_from_partial_words<IN, 256>(pw, inv_divisor, red);
+        else sc = scale_from_whole_chunks<IN, 256>(wc, inv_divisor, red);
+        if (blockIdx.x == 0 && threadIdx.x == 0) *scale_out = sc;
     }
-    const float sc = scale[0];
     const float r = round_to<IN>(1.0f / sc);
     while (t < tiles) {
         const uint32_t tn = t + W;
@@ -313,6 +334,67 @@ using namespace ckh;
         }                           \
     } while (0)
 
+namespace {
+
+// The persistent kernel takes the call: aligned 16-bit input of at least one wave-tile.
+bool fp8_pipe_applies(const void* x, const void* out, int64_t numel, int in_code) {
+    return aligned(x, 16) && aligned(out, 16) && in_code != CKH_F32 && numel >= 1024;
+}
+
+// DYN: see quantize_fp8_pipe_kernel
+template <int DYN>
+void launch_fp8_pipe(const void* x, uint8_t* out, const float* scale, int64_t numel, int in_code, int out_code,
+                     const uint32_t* partial, uint32_t nparts, float inv_divisor, float* scale_out, hipStream_t st) {
+    // waves: at most kQWavesPerCU per CU, as many tiles per wave as that forces, and the
+    // tiles spread evenly over the waves
+    const int64_t tiles = numel >> 10;
+    const int64_t per_wave = cdiv(tiles, static_cast<int64_t>(device_cus()) * kQWavesPerCU);
+    const dim3 grid(static_cast<unsigned>(cdiv(cdiv(tiles, per_wave), 4)));
+#define LAUNCH_P(I, O)                                                                                         \
+    hipLaunchKernelGGL((quantize_fp8_pipe_kernel<I, O, DYN>), grid, dim3(256), 0, st, x, scale, out, numel, partial, \
+                       nparts, inv_divisor, scale_out)
+    if (out_code == CKH_E4M3) {
+        if (in_code == CKH_F16) LAUNCH_P(CKH_F16, CKH_E4M3);
+        else LAUNCH_P(CKH_BF16, CKH_E4M3);
+    } else {
+        if (in_code == CKH_F16) LAUNCH_P(CKH_F16, CKH_E5M2);
+        else LAUNCH_P(CKH_BF16, CKH_E5M2);
+    }
+#undef LAUNCH_P
+}
+
+}  // namespace
+
+extern "C" int ckh_quantize_fp8_dynamic(const void* x, float divisor, void* scale_out, void* out, int64_t numel,
+                                        int in_code, int out_code, void* workspace, uintptr_t stream) {
+    CKH_REQUIRE(x && scale_out && out && workspace, "quantize_fp8_dynamic: null pointer");
+    CKH_REQUIRE(numel > 0, "quantize_fp8_dynamic: empty tensor (torch.amax of an empty tensor is an error too)");
+    CKH_REQUIRE(in_code == CKH_F32 || in_code == CKH_F16 || in_code == CKH_BF16,
+                "quantize_fp8_dynamic: unsupported input dtype code %d", in_code);
+    CKH_REQUIRE(out_code == CKH_E4M3 || out_code == CKH_E5M2,
+                "quantize_fp8_dynamic: unsupported output dtype code %d", out_code);
+    CKH_REQUIRE(aligned(scale_out, 4) && aligned(workspace, 4), "quantize_fp8_dynamic: scale or workspace misaligned");
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    uint8_t* o = static_cast<uint8_t*>(out);
+    float* so = static_cast<float*>(scale_out);
+    uint32_t* partial = static_cast<uint32_t*>(workspace);
+    const bool pipe = fp8_pipe_applies(x, out, numel, in_code);
+    if (pipe && numel % 8 == 0 && numel * 2 <= kWholeAmaxBytes) {
+        launch_fp8_pipe<2>(x, o, nullptr, numel, in_code, out_code, nullptr, 0u, 1.0f / divisor, so, st);
+        return check_launch("quantize_fp8_dynamic");
+    }
+    const int nparts = amax_partials(x, numel, in_code, partial, st);
+    if (pipe) {
+        launch_fp8_pipe<1>(x, o, nullptr, numel, in_code, out_code, partial, static_cast<uint32_t>(nparts),
+                           1.0f / divisor, so, st);
+        return check_launch("quantize_fp8_dynamic");
+    }
+    // f32 or unaligned x: the scale as its own launch, then the quantize reading it
+    amax_finalize(partial, nparts, in_code, divisor, so, st);
+    if (int rc = check_launch("quantize_fp8_dynamic")) return rc;
+    return ckh_quantize_fp8(x, out, scale_out, numel, in_code, out_code, stream);
+}
+
 extern "C" int ckh_quantize_fp8(const void* x, void* out, const void* scale, int64_t numel, int in_code,
                                 int out_code, uintptr_t stream) {
     CKH_REQUIRE(numel >= 0, "quantize_fp8: numel < 0");
@@ -323,24 +405,9 @@ extern "C" int ckh_quantize_fp8(const void* x, void* out, const void* scale, int
     CKH_REQUIRE(out_code == CKH_E4M3 || out_code == CKH_E5M2, "quantize_fp8: unsupported output dtype code %d",
                 out_code);
     const bool vec = aligned(x, 16) && aligned(out, 16);
-    if (vec && in_code != CKH_F32 && numel >= 1024) {
-        // waves: at most kQWavesPerCU per CU, as many tiles per wave as that forces, and the
-        // tiles spread evenly over the waves
-        const int64_t tiles = numel >> 10;
-        const int64_t per_wave = cdiv(tiles, static_cast<int64_t>(device_cus()) * kQWavesPerCU);
-        const dim3 pgrid(static_cast<unsigned>(cdiv(cdiv(tiles, per_wave), 4)));
-        hipStream_t pst = reinterpret_cast<hipStream_t>(stream);
-        const float* psp = static_cast<const float*>(scale);
-        uint8_t* po = static_cast<uint8_t*>(out);
-#define LAUNCH_P(I, O) hipLaunchKernelGGL((quantize_fp8_pipe_kernel<I, O>), pgrid, dim3(256), 0, pst, x, psp, po, numel)
-        if (out_code == CKH_E4M3) {
-            if (in_code == CKH_F16) LAUNCH_P(CKH_F16, CKH_E4M3);
-            else LAUNCH_P(CKH_BF16, CKH_E4M3);
-        } else {
-            if (in_code == CKH_F16) LAUNCH_P(CKH_F16, CKH_E5M2);
-            else LAUNCH_P(CKH_BF16, CKH_E5M2);
-        }
-#undef LAUNCH_P
+    if (fp8_pipe_applies(x, out, numel, in_code)) {
+        launch_fp8_pipe<0>(x, static_cast<uint8_t*>(out), static_cast<const float*>(scale), numel, in_code, out_code,
+                           nullptr, 0u, 0.0f, nullptr, reinterpret_cast<hipStream_t>(stream));
         return check_launch("quantize_fp8");
     }
     dim3 grid(static_cast<unsigned>(cdiv(numel, kThreads * kPerThread)));

@@ -193,4 +193,33 @@ __device__ __forceinline__ v2h scale_pair(uint32_t word, int sh) {
     return __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(word >> sh, 1.0f, false);
 }
 
+// Both passes in one launch for a small 16-bit tensor: every workgroup reads all of it
+// (whole 16-byte chunks, at most kWholeAmaxBytes, all loads in flight at once; chunks past
+// the end read as zeros) and reduces it itself.
+constexpr int64_t kWholeAmaxBytes = 64 * 1024;
+template <int NT>
+struct WholeChunks {
+    static constexpr int N = static_cast<int>(kWholeAmaxBytes / 16 / NT);
+    ckh_u32x4 v[N];
+};
+
+template <int NT>
+__device__ __forceinline__ WholeChunks<NT> load_whole_chunks(const void* __restrict__ x, uint32_t bytes) {
+    const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(x, bytes);
+    WholeChunks<NT> w;
+#pragma unroll
+    for (int i = 0; i < WholeChunks<NT>::N; ++i)
+        w.v[i] = __builtin_bit_cast(ckh_u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (threadIdx.x + i * NT) * 16u, 0, 0));
+    return w;
+}
+
+template <int IN, int NT>
+__device__ __forceinline__ float scale_from_whole_chunks(const WholeChunks<NT>& w, float inv_divisor, uint32_t* red) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int i = 0; i < WholeChunks<NT>::N; ++i)
+        m = max(m, amax16x8(make_uint4(w.v[i].x, w.v[i].y, w.v[i].z, w.v[i].w)));
+    return scale_of_amax_bits<IN>(amax16_to_f32_bits<IN>(workgroup_max<NT>(m, red)), inv_divisor);
+}
+
 }  // namespace ckh
