@@ -72,10 +72,14 @@ class TensorCoreMXFP8Layout(QuantizedLayout):
 
 
 def _gemm(x: QuantizedTensor, w: QuantizedTensor, bias, out_dtype, rows: int, cols: int) -> torch.Tensor:
-    """x @ w_physical.T on the MXFP8 GEMM (w's storage is [N, K]), sliced to [rows, cols]."""
+    """x @ w_physical.T on the MXFP8 GEMM (w's storage is [N, K]), sliced to [rows, cols].
+
+    x's padding rows are not multiplied: one row as such, rather than as the 32 it is padded
+    to, takes the GEMM's 8-row form (18432 x 3072: 12.7 against 16.4 us)."""
     import comfy_kitchen as ck
 
     xq, sa = TensorCoreMXFP8Layout.get_plain_tensors(x)
+    xq = xq[:rows]
     wq, sb = TensorCoreMXFP8Layout.get_plain_tensors(w)
     if bias is not None and bias.numel() != wq.shape[0]:  # the kernel's N is the padded one
         bias = torch.nn.functional.pad(bias.reshape(-1), (0, wq.shape[0] - bias.numel()))

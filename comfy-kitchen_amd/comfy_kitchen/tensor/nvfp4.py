@@ -90,10 +90,12 @@ class TensorCoreNVFP4Layout(QuantizedLayout):
 
 
 def _gemm(x: QuantizedTensor, w: QuantizedTensor, bias, out_dtype, rows: int, cols: int) -> torch.Tensor:
-    """x @ w_physical.T on the NVFP4 GEMM (w's storage is [N, K/2]), sliced to [rows, cols]."""
+    """x @ w_physical.T on the NVFP4 GEMM (w's storage is [N, K/2]), sliced to [rows, cols];
+    x's padding rows are not multiplied."""
     import comfy_kitchen as ck
 
     xq, ts_a, bs_a = TensorCoreNVFP4Layout.get_plain_tensors(x)
+    xq = xq[:rows]
     wq, ts_b, bs_b = TensorCoreNVFP4Layout.get_plain_tensors(w)
     if bias is not None and bias.numel() != wq.shape[0]:  # the kernel's N is the padded one
         bias = torch.nn.functional.pad(bias.reshape(-1), (0, wq.shape[0] - bias.numel()))
