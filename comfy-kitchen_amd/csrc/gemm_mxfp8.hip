@@ -52,6 +52,7 @@
 #include <utility>
 
 #include "ckh_common.h"
+#include "gemm_mid.h"
 #include "skinny.h"
 
 namespace ckh {
@@ -1181,18 +1182,80 @@ void launch_split(mx::Args p, int out_code, int bias_code, bool has_bias, hipStr
 #undef LAUNCH
 }
 
+// Small tiles (gemm_mid.h): the first of these whose grid fits the CUs in one round.  The
+// order is by operand rows, i.e. by time: over 200 measured shapes the first that fits was
+// within 3% of the fastest that fits.  Larger tiles than these (or a second round) were slower
+// than the 256 x 256 kernel's half tiles.
+struct MidTile {
+    int tm, tn;
+};
+constexpr MidTile kMidTiles[] = {{64, 64}, {128, 64}, {128, 96}, {128, 128}, {128, 160}, {128, 192}};
+
+// Index of the small tile to use, or -1: the estimated time (us) of the first that fits against
+// that of the 256 x 256 kernel.  Fitted to the same shapes:
+//   small tiles  2.0 + 0.0165 rows + 0.00228 rows per 128-byte stage (rows = TM + TN);
+//   split-K      14.7 + 0.575 per stage of a K range in half tiles, 1.09 in full tiles (two
+//                launches; 200 x 5120 x 13824, six ranges of 36: 35.4 measured, small tiles 50);
+//   half tiles   6.2 + 0.4 per stage of K (200 x 21504 x 512: 9.5 measured, small tiles 12.1).
+int mid_tile(int M, int N, int K, const SplitPlan& sp, int cus) {
+    for (int i = 0; i < static_cast<int>(sizeof(kMidTiles) / sizeof(kMidTiles[0])); ++i) {
+        const MidTile t = kMidTiles[i];
+        if (cdiv(M, t.tm) * cdiv(N, t.tn) > cus) continue;
+        const double rows = t.tm + t.tn;
+        const double mid = 2.0 + 0.0165 * rows + 0.00228 * rows * static_cast<double>(cdiv(K, 128));
+        const double big = sp.S > 1 ? 14.7 + (sp.nw == 2 ? 0.575 : 1.09) * sp.ks : 6.2 + 0.4 * static_cast<double>(cdiv(K, mx::BK));
+        return mid < big ? i : -1;
+    }
+    return -1;
+}
+
+template <bool UNIT, int TM, int TN, int NST>
+void launch_mid_tile(const mid::Args& p, int out_code, hipStream_t st) {
+    const dim3 grid(static_cast<unsigned>(p.tiles_m * cdiv(p.N, TN)));
+#define LAUNCH(O) hipLaunchKernelGGL((mid::gemm_mid_kernel<O, UNIT, TM, TN, NST>), grid, dim3(mid::kThreads), 0, st, p)
+    if (out_code == CKH_BF16) LAUNCH(CKH_BF16);
+    else if (out_code == CKH_F16) LAUNCH(CKH_F16);
+    else LAUNCH(CKH_F32);
+#undef LAUNCH
+}
+
+template <bool UNIT>
+void launch_mid(const mx::Args& q, int tile, int out_code, int bias_code, bool has_bias, hipStream_t st) {
+    mid::Args p{};
+    p.a = q.a; p.b = q.b; p.sa = q.sa; p.sb = q.sb; p.out = q.out;
+    p.bias = has_bias ? q.bias : nullptr;
+    p.bias_code = bias_code;
+    p.M = q.M; p.N = q.N; p.K = q.K; p.ncb = q.ncb; p.sa_rows = q.sa_rows; p.sb_rows = q.sb_rows;
+    p.tsa = q.tsa; p.tsb = q.tsb;
+    p.tiles_m = static_cast<int>(cdiv(p.M, kMidTiles[tile].tm));
+    switch (tile) {  // ring depth: what fits in LDS beside the staged output
+        case 0: launch_mid_tile<UNIT, 64, 64, 6>(p, out_code, st); break;
+        case 1: launch_mid_tile<UNIT, 128, 64, 5>(p, out_code, st); break;
+        case 2: launch_mid_tile<UNIT, 128, 96, 4>(p, out_code, st); break;
+        case 3: launch_mid_tile<UNIT, 128, 128, 4>(p, out_code, st); break;
+        case 4: launch_mid_tile<UNIT, 128, 160, 3>(p, out_code, st); break;
+        default: launch_mid_tile<UNIT, 128, 192, 3>(p, out_code, st); break;
+    }
+}
+
 // The 256 x 256 tiles run one per CU in rounds.  When the last round would be at most
 // half full (e.g. 864 tiles = 3 rounds + 96), its tiles run as twice as many 256 x 128
 // half tiles (about 55% of a full tile's time each), in the same grid.  A grid of one
 // round fills the remaining CUs with weight-prefetch workgroups (prefetch_weight).
-// Activations of at most kSkinnyMaxM rows take the skinny kernel, and small grids split K
-// when the caller gives a workspace.
+// Activations of at most kSkinnyMaxM rows take the skinny kernel, a few hundred rows the small
+// tiles, and small grids with long K split K when the caller gives a workspace.
 template <bool UNIT>
 int launch_gemm(mx::Args p, int out_code, int bias_code, bool has_bias, void* workspace, int64_t workspace_bytes,
                 hipStream_t st) {
     if (p.M <= kSkinnyMaxM) return launch_skinny<UNIT>(p, out_code, bias_code, has_bias, st);
-    const SplitPlan sp = split_plan(p.M, p.N, p.K);
-    if (sp.S > 1 && workspace && workspace_bytes >= split_workspace_bytes(p.M, p.N, p.K)) {
+    SplitPlan sp = split_plan(p.M, p.N, p.K);
+    if (!workspace || workspace_bytes < split_workspace_bytes(p.M, p.N, p.K)) sp.S = 1;
+    const int cus = device_cus();
+    if (const int tile = mid_tile(p.M, p.N, p.K, sp, cus); tile >= 0) {
+        launch_mid<UNIT>(p, tile, out_code, bias_code, has_bias, st);
+        return check_launch(UNIT ? "scaled_mm_fp8" : "scaled_mm_mxfp8");
+    }
+    if (sp.S > 1) {
         p.splits = sp.S;
         p.ks = sp.ks;
         p.part = static_cast<float*>(workspace);
@@ -1209,7 +1272,6 @@ int launch_gemm(mx::Args p, int out_code, int bias_code, bool has_bias, void* wo
     const int wgs = p.n_full + 2 * p.n_half;
     // (the CUs the device has, which a partitioned GPU reduces: prefetch workgroups that
     // found no idle CU would run after the tiles, for nothing)
-    const int cus = device_cus();
     p.n_pref = wgs < cus ? cus - wgs : 0;
     p.bias_code = bias_code;
     launch_grid<UNIT>(p, static_cast<unsigned>(wgs + p.n_pref), out_code, has_bias, st);

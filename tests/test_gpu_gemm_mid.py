@@ -1,0 +1,55 @@
+"""The small-tile GEMMs of a few hundred activation rows, every tile shape: rows past M, columns
+past N (N odd, so that elements are stored one by one, and N a multiple of 8), K ending inside
+a stage, one to three stages (fewer than the ring holds), bias and output types, against an
+fp32 matmul of the dequantized operands."""
+import pytest
+import torch
+
+import comfy_kitchen as ck
+
+pytestmark = pytest.mark.gpu
+
+# fp32 output: the order of the fp32 sums; 16-bit outputs: one rounding (2^-9 and 2^-12 relative)
+REL = {torch.float32: 1e-4, torch.float16: 1e-3, torch.bfloat16: 4e-3}
+
+# (m, n, k): 64 x 64 tiles (one stage, three stages, many), then 128 x 64, 96, 128, 160, 192
+SHAPES = [(65, 33, 32), (70, 1000, 352), (200, 2001, 1152), (200, 7001, 1056), (201, 6992, 128), (300, 7001, 1120),
+          (300, 9003, 2080), (500, 9008, 2080), (500, 9004, 2112), (500, 11001, 4128), (512, 12288, 4096)]
+
+
+def _rel(got, want):
+    return ((got.double() - want.double()).norm() / want.double().norm()).item()
+
+
+@pytest.mark.parametrize("out_dtype,bias_dtype", [(torch.float32, None), (torch.bfloat16, torch.bfloat16),
+                                                  (torch.float16, torch.float32), (torch.bfloat16, None)])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_small_tiles(m, n, k, out_dtype, bias_dtype, hip):
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device="cuda") * torch.exp(torch.randn(m, 1, generator=g, device="cuda"))
+    w = torch.randn(n, k, generator=g, device="cuda") * 0.02
+    bias = None if bias_dtype is None else torch.randn(n, generator=g, device="cuda").to(bias_dtype)
+    b32 = 0.0 if bias is None else bias.float()
+    qx, sx = ck.quantize_mxfp8(x.bfloat16())
+    qw, sw = ck.quantize_mxfp8(w.bfloat16())
+    want = ck.dequantize_mxfp8(qx, sx, torch.float32) @ ck.dequantize_mxfp8(qw, sw, torch.float32).t() + b32
+    got = ck.scaled_mm_mxfp8(qx, qw, sx, sw, bias=bias, out_dtype=out_dtype)
+    assert got.shape == (m, n) and got.dtype == out_dtype
+    assert _rel(got, want) <= REL[out_dtype]
+    ta, tb = torch.full((1,), 0.37, device="cuda"), torch.full((1,), 0.021, device="cuda")
+    want = (qx.float() @ qw.float().t()) * (ta * tb) + b32
+    got = ck.scaled_mm_fp8(qx, qw, ta, tb, bias=bias, out_dtype=out_dtype)
+    assert _rel(got, want) <= REL[out_dtype]
+
+
+def test_small_tiles_read_no_neighbour(hip):
+    """Operands inside larger buffers full of NaN codes: nothing outside them is used."""
+    m, n, k = 129, 97, 160
+    pad = torch.full((m + n + 8, k), 0x7F, dtype=torch.uint8, device="cuda").view(torch.float8_e4m3fn)
+    x, _ = ck.quantize_mxfp8(torch.randn(m, k, device="cuda").bfloat16())
+    w, _ = ck.quantize_mxfp8(torch.randn(n, k, device="cuda").bfloat16())
+    pad.view(torch.uint8)[:m] = x.view(torch.uint8)
+    pad.view(torch.uint8)[m + 4:m + 4 + n] = w.view(torch.uint8)
+    one = torch.ones(1, device="cuda")
+    got = ck.scaled_mm_fp8(pad[:m], pad[m + 4:m + 4 + n], one, one, out_dtype=torch.float32)
+    assert _rel(got, x.float() @ w.float().t()) <= 1e-4
