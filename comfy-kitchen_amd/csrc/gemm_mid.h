@@ -90,6 +90,150 @@ __device__ __forceinline__ void wait_barrier() {
     __asm__ volatile("" ::: "memory");
 }
 
+// The end of a tile, in LDS that no load writes any more (at least TM * TN * 2 KG bytes): the sums
+// of the KG K groups (of WM x WN waves, wave = WM WN kg + WM wn + wm) added, times alpha
+// (SCALE), plus the bias in lds_bias, rounded and stored.  acc: a wave's NT x MT MFMA tiles;
+// result lane 32 h + r, register 4 g + e of tile (i, j) holds column 32 i + 8 g + 4 h + e, row
+// 32 j + r of the wave's part.
+template <int OUT, bool SCALE, int TM, int TN, int KG, int WM, int MT, int NT>
+__device__ __forceinline__ void finish_tile(v16f (&acc)[NT][MT], uint8_t* lds, const float* lds_bias, float alpha,
+                                            bool bias, void* out, int M, int N, int m0, int n0, int wave, int lane) {
+    constexpr int WPG = 8 / KG, WN = WPG / WM, PITCH = TN * 2 + 16;  // staged 16-bit output row
+    const int kg = wave / WPG, wig = wave % WPG, wm = wig % WM, wn = wig / WM;
+    const int h = lane >> 5, r = lane & 31;
+    // The upper half of the groups gives its sums to the lower half, until two are left.
+#pragma unroll
+    for (int G = KG; G > 2; G /= 2) {
+        float4* red = reinterpret_cast<float4*>(lds) + (kg % (G / 2) * WPG + wig) * (MT * NT * 4 * 64) + lane;
+        if (kg >= G / 2 && kg < G) {
+#pragma unroll
+            for (int q = 0; q < MT * NT * 4; ++q) {
+                const v16f& a = acc[q / 4 / MT][q / 4 % MT];
+                red[q * 64] = make_float4(a[4 * (q % 4)], a[4 * (q % 4) + 1], a[4 * (q % 4) + 2], a[4 * (q % 4) + 3]);
+            }
+        }
+        wait_barrier<63>();
+        if (kg < G / 2) {
+#pragma unroll
+            for (int q = 0; q < MT * NT * 4; ++q) {
+                v16f& a = acc[q / 4 / MT][q / 4 % MT];
+                const float4 o = red[q * 64];
+                a[4 * (q % 4)] += o.x;
+                a[4 * (q % 4) + 1] += o.y;
+                a[4 * (q % 4) + 2] += o.z;
+                a[4 * (q % 4) + 3] += o.w;
+            }
+        }
+        wait_barrier<63>();
+    }
+    // The last two K groups exchange halves of every MFMA tile (register quads g = 0, 1 and 2, 3):
+    // group 0 ends with quads 0, 1, group 1 with 2, 3.
+    float4* red = reinterpret_cast<float4*>(lds) + wig * (MT * NT * 4 * 64) + lane;
+    auto send = [&](auto g0_c) __attribute__((always_inline)) {
+        constexpr int g0 = decltype(g0_c)::value;
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int j = 0; j < MT; ++j)
+#pragma unroll
+                for (int g = g0; g < g0 + 2; ++g)
+                    red[((i * MT + j) * 4 + g) * 64] = make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1],
+                                                                   acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
+    };
+    if (kg == 0) send(std::integral_constant<int, 2>{});
+    else if (kg == 1) send(std::integral_constant<int, 0>{});
+    wait_barrier<63>();
+    float4 v[NT][MT][2];
+    auto recv = [&](auto g0_c) __attribute__((always_inline)) {
+        constexpr int g0 = decltype(g0_c)::value;
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int j = 0; j < MT; ++j)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const int g = g0 + q;
+                    const float4 o = red[((i * MT + j) * 4 + g) * 64];
+                    v[i][j][q] = make_float4(acc[i][j][4 * g] + o.x, acc[i][j][4 * g + 1] + o.y,
+                                             acc[i][j][4 * g + 2] + o.z, acc[i][j][4 * g + 3] + o.w);
+                }
+    };
+    if (kg == 0) recv(std::integral_constant<int, 0>{});
+    else if (kg == 1) recv(std::integral_constant<int, 2>{});
+
+    const int ml = wm * (TM / WM) + r;                 // row of MFMA row tile 0
+    const int nl = wn * (TN / WN) + 16 * kg + 4 * h;   // column of MFMA column tile 0, quad 0
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            float4 bv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (bias) bv = *reinterpret_cast<const float4*>(lds_bias + nl + 32 * i + 8 * q);
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                float4& o = v[i][j][q];
+                if constexpr (SCALE) o = make_float4(o.x * alpha, o.y * alpha, o.z * alpha, o.w * alpha);
+                if (bias) o = make_float4(o.x + bv.x, o.y + bv.y, o.z + bv.z, o.w + bv.w);
+            }
+        }
+    if constexpr (OUT == CKH_F32) {
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const int m = m0 + ml + 32 * j;
+            if (m >= M || kg > 1) continue;
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const int n = n0 + nl + 32 * i + 8 * q;
+                    float* o = static_cast<float*>(out) + static_cast<int64_t>(m) * N + n;
+                    const float e[4] = {v[i][j][q].x, v[i][j][q].y, v[i][j][q].z, v[i][j][q].w};
+                    if (n + 3 < N && (N & 3) == 0) {
+                        *reinterpret_cast<float4*>(o) = v[i][j][q];
+                    } else {
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            if (n + k < N) o[k] = e[k];
+                    }
+                }
+        }
+    } else {
+        // 16-bit output: staged as TM rows in LDS, then whole rows, 16 bytes per lane
+        wait_barrier<63>();  // the exchange area is read
+        if (kg < 2) {
+#pragma unroll
+            for (int j = 0; j < MT; ++j)
+#pragma unroll
+                for (int i = 0; i < NT; ++i)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const float4 o = v[i][j][q];
+                        *reinterpret_cast<uint2*>(lds + (ml + 32 * j) * PITCH + (nl + 32 * i + 8 * q) * 2) =
+                            make_uint2(pack2<OUT>(o.x, o.y), pack2<OUT>(o.z, o.w));
+                    }
+        }
+        wait_barrier<63>();
+        constexpr int LPR = TN / 8;  // 16-byte pieces per output row
+        const bool n8 = (N & 7) == 0;
+#pragma unroll
+        for (int k = 0; k < TM * LPR / kThreads; ++k) {
+            const int piece = k * kThreads + wave * 64 + lane, row = piece / LPR, lr = piece - row * LPR;
+            const int n = n0 + 8 * lr;
+            const bool vec = n8 && n + 8 <= N;
+            const v4u d = *reinterpret_cast<const v4u*>(lds + row * PITCH + lr * 16);
+            if (m0 + row >= M) continue;
+            uint16_t* o = static_cast<uint16_t*>(out) + static_cast<int64_t>(m0 + row) * N + n;
+            if (vec) {
+                __builtin_nontemporal_store(d, reinterpret_cast<v4u*>(o));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (n + e < N) o[e] = static_cast<uint16_t>(d[e >> 1] >> (16 * (e & 1)));
+            }
+        }
+    }
+}
+
 template <bool UNIT, int TM, int TN, int NST>
 struct Shape {
     static constexpr int WM = TM >= 128 ? 4 : 2, WN = 4 / WM;         // waves of a K group along m, n
@@ -99,8 +243,7 @@ struct Shape {
     static constexpr int LPW = AL + BL + (UNIT ? 0 : 1);              // loads per wave and stage
     static constexpr int CODES = (AL + BL) * 8192;         // (TN = 96: the last 32 rows stay zero)
     static constexpr int STG = CODES + (UNIT ? 0 : 2048);  // + scale words: 1 KB per operand
-    static constexpr int PITCH = TN * 2 + 16;              // staged 16-bit output row
-    static_assert(TM * TN * 4 <= NST * STG && TM * PITCH <= NST * STG, "the epilogue reuses the ring");
+    static_assert(TM * TN * 4 <= NST * STG && TM * (TN * 2 + 16) <= NST * STG, "the epilogue reuses the ring");
     static_assert((NST - 1) * LPW < 64, "vmcnt range");
 };
 
@@ -241,111 +384,8 @@ __global__ __launch_bounds__(kThreads) void gemm_mid_kernel(Args p) {
     if (p.bias && tid < TN) lds_bias[tid] = bias_value(bias_bits, p.bias_code);
     wait_barrier<0>();  // trailing loads have landed and every read is done: LDS is free
 
-    // The two K groups exchange halves of every MFMA tile (register quads g = 0, 1 and 2, 3):
-    // group 0 ends with quads 0, 1, group 1 with 2, 3.
-    float4* red = reinterpret_cast<float4*>(lds) + (wave & 3) * (MT * NT * 4 * 64) + lane;
-    auto send = [&](auto g0_c) __attribute__((always_inline)) {
-        constexpr int g0 = decltype(g0_c)::value;
-#pragma unroll
-        for (int i = 0; i < NT; ++i)
-#pragma unroll
-            for (int j = 0; j < MT; ++j)
-#pragma unroll
-                for (int g = g0; g < g0 + 2; ++g)
-                    red[((i * MT + j) * 4 + g) * 64] = make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1],
-                                                                   acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
-    };
-    if (kg == 0) send(std::integral_constant<int, 2>{});
-    else send(std::integral_constant<int, 0>{});
-    wait_barrier<63>();
-    float4 v[NT][MT][2];
-    auto recv = [&](auto g0_c) __attribute__((always_inline)) {
-        constexpr int g0 = decltype(g0_c)::value;
-#pragma unroll
-        for (int i = 0; i < NT; ++i)
-#pragma unroll
-            for (int j = 0; j < MT; ++j)
-#pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    const int g = g0 + q;
-                    const float4 o = red[((i * MT + j) * 4 + g) * 64];
-                    v[i][j][q] = make_float4(acc[i][j][4 * g] + o.x, acc[i][j][4 * g + 1] + o.y,
-                                             acc[i][j][4 * g + 2] + o.z, acc[i][j][4 * g + 3] + o.w);
-                }
-    };
-    if (kg == 0) recv(std::integral_constant<int, 0>{});
-    else recv(std::integral_constant<int, 2>{});
-
-    const int ml = wm * (TM / S::WM) + r;                 // row of MFMA row tile 0
-    const int nl = wn * (TN / S::WN) + 16 * kg + 4 * h;   // column of MFMA column tile 0, quad 0
-    const float alpha = UNIT ? p.tsa[0] * p.tsb[0] : 1.0f;
-#pragma unroll
-    for (int i = 0; i < NT; ++i)
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            float4 bv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (p.bias) bv = *reinterpret_cast<const float4*>(lds_bias + nl + 32 * i + 8 * q);
-#pragma unroll
-            for (int j = 0; j < MT; ++j) {
-                float4& o = v[i][j][q];
-                if constexpr (UNIT) o = make_float4(o.x * alpha, o.y * alpha, o.z * alpha, o.w * alpha);
-                if (p.bias) o = make_float4(o.x + bv.x, o.y + bv.y, o.z + bv.z, o.w + bv.w);
-            }
-        }
-    if constexpr (OUT == CKH_F32) {
-#pragma unroll
-        for (int j = 0; j < MT; ++j) {
-            const int m = m0 + ml + 32 * j;
-            if (m >= p.M) continue;
-#pragma unroll
-            for (int i = 0; i < NT; ++i)
-#pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    const int n = n0 + nl + 32 * i + 8 * q;
-                    float* o = static_cast<float*>(p.out) + static_cast<int64_t>(m) * p.N + n;
-                    const float e[4] = {v[i][j][q].x, v[i][j][q].y, v[i][j][q].z, v[i][j][q].w};
-                    if (n + 3 < p.N && (p.N & 3) == 0) {
-                        *reinterpret_cast<float4*>(o) = v[i][j][q];
-                    } else {
-#pragma unroll
-                        for (int k = 0; k < 4; ++k)
-                            if (n + k < p.N) o[k] = e[k];
-                    }
-                }
-        }
-    } else {
-        // 16-bit output: staged as TM rows in LDS, then whole rows, 16 bytes per lane
-        wait_barrier<63>();  // the exchange area is read
-#pragma unroll
-        for (int j = 0; j < MT; ++j)
-#pragma unroll
-            for (int i = 0; i < NT; ++i)
-#pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    const float4 o = v[i][j][q];
-                    *reinterpret_cast<uint2*>(lds + (ml + 32 * j) * S::PITCH + (nl + 32 * i + 8 * q) * 2) =
-                        make_uint2(pack2<OUT>(o.x, o.y), pack2<OUT>(o.z, o.w));
-                }
-        wait_barrier<63>();
-        constexpr int LPR = TN / 8;  // 16-byte pieces per output row
-        const bool n8 = (p.N & 7) == 0;
-#pragma unroll
-        for (int k = 0; k < TM * LPR / kThreads; ++k) {
-            const int piece = k * kThreads + tid, row = piece / LPR, lr = piece - row * LPR;
-            const int n = n0 + 8 * lr;
-            const bool vec = n8 && n + 8 <= p.N;
-            const v4u d = *reinterpret_cast<const v4u*>(lds + row * S::PITCH + lr * 16);
-            if (m0 + row >= p.M) continue;
-            uint16_t* o = static_cast<uint16_t*>(p.out) + static_cast<int64_t>(m0 + row) * p.N + n;
-            if (vec) {
-                __builtin_nontemporal_store(d, reinterpret_cast<v4u*>(o));
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (n + e < p.N) o[e] = static_cast<uint16_t>(d[e >> 1] >> (16 * (e & 1)));
-            }
-        }
-    }
+    finish_tile<OUT, UNIT, TM, TN, 2, S::WM, MT, NT>(acc, lds, lds_bias, UNIT ? p.tsa[0] * p.tsb[0] : 1.0f,
+                                                  p.bias != nullptr, p.out, p.M, p.N, m0, n0, wave, lane);
 }
 
 }  // namespace mid

@@ -46,6 +46,7 @@
 #include <utility>
 
 #include "ckh_common.h"
+#include "gemm_mid_nv.h"
 #include "quant_math.h"
 #include "skinny.h"
 
@@ -1011,6 +1012,59 @@ int64_t nv_split_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     return cdiv(M, nv::BM) * cdiv(N, nv::BN) * sp.S * static_cast<int64_t>(nv::kPartTile) * 4;
 }
 
+// Small tiles (gemm_mid_nv.h): the first of these whose grid fits the CUs in one round, which
+// was the fastest of those that fit on all of 200 measured shapes of 65-1333 rows.  Time (us):
+// base + line per 256 elements of K.
+struct NvMidTile {
+    int tm, tn;
+    double base, line;
+};
+constexpr NvMidTile kNvMidTiles[] = {{64, 64, 5.0, 0.62}, {64, 128, 6.2, 0.8}, {128, 128, 8.5, 1.25}, {128, 192, 11.0, 1.75}};
+
+// Index of the small tile to use, or -1: that estimate against the 256 x 256 kernel's, fitted to
+// the same shapes: split-K 14 + 2.6 per group of a K range in half tiles (4.5 in whole tiles),
+// half tiles without a split 8.5 + 2.4 per group.  It took the slower form on 12 of the 200, by
+// 20% at most (768 x 1024 x 8192, where both formats' estimates are 24.5), and the small tiles
+// gained 1.39 x over all: 256 x 13824 x 5120 50.4 -> 41.9 us, 300 x 4096 x 4096 33.5 -> 19.7,
+// 128 x 3072 x 3072 21.7 -> 12.5, 65 x 5120 x 2048 22.4 -> 10.3.
+int nv_mid_tile(int M, int N, int K, const NvSplitPlan& sp, int cus) {
+    const double groups = static_cast<double>(cdiv(K, 256));
+    for (int i = 0; i < static_cast<int>(sizeof(kNvMidTiles) / sizeof(kNvMidTiles[0])); ++i) {
+        const NvMidTile& t = kNvMidTiles[i];
+        if (cdiv(M, t.tm) * cdiv(N, t.tn) > cus) continue;
+        const double big = sp.S > 1 ? 14.0 + (sp.nw == 2 ? 2.6 : 4.5) * sp.ks : 8.5 + 2.4 * groups;
+        return t.base + t.line * groups < big ? i : -1;
+    }
+    return -1;
+}
+
+template <int TM, int TN, int KG, int NST>
+void launch_nv_mid_tile(const midnv::Args& p, int out_code, hipStream_t st) {
+    const dim3 grid(static_cast<unsigned>(p.tiles_m * cdiv(p.N, TN)));
+#define LAUNCH(O) hipLaunchKernelGGL((midnv::gemm_mid_nv_kernel<O, TM, TN, KG, NST>), grid, dim3(mid::kThreads), 0, st, p)
+    if (out_code == CKH_BF16) LAUNCH(CKH_BF16);
+    else if (out_code == CKH_F16) LAUNCH(CKH_F16);
+    else LAUNCH(CKH_F32);
+#undef LAUNCH
+}
+
+void launch_nv_mid(const nv::Args& q, int tile, int out_code, int bias_code, hipStream_t st) {
+    midnv::Args p{};
+    p.a = q.a; p.b = q.b; p.sa = q.sa; p.sb = q.sb; p.alpha = q.alpha; p.bias = q.bias; p.out = q.out;
+    p.bias_code = bias_code;
+    p.M = q.M; p.N = q.N; p.K = q.K; p.ncb = q.ncb; p.sa_rows = q.sa_rows; p.sb_rows = q.sb_rows;
+    p.tiles_m = static_cast<int>(cdiv(p.M, kNvMidTiles[tile].tm));
+    // K groups: the more, the larger a wave's part of the tile and the fewer operand decodes per
+    // MFMA (64 x 128 with 4 groups, 64 x 64 a wave: 15.7 us on 128 x 3072 x 3072; with 2 groups,
+    // 32 x 64 a wave, 18.1; with 8, which add up three times in the epilogue, 18.7)
+    switch (tile) {
+        case 0: launch_nv_mid_tile<64, 64, 4, 6>(p, out_code, st); break;
+        case 1: launch_nv_mid_tile<64, 128, 4, 5>(p, out_code, st); break;
+        case 2: launch_nv_mid_tile<128, 128, 4, 4>(p, out_code, st); break;
+        default: launch_nv_mid_tile<128, 192, 2, 3>(p, out_code, st); break;
+    }
+}
+
 template <int NW>
 void launch_nv_split(const nv::Args& p, int out_code, int bias_code, bool has_bias, hipStream_t st) {
     const int units = p.tiles_m * p.tiles_n * (4 / NW);
@@ -1129,8 +1183,13 @@ extern "C" int ckh_scaled_mm_nvfp4(const void* a, const void* b, const void* sa,
     p.tiles_n = static_cast<int>(cdiv(N, nv::BN));
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     if (p.M <= kNvSkinnyMaxM) return launch_nv_skinny(p, out_code, bias_code, bias != nullptr, st);
-    const NvSplitPlan sp = nv_split_plan(M, N, K);
-    if (sp.S > 1 && workspace && workspace_bytes >= nv_split_workspace_bytes(M, N, K)) {
+    NvSplitPlan sp = nv_split_plan(M, N, K);
+    if (!workspace || workspace_bytes < nv_split_workspace_bytes(M, N, K)) sp.S = 1;
+    if (const int tile = nv_mid_tile(p.M, p.N, p.K, sp, device_cus()); tile >= 0) {
+        launch_nv_mid(p, tile, out_code, bias_code, st);
+        return check_launch("scaled_mm_nvfp4");
+    }
+    if (sp.S > 1) {
         p.splits = sp.S;
         p.ks = sp.ks;
         p.part = static_cast<float*>(workspace);

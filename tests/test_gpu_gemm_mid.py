@@ -42,6 +42,29 @@ def test_small_tiles(m, n, k, out_dtype, bias_dtype, hip):
     assert _rel(got, want) <= REL[out_dtype]
 
 
+# (m, n, k): 64 x 64 tiles (part of a line, two lines, an odd number of them), 64 x 128, 128 x 128
+# and 128 x 192
+NV_SHAPES = [(65, 33, 32), (70, 1000, 480), (200, 2001, 1312), (200, 7001, 1056), (201, 6992, 256), (300, 9003, 2080),
+             (500, 7000, 800), (500, 9004, 2112), (512, 12288, 1024)]
+
+
+@pytest.mark.parametrize("out_dtype,bias_dtype", [(torch.float32, None), (torch.bfloat16, torch.bfloat16),
+                                                  (torch.float16, torch.float32), (torch.bfloat16, None)])
+@pytest.mark.parametrize("m,n,k", NV_SHAPES)
+def test_small_tiles_nvfp4(m, n, k, out_dtype, bias_dtype, hip):
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device="cuda") * torch.exp(torch.randn(m, 1, generator=g, device="cuda"))
+    w = torch.randn(n, k, generator=g, device="cuda") * 0.02
+    bias = None if bias_dtype is None else torch.randn(n, generator=g, device="cuda").to(bias_dtype)
+    qx, sx, gx = ck.quantize_nvfp4_dynamic(x.bfloat16())
+    qw, sw, gw = ck.quantize_nvfp4_dynamic(w.bfloat16())
+    want = ck.dequantize_nvfp4(qx, gx, sx, torch.float32) @ ck.dequantize_nvfp4(qw, gw, sw, torch.float32).t()
+    want = want + (0.0 if bias is None else bias.float())
+    got = ck.scaled_mm_nvfp4(qx, qw, gx, gw, sx, sw, bias=bias, out_dtype=out_dtype)
+    assert got.shape == (m, n) and got.dtype == out_dtype
+    assert _rel(got, want) <= REL[out_dtype]
+
+
 def test_small_tiles_read_no_neighbour(hip):
     """Operands inside larger buffers full of NaN codes: nothing outside them is used."""
     m, n, k = 129, 97, 160
