@@ -61,6 +61,7 @@ SIGNATURES: dict[str, tuple] = {
     "ckh_scaled_mm_mxfp8": (_i32, [_p] * 6 + [_i64] * 3 + [_i32, _i32, _p, _i64, _u64]),
     "ckh_scaled_mm_fp8": (_i32, [_p] * 6 + [_i64] * 3 + [_i32, _i32, _p, _i64, _u64]),
     "ckh_scaled_mm_nvfp4": (_i32, [_p] * 7 + [_i64] * 3 + [_i32, _i32, _p, _i64, _u64]),
+    "ckh_scaled_mm_nvfp4_scales": (_i32, [_p] * 8 + [_i64] * 3 + [_i32, _i32, _p, _i64, _u64]),
     "ckh_scaled_mm_nvfp4_workspace_bytes": (_i64, [_i64] * 3),
     "ckh_amax_scale": (_i32, [_p, _i64, _i32, _f32, _p, _p, _u64]),
     "ckh_amax_scale_noalloc": (_i32, [_p, _i64, _i32, _f32, _p, _u64]),
@@ -386,10 +387,12 @@ def scaled_mm_nvfp4(a: torch.Tensor, b: torch.Tensor, tensor_scale_a: torch.Tens
     if ka != kb:
         raise ValueError(f"scaled_mm_nvfp4: K mismatch {2 * ka} vs {2 * kb}")
     k = 2 * ka
-    if alpha is None:
-        alpha = _scalar_on(tensor_scale_a, a.device, "tensor_scale_a") * _scalar_on(tensor_scale_b, a.device,
-                                                                                    "tensor_scale_b")
-    alpha = _scalar_on(alpha, a.device, "alpha")
+    if alpha is None:  # the kernel multiplies the two tensor scales
+        fn = "ckh_scaled_mm_nvfp4_scales"
+        scales = (_scalar_on(tensor_scale_a, a.device, "tensor_scale_a"),
+                  _scalar_on(tensor_scale_b, a.device, "tensor_scale_b"))
+    else:
+        fn, scales = "ckh_scaled_mm_nvfp4", (_scalar_on(alpha, a.device, "alpha"),)
     sa = block_scale_a.contiguous().view(torch.uint8)
     sb = block_scale_b.contiguous().view(torch.uint8)
     for name, s, rows in (("block_scale_a", sa, m), ("block_scale_b", sb, n)):
@@ -400,7 +403,7 @@ def scaled_mm_nvfp4(a: torch.Tensor, b: torch.Tensor, tensor_scale_a: torch.Tens
     out = torch.empty((m, n), dtype=out_dtype, device=a.device)
     ws, ws_bytes = _gemm_workspace(m, n, k, a.device, "ckh_scaled_mm_nvfp4_workspace_bytes")
     with _on_device(a):
-        _call("ckh_scaled_mm_nvfp4", a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), alpha.data_ptr(),
+        _call(fn, a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), *(s.data_ptr() for s in scales),
               _ptr(bias_t), out.data_ptr(), m, n, k, DTYPE_TO_CODE[out_dtype], bias_code, _ptr(ws), ws_bytes,
               _stream(a))
     return out

@@ -312,6 +312,10 @@ __device__ __forceinline__ float load1(const void* p, int64_t i) {
     else return f16_to_f(reinterpret_cast<const uint16_t*>(p)[i]);
 }
 
+// The tensor scale of an NVFP4 GEMM: *a, times *b where the caller gives the two operands'
+// scales rather than their product (forming it ahead of the GEMM was a launch of its own).
+__device__ __forceinline__ float tensor_scale(const float* a, const float* b) { return b ? a[0] * b[0] : a[0]; }
+
 // The bias of a GEMM tile's columns, staged in LDS as fp32: thread i loads element n0 + i
 // (raw bits; zeros past N, for a bias never read out of range) before the tile's operand
 // loads are issued and writes it after them, so neither waits for the other; the caller's

@@ -29,7 +29,8 @@ struct Args {
     const uint8_t* b;   // [N, K / 2]
     const uint8_t* sa;  // swizzled E4M3
     const uint8_t* sb;
-    const float* alpha;
+    const float* alpha;    // tensor scale, or the activation's
+    const float* alpha_b;  // the weight's (null: alpha is the product)
     const void* bias;  // null: none
     int bias_code;
     void* out;
@@ -235,7 +236,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mid_nv_kernel(Args p) {
     }
     if (p.bias && tid < TN) lds_bias[tid] = bias_value(bias_bits, p.bias_code);
     wait_barrier<0>();  // trailing loads have landed and every read is done: LDS is free
-    finish_tile<OUT, true, TM, TN, KG, S::WM, MT, NT>(acc, lds, lds_bias, p.alpha[0], p.bias != nullptr, p.out, p.M, p.N, m0,
+    finish_tile<OUT, true, TM, TN, KG, S::WM, MT, NT>(acc, lds, lds_bias, tensor_scale(p.alpha, p.alpha_b), p.bias != nullptr, p.out, p.M, p.N, m0,
                                               n0, wave, lane);
 }
 

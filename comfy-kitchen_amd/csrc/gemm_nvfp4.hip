@@ -96,7 +96,8 @@ struct Args {
     const uint8_t* b;
     const uint8_t* sa;
     const uint8_t* sb;
-    const float* alpha;
+    const float* alpha;    // tensor scale, or the activation's
+    const float* alpha_b;  // the weight's (null: alpha is the product)
     const void* bias;
     int bias_code;  // dtype code of bias
     void* out;
@@ -444,7 +445,7 @@ __device__ __forceinline__ void gemm_tile(const Args& p, int bid, uint8_t* lds0,
 
     // Epilogue: lane holds out[m][n..n+3] for m = r32-th row of activation tile j and
     // n = 8*gg + 4*half (+0..3) of weight tile i; times alpha, plus bias.
-    const float alpha = p.alpha[0];
+    const float alpha = tensor_scale(p.alpha, p.alpha_b);
     auto value = [&](float a, float b) { return a * alpha + b; };
     // the bias of the 4 columns from nl on (nl a multiple of 4), zeros without a bias
     auto bias4 = [&](int nl) { return BIAS ? *reinterpret_cast<const float4*>(lds_bias + nl) : float4{}; };
@@ -566,7 +567,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(Args p) {
     const int m = tm * BM + (wave & 1) * 128 + j * 32 + (lane & 31);
     const int n = tn * BN + (NW == 4 ? 0 : (U & 1) * 128) + (wave >> 1) * 32 * NW + i * 32 + 8 * g + 4 * (lane >> 5);
     if (m >= p.M || n >= p.N) return;
-    const float alpha = p.alpha[0];
+    const float alpha = tensor_scale(p.alpha, p.alpha_b);
     const float s4[4] = {v.x, v.y, v.z, v.w};
     float o[4];
 #pragma unroll
@@ -617,7 +618,8 @@ struct Args {
     const uint8_t* b;
     const uint8_t* sa;
     const uint8_t* sb;
-    const float* alpha;
+    const float* alpha;    // tensor scale, or the activation's
+    const float* alpha_b;  // the weight's (null: alpha is the product)
     const void* bias;
     void* out;
     int M, N, K;           // K in elements
@@ -892,7 +894,7 @@ __device__ __forceinline__ void skinny_tile(const Args& p) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) red[wave][u][t][v][lane] = acc[u][t][v];
     __syncthreads();
-    const float alpha = p.alpha[0];
+    const float alpha = tensor_scale(p.alpha, p.alpha_b);
     // registers v .. v + G - 1 of a group hold consecutive columns (G <= 4, v % G == 0)
     constexpr int G = RPW < 4 ? RPW : 4;
     const int v0 = RPW * wave;
@@ -1050,7 +1052,7 @@ void launch_nv_mid_tile(const midnv::Args& p, int out_code, hipStream_t st) {
 
 void launch_nv_mid(const nv::Args& q, int tile, int out_code, int bias_code, hipStream_t st) {
     midnv::Args p{};
-    p.a = q.a; p.b = q.b; p.sa = q.sa; p.sb = q.sb; p.alpha = q.alpha; p.bias = q.bias; p.out = q.out;
+    p.a = q.a; p.b = q.b; p.sa = q.sa; p.sb = q.sb; p.alpha = q.alpha; p.alpha_b = q.alpha_b; p.bias = q.bias; p.out = q.out;
     p.bias_code = bias_code;
     p.M = q.M; p.N = q.N; p.K = q.K; p.ncb = q.ncb; p.sa_rows = q.sa_rows; p.sb_rows = q.sb_rows;
     p.tiles_m = static_cast<int>(cdiv(p.M, kNvMidTiles[tile].tm));
@@ -1088,7 +1090,7 @@ void launch_nv_split(const nv::Args& p, int out_code, int bias_code, bool has_bi
 
 int launch_nv_skinny(const nv::Args& q, int out_code, int bias_code, bool has_bias, hipStream_t st) {
     nvsk::Args p{};
-    p.a = q.a; p.b = q.b; p.sa = q.sa; p.sb = q.sb; p.alpha = q.alpha; p.bias = q.bias; p.out = q.out;
+    p.a = q.a; p.b = q.b; p.sa = q.sa; p.sb = q.sb; p.alpha = q.alpha; p.alpha_b = q.alpha_b; p.bias = q.bias; p.out = q.out;
     p.M = q.M; p.N = q.N; p.K = q.K; p.ncb = q.ncb; p.sa_rows = q.sa_rows; p.sb_rows = q.sb_rows;
     // Per activation size: waves per workgroup, weight tiles per workgroup, activation tiles,
     // activation rows decoded to LDS, chunks in flight per wave.  Measured (graph-timed, K = 5120,
@@ -1149,9 +1151,12 @@ extern "C" int64_t ckh_scaled_mm_nvfp4_workspace_bytes(int64_t M, int64_t N, int
     return nv_split_workspace_bytes(M, N, K);
 }
 
-extern "C" int ckh_scaled_mm_nvfp4(const void* a, const void* b, const void* sa, const void* sb, const void* alpha,
-                                   const void* bias, void* out, int64_t M, int64_t N, int64_t K, int out_code,
-                                   int bias_code, void* workspace, int64_t workspace_bytes, uintptr_t stream) {
+namespace {
+
+// Both entry points; alpha_b null: alpha is the whole tensor scale.
+int scaled_mm_nvfp4(const void* a, const void* b, const void* sa, const void* sb, const void* alpha,
+                    const void* alpha_b, const void* bias, void* out, int64_t M, int64_t N, int64_t K, int out_code,
+                    int bias_code, void* workspace, int64_t workspace_bytes, uintptr_t stream) {
     CKH_REQUIRE(a && b && sa && sb && alpha && out, "scaled_mm_nvfp4: null pointer");
     CKH_REQUIRE(M >= 0 && N >= 0 && K > 0, "scaled_mm_nvfp4: sizes must be M, N >= 0 and K > 0");
     CKH_REQUIRE(K % 32 == 0, "scaled_mm_nvfp4: K (%lld) must be a multiple of 32", (long long)K);
@@ -1162,7 +1167,7 @@ extern "C" int ckh_scaled_mm_nvfp4(const void* a, const void* b, const void* sa,
     CKH_REQUIRE(!bias || bias_code == CKH_F32 || bias_code == CKH_F16 || bias_code == CKH_BF16,
                 "scaled_mm_nvfp4: unsupported bias dtype code %d", bias_code);
     CKH_REQUIRE(aligned(a, 16) && aligned(b, 16) && aligned(sa, 16) && aligned(sb, 16) && aligned(out, 16) &&
-                    aligned(alpha, 4) && (!workspace || aligned(workspace, 16)),
+                    aligned(alpha, 4) && aligned(alpha_b, 4) && (!workspace || aligned(workspace, 16)),
                 "scaled_mm_nvfp4: pointers misaligned");
     if (M == 0 || N == 0) return CKH_OK;
     nv::Args p{};
@@ -1171,6 +1176,7 @@ extern "C" int ckh_scaled_mm_nvfp4(const void* a, const void* b, const void* sa,
     p.sa = static_cast<const uint8_t*>(sa);
     p.sb = static_cast<const uint8_t*>(sb);
     p.alpha = static_cast<const float*>(alpha);
+    p.alpha_b = static_cast<const float*>(alpha_b);
     p.bias = bias;
     p.out = out;
     p.M = static_cast<int>(M);
@@ -1216,4 +1222,22 @@ extern "C" int ckh_scaled_mm_nvfp4(const void* a, const void* b, const void* sa,
     else LAUNCH(CKH_F32);
 #undef LAUNCH
     return check_launch("scaled_mm_nvfp4");
+}
+
+}  // namespace
+
+extern "C" int ckh_scaled_mm_nvfp4(const void* a, const void* b, const void* sa, const void* sb, const void* alpha,
+                                   const void* bias, void* out, int64_t M, int64_t N, int64_t K, int out_code,
+                                   int bias_code, void* workspace, int64_t workspace_bytes, uintptr_t stream) {
+    return scaled_mm_nvfp4(a, b, sa, sb, alpha, nullptr, bias, out, M, N, K, out_code, bias_code, workspace,
+                           workspace_bytes, stream);
+}
+
+extern "C" int ckh_scaled_mm_nvfp4_scales(const void* a, const void* b, const void* sa, const void* sb,
+                                          const void* scale_a, const void* scale_b, const void* bias, void* out,
+                                          int64_t M, int64_t N, int64_t K, int out_code, int bias_code,
+                                          void* workspace, int64_t workspace_bytes, uintptr_t stream) {
+    CKH_REQUIRE(scale_b, "scaled_mm_nvfp4: null pointer");
+    return scaled_mm_nvfp4(a, b, sa, sb, scale_a, scale_b, bias, out, M, N, K, out_code, bias_code, workspace,
+                           workspace_bytes, stream);
 }

@@ -204,6 +204,16 @@ int ckh_scaled_mm_nvfp4(const void* a, const void* b, const void* sa, const void
                         int64_t workspace_bytes, uintptr_t stream);
 
 /*
+ * ckh_scaled_mm_nvfp4 with the operands' tensor scales (one f32 each on device) in place of
+ * their product alpha: the kernel multiplies them, so a caller needs no launch to do so.
+ */
+int ckh_scaled_mm_nvfp4_scales(const void* a, const void* b, const void* sa, const void* sb,
+                               const void* scale_a, const void* scale_b, const void* bias,
+                               void* out, int64_t M, int64_t N, int64_t K, int out_code,
+                               int bias_code, void* workspace, int64_t workspace_bytes,
+                               uintptr_t stream);
+
+/*
  * Bytes of device workspace ckh_scaled_mm_nvfp4 uses at this shape to split K (0: no
  * split): grids of at most 64 output tiles of 256 x 256 with K of at least 2048 (split as
  * 256 x 128 half tiles), and grids of 65-128 tiles with K of at least 4096 when three K

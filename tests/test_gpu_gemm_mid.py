@@ -76,3 +76,14 @@ def test_small_tiles_read_no_neighbour(hip):
     one = torch.ones(1, device="cuda")
     got = ck.scaled_mm_fp8(pad[:m], pad[m + 4:m + 4 + n], one, one, out_dtype=torch.float32)
     assert _rel(got, x.float() @ w.float().t()) <= 1e-4
+
+
+@pytest.mark.parametrize("m", [3, 40, 100, 4352])
+def test_nvfp4_tensor_scales_multiplied_in_the_kernel(m, hip):
+    """Two tensor scales give the bits that their fp32 product, passed as alpha, gives: skinny,
+    small-tile and whole-tile kernels, and split-K (its reduce kernel)."""
+    for n, k in ((4000, 64), (1000, 8192)):
+        qx, sx, gx = ck.quantize_nvfp4_dynamic(torch.randn(m, k, device="cuda").bfloat16())
+        qw, sw, gw = ck.quantize_nvfp4_dynamic(torch.randn(n, k, device="cuda").bfloat16())
+        got = ck.scaled_mm_nvfp4(qx, qw, gx, gw, sx, sw, out_dtype=torch.float32)
+        assert torch.equal(got, ck.scaled_mm_nvfp4(qx, qw, gx, gw, sx, sw, alpha=gx * gw, out_dtype=torch.float32))
