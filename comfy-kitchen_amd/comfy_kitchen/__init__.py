@@ -16,7 +16,7 @@ from .exceptions import (
     NoCapableBackendError,
 )
 from .float_utils import from_blocked, swap_nibbles, to_blocked
-from .ops import DTYPE_TO_CODE
+from .ops import DTYPE_TO_CODE, _dispatch, direct
 from .registry import registry
 
 __version__ = "0.1.0"
@@ -57,13 +57,19 @@ def amax_scale(x: torch.Tensor, divisor: float) -> torch.Tensor:
     quantize (reference tensor/fp8.py:56-61, tensor/nvfp4.py:64-69) as one device-side
     reduction, so dynamic quantization needs no host round trip.
     """
-    return torch.ops.comfy_kitchen.amax_scale(x, float(divisor))
+    divisor = float(divisor)
+    if direct(x):
+        return _dispatch("amax_scale", x=x, divisor=divisor)
+    return torch.ops.comfy_kitchen.amax_scale(x, divisor)
 
 
 def quantize_per_tensor_fp8(x: torch.Tensor, scale: torch.Tensor,
                             output_type: torch.dtype = torch.float8_e4m3fn) -> torch.Tensor:
     """FP8 quantize with one fp32 scale: fp8(clamp(x * (1/scale), +-max))."""
-    return torch.ops.comfy_kitchen.quantize_fp8(x, scale, DTYPE_TO_CODE[output_type])
+    code = DTYPE_TO_CODE[output_type]
+    if direct(x, scale):
+        return _dispatch("quantize_per_tensor_fp8", x=x, scale=scale, output_type=output_type)
+    return torch.ops.comfy_kitchen.quantize_fp8(x, scale, code)
 
 
 def quantize_fp8_dynamic(x: torch.Tensor, divisor: float = 448.0,
@@ -74,13 +80,19 @@ def quantize_fp8_dynamic(x: torch.Tensor, divisor: float = 448.0,
     Not part of the reference's public API: it is the scale=None branch of the FP8 layout's
     quantize (reference tensor/fp8.py:56-61) with the reduction fused into the quantize
     launch.  The results equal amax_scale followed by quantize_per_tensor_fp8 bit for bit."""
-    return torch.ops.comfy_kitchen.quantize_fp8_dynamic(x, float(divisor), DTYPE_TO_CODE[output_type])
+    divisor, code = float(divisor), DTYPE_TO_CODE[output_type]
+    if direct(x):
+        return _dispatch("quantize_fp8_dynamic", x=x, divisor=divisor, output_type=output_type)
+    return torch.ops.comfy_kitchen.quantize_fp8_dynamic(x, divisor, code)
 
 
 def dequantize_per_tensor_fp8(x: torch.Tensor, scale: torch.Tensor,
                               output_type: torch.dtype = torch.bfloat16) -> torch.Tensor:
     """FP8 dequantize: x.to(output_type) * scale.to(output_type)."""
-    return torch.ops.comfy_kitchen.dequantize_fp8(x, scale, DTYPE_TO_CODE[output_type])
+    code = DTYPE_TO_CODE[output_type]
+    if direct(x, scale):
+        return _dispatch("dequantize_per_tensor_fp8", x=x, scale=scale, output_type=output_type)
+    return torch.ops.comfy_kitchen.dequantize_fp8(x, scale, code)
 
 
 def stochastic_rounding_fp8(x: torch.Tensor, rng: torch.Tensor,
@@ -93,6 +105,9 @@ def stochastic_rounding_fp8(x: torch.Tensor, rng: torch.Tensor,
 def quantize_nvfp4(x: torch.Tensor, per_tensor_scale: torch.Tensor, epsilon: float = 0.0,
                    pad_16x: bool = False, hi_first: bool = True) -> tuple[torch.Tensor, torch.Tensor]:
     """NVFP4: packed E2M1 codes [M, K/2] uint8 and swizzled E4M3 block-16 scales."""
+    if type(epsilon) is float and type(pad_16x) is bool and type(hi_first) is bool and direct(x, per_tensor_scale):
+        return _dispatch("quantize_nvfp4", x=x, per_tensor_scale=per_tensor_scale, epsilon=epsilon,
+                         pad_16x=pad_16x, hi_first=hi_first)
     return torch.ops.comfy_kitchen.quantize_nvfp4(x, per_tensor_scale, epsilon, pad_16x, hi_first)
 
 
@@ -105,13 +120,19 @@ def quantize_nvfp4_dynamic(x: torch.Tensor, divisor: float = 448.0 * 6.0, pad_16
     layout's quantize (reference tensor/nvfp4.py:64-69, the dynamic activation scale of
     samples/nvfp4_linear.py:55-59) with the reduction fused into the quantize launch.
     The results equal amax_scale followed by quantize_nvfp4 bit for bit."""
-    return torch.ops.comfy_kitchen.quantize_nvfp4_dynamic(x, float(divisor), pad_16x, hi_first)
+    divisor = float(divisor)
+    if type(pad_16x) is bool and type(hi_first) is bool and direct(x):
+        return _dispatch("quantize_nvfp4_dynamic", x=x, divisor=divisor, pad_16x=pad_16x, hi_first=hi_first)
+    return torch.ops.comfy_kitchen.quantize_nvfp4_dynamic(x, divisor, pad_16x, hi_first)
 
 
 def dequantize_nvfp4(qx: torch.Tensor, per_tensor_scale: torch.Tensor, block_scales: torch.Tensor,
                      output_type: torch.dtype = torch.bfloat16, hi_first: bool = True) -> torch.Tensor:
-    return torch.ops.comfy_kitchen.dequantize_nvfp4(
-        qx, per_tensor_scale, block_scales, DTYPE_TO_CODE[output_type], hi_first)
+    code = DTYPE_TO_CODE[output_type]
+    if type(hi_first) is bool and direct(qx, per_tensor_scale, block_scales):
+        return _dispatch("dequantize_nvfp4", qx=qx, per_tensor_scale=per_tensor_scale, block_scales=block_scales,
+                         output_type=output_type, hi_first=hi_first)
+    return torch.ops.comfy_kitchen.dequantize_nvfp4(qx, per_tensor_scale, block_scales, code, hi_first)
 
 
 def scaled_mm_nvfp4(a: torch.Tensor, b: torch.Tensor, tensor_scale_a: torch.Tensor,
@@ -120,26 +141,40 @@ def scaled_mm_nvfp4(a: torch.Tensor, b: torch.Tensor, tensor_scale_a: torch.Tens
                     out_dtype: torch.dtype | None = None,
                     alpha: torch.Tensor | None = None) -> torch.Tensor:
     """y = (a @ b.T) * (tensor_scale_a * tensor_scale_b) + bias on NVFP4 operands."""
-    code = DTYPE_TO_CODE[out_dtype if out_dtype is not None else torch.bfloat16]
+    out_dtype = out_dtype if out_dtype is not None else torch.bfloat16
+    code = DTYPE_TO_CODE[out_dtype]
+    if direct(a, b, tensor_scale_a, tensor_scale_b, block_scale_a, block_scale_b, bias, alpha):
+        return _dispatch("scaled_mm_nvfp4", a=a, b=b, tensor_scale_a=tensor_scale_a, tensor_scale_b=tensor_scale_b,
+                         block_scale_a=block_scale_a, block_scale_b=block_scale_b, bias=bias, out_dtype=out_dtype,
+                         alpha=alpha)
     return torch.ops.comfy_kitchen.scaled_mm_nvfp4(
         a, b, tensor_scale_a, tensor_scale_b, block_scale_a, block_scale_b, bias, code, alpha)
 
 
 def quantize_mxfp8(x: torch.Tensor, pad_32x: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
     """MXFP8: E4M3 codes [M, K] and swizzled E8M0 block-32 scales."""
+    if type(pad_32x) is bool and direct(x):
+        return _dispatch("quantize_mxfp8", x=x, pad_32x=pad_32x)
     return torch.ops.comfy_kitchen.quantize_mxfp8(x, pad_32x)
 
 
 def dequantize_mxfp8(qx: torch.Tensor, block_scales: torch.Tensor,
                      output_type: torch.dtype = torch.bfloat16) -> torch.Tensor:
-    return torch.ops.comfy_kitchen.dequantize_mxfp8(qx, block_scales, DTYPE_TO_CODE[output_type])
+    code = DTYPE_TO_CODE[output_type]
+    if direct(qx, block_scales):
+        return _dispatch("dequantize_mxfp8", qx=qx, block_scales=block_scales, output_type=output_type)
+    return torch.ops.comfy_kitchen.dequantize_mxfp8(qx, block_scales, code)
 
 
 def scaled_mm_mxfp8(a: torch.Tensor, b: torch.Tensor, block_scale_a: torch.Tensor,
                     block_scale_b: torch.Tensor, bias: torch.Tensor | None = None,
                     out_dtype: torch.dtype | None = None) -> torch.Tensor:
     """y = a @ b.T + bias on MXFP8 operands (both K-major, E8M0 block-32 scales)."""
-    code = DTYPE_TO_CODE[out_dtype if out_dtype is not None else torch.bfloat16]
+    out_dtype = out_dtype if out_dtype is not None else torch.bfloat16
+    code = DTYPE_TO_CODE[out_dtype]
+    if direct(a, b, block_scale_a, block_scale_b, bias):
+        return _dispatch("scaled_mm_mxfp8", a=a, b=b, block_scale_a=block_scale_a, block_scale_b=block_scale_b,
+                         bias=bias, out_dtype=out_dtype)
     return torch.ops.comfy_kitchen.scaled_mm_mxfp8(a, b, block_scale_a, block_scale_b, bias, code)
 
 
@@ -150,17 +185,24 @@ def scaled_mm_fp8(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor, scale
     Not part of the reference's public API: it is the matmul behind TensorCoreFP8Layout's
     linear / mm / addmm, where the reference calls torch F.scaled_mm (scaled_mm_v2.py:27-53).
     """
-    code = DTYPE_TO_CODE[out_dtype if out_dtype is not None else torch.bfloat16]
+    out_dtype = out_dtype if out_dtype is not None else torch.bfloat16
+    code = DTYPE_TO_CODE[out_dtype]
+    if direct(a, b, scale_a, scale_b, bias):
+        return _dispatch("scaled_mm_fp8", a=a, b=b, scale_a=scale_a, scale_b=scale_b, bias=bias, out_dtype=out_dtype)
     return torch.ops.comfy_kitchen.scaled_mm_fp8(a, b, scale_a, scale_b, bias, code)
 
 
 def apply_rope(xq: torch.Tensor, xk: torch.Tensor,
                freqs_cis: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """Rotate query and key by the 2x2 matrices in freqs_cis [..., head_dim/2, 2, 2]."""
+    if direct(xq, xk, freqs_cis):
+        return _dispatch("apply_rope", xq=xq, xk=xk, freqs_cis=freqs_cis)
     return torch.ops.comfy_kitchen.apply_rope(xq, xk, freqs_cis)
 
 
 def apply_rope1(x: torch.Tensor, freqs_cis: torch.Tensor) -> torch.Tensor:
+    if direct(x, freqs_cis):
+        return _dispatch("apply_rope1", x=x, freqs_cis=freqs_cis)
     return torch.ops.comfy_kitchen.apply_rope1(x, freqs_cis)
 
 

@@ -104,26 +104,18 @@ def _call(name: str, *args) -> None:
         raise RuntimeError(f"{name}: {_lib.ckh_last_error().decode(errors='replace')}")
 
 
-def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
-class _on_device:
-    """Make t's device current for the launch (a no-op when it already is)."""
-
-    def __init__(self, t: torch.Tensor):
-        self.idx = t.device.index
-        self.prev = None
-
-    def __enter__(self):
-        cur = torch.cuda.current_device()
-        if self.idx is not None and self.idx != cur:
-            self.prev = cur
-            torch.cuda.set_device(self.idx)
-
-    def __exit__(self, *exc):
-        if self.prev is not None:
-            torch.cuda.set_device(self.prev)
+def _launch(name: str, t: torch.Tensor, *args) -> None:
+    """Call entry point `name` with args and the current stream of t's device, which is made
+    current for the call (a no-op when it already is)."""
+    device = t.get_device()
+    if device == _current_device():
+        return _call(name, *args, _raw_stream(device))
+    with torch.cuda.device(device):
+        _call(name, *args, _raw_stream(device))
 
 
 def _scalar_on(t: torch.Tensor | float, device: torch.device, name: str) -> torch.Tensor:
@@ -134,9 +126,7 @@ def _scalar_on(t: torch.Tensor | float, device: torch.device, name: str) -> torc
         raise ValueError(f"{name} must have exactly one element, got shape {tuple(t.shape)}")
     if t.dtype != torch.float32:
         t = t.to(torch.float32)
-    if t.device != device:
-        t = t.to(device)
-    return t.reshape(1).contiguous()
+    return t if t.device == device else t.to(device)
 
 
 def _scalar_keep(t: torch.Tensor, device: torch.device, name: str) -> torch.Tensor:
@@ -146,9 +136,7 @@ def _scalar_keep(t: torch.Tensor, device: torch.device, name: str) -> torch.Tens
         return _scalar_on(t, device, name)
     if t.numel() != 1:
         raise ValueError(f"{name} must have exactly one element, got shape {tuple(t.shape)}")
-    if t.device != device:
-        t = t.to(device)
-    return t.reshape(1).contiguous()
+    return t if t.device == device else t.to(device)
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -160,11 +148,10 @@ def quantize_per_tensor_fp8(x: torch.Tensor, scale: torch.Tensor,
                             output_type: torch.dtype = torch.float8_e4m3fn) -> torch.Tensor:
     x = x.contiguous()
     s = _scalar_on(scale, x.device, "scale")
-    out = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-    with _on_device(x):
-        _call("ckh_quantize_fp8", x.data_ptr(), out.data_ptr(), s.data_ptr(), x.numel(),
-              DTYPE_TO_CODE[x.dtype], DTYPE_TO_CODE[output_type], _stream(x))
-    return out.view(output_type)
+    out = torch.empty(x.shape, dtype=output_type, device=x.device)
+    _launch("ckh_quantize_fp8", x, x.data_ptr(), out.data_ptr(), s.data_ptr(), x.numel(),
+            DTYPE_TO_CODE[x.dtype], DTYPE_TO_CODE[output_type])
+    return out
 
 
 def dequantize_per_tensor_fp8(x: torch.Tensor, scale: torch.Tensor,
@@ -172,9 +159,8 @@ def dequantize_per_tensor_fp8(x: torch.Tensor, scale: torch.Tensor,
     x = x.contiguous()
     s = _scalar_keep(scale, x.device, "scale")
     out = torch.empty(x.shape, dtype=output_type, device=x.device)
-    with _on_device(x):
-        _call("ckh_dequantize_fp8", x.data_ptr(), out.data_ptr(), s.data_ptr(), x.numel(),
-              DTYPE_TO_CODE[x.dtype], DTYPE_TO_CODE[output_type], DTYPE_TO_CODE[s.dtype], _stream(x))
+    _launch("ckh_dequantize_fp8", x, x.data_ptr(), out.data_ptr(), s.data_ptr(), x.numel(),
+            DTYPE_TO_CODE[x.dtype], DTYPE_TO_CODE[output_type], DTYPE_TO_CODE[s.dtype])
     return out
 
 
@@ -187,9 +173,8 @@ def amax_scale(x: torch.Tensor, divisor: float) -> torch.Tensor:
     out = torch.empty((), dtype=torch.float32, device=x.device)
     # per-workgroup partial maxima (CKH_AMAX_WORKSPACE_BYTES), from torch's allocator
     work = torch.empty(AMAX_WORKSPACE_BYTES // 4, dtype=torch.int32, device=x.device)
-    with _on_device(x):
-        _call("ckh_amax_scale", x.data_ptr(), x.numel(), DTYPE_TO_CODE[x.dtype], float(divisor), out.data_ptr(),
-              work.data_ptr(), _stream(x))
+    _launch("ckh_amax_scale", x, x.data_ptr(), x.numel(), DTYPE_TO_CODE[x.dtype], float(divisor),
+            out.data_ptr(), work.data_ptr())
     return out
 
 
@@ -200,13 +185,12 @@ def quantize_fp8_dynamic(x: torch.Tensor, divisor: float,
     x = x.contiguous()
     if x.numel() == 0:
         raise RuntimeError("quantize_fp8_dynamic: empty tensor")
-    out = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
+    out = torch.empty(x.shape, dtype=output_type, device=x.device)
     scale = torch.empty((), dtype=torch.float32, device=x.device)
     work = torch.empty(AMAX_WORKSPACE_BYTES // 4, dtype=torch.int32, device=x.device)
-    with _on_device(x):
-        _call("ckh_quantize_fp8_dynamic", x.data_ptr(), float(divisor), scale.data_ptr(), out.data_ptr(), x.numel(),
-              DTYPE_TO_CODE[x.dtype], DTYPE_TO_CODE[output_type], work.data_ptr(), _stream(x))
-    return out.view(output_type), scale
+    _launch("ckh_quantize_fp8_dynamic", x, x.data_ptr(), float(divisor), scale.data_ptr(), out.data_ptr(),
+            x.numel(), DTYPE_TO_CODE[x.dtype], DTYPE_TO_CODE[output_type], work.data_ptr())
+    return out, scale
 
 
 # --------------------------------------------------------------------------- MXFP8
@@ -219,26 +203,24 @@ def quantize_mxfp8(x: torch.Tensor, pad_32x: bool = False) -> tuple[torch.Tensor
     if cols % 32:
         raise ValueError(f"K dimension must be divisible by 32 (got {cols}); pass pad_32x=True")
     qx = torch.empty((rows, cols), dtype=torch.float8_e4m3fn, device=x.device)
-    sx = torch.empty((roundup(rows, 128), roundup(cols // 32, 4)), dtype=torch.uint8, device=x.device)
-    with _on_device(x):
-        _call("ckh_quantize_mxfp8", x.data_ptr(), qx.data_ptr(), sx.data_ptr(), rows, cols, orows, ocols,
-              DTYPE_TO_CODE[x.dtype], _stream(x))
-    return qx, sx.view(torch.float8_e8m0fnu)
+    sx = torch.empty((roundup(rows, 128), roundup(cols // 32, 4)), dtype=torch.float8_e8m0fnu, device=x.device)
+    _launch("ckh_quantize_mxfp8", x, x.data_ptr(), qx.data_ptr(), sx.data_ptr(), rows, cols, orows, ocols,
+            DTYPE_TO_CODE[x.dtype])
+    return qx, sx
 
 
 def dequantize_mxfp8(qx: torch.Tensor, block_scales: torch.Tensor,
                      output_type: torch.dtype = torch.bfloat16) -> torch.Tensor:
     qx = qx.contiguous()
     rows, cols = qx.shape
-    sc = block_scales.contiguous().view(torch.uint8)
+    sc = block_scales.contiguous()
     need = roundup(rows, 128) * roundup(cols // 32, 4)
-    if cols % 32 or sc.numel() < need:
+    if cols % 32 or sc.nbytes < need:
         raise ValueError(f"dequantize_mxfp8: qx {tuple(qx.shape)} needs K % 32 == 0 and {need} scale bytes, "
-                         f"got {sc.numel()}")
+                         f"got {sc.nbytes}")
     out = torch.empty((rows, cols), dtype=output_type, device=qx.device)
-    with _on_device(qx):
-        _call("ckh_dequantize_mxfp8", qx.data_ptr(), sc.data_ptr(), out.data_ptr(), rows, cols,
-              DTYPE_TO_CODE[output_type], _stream(qx))
+    _launch("ckh_dequantize_mxfp8", qx, qx.data_ptr(), sc.data_ptr(), out.data_ptr(), rows, cols,
+            DTYPE_TO_CODE[output_type])
     return out
 
 
@@ -254,11 +236,10 @@ def quantize_nvfp4(x: torch.Tensor, per_tensor_scale: torch.Tensor, epsilon: flo
     if cols % 16:
         raise ValueError(f"K dimension must be divisible by 16 (got {cols}); pass pad_16x=True")
     qx = torch.empty((rows, cols // 2), dtype=torch.uint8, device=x.device)
-    sx = torch.empty((roundup(rows, 128), roundup(cols // 16, 4)), dtype=torch.uint8, device=x.device)
-    with _on_device(x):
-        _call("ckh_quantize_nvfp4", x.data_ptr(), g.data_ptr(), qx.data_ptr(), sx.data_ptr(), rows, cols,
-              orows, ocols, float(epsilon), DTYPE_TO_CODE[x.dtype], int(bool(hi_first)), _stream(x))
-    return qx, sx.view(torch.float8_e4m3fn)
+    sx = torch.empty((roundup(rows, 128), roundup(cols // 16, 4)), dtype=torch.float8_e4m3fn, device=x.device)
+    _launch("ckh_quantize_nvfp4", x, x.data_ptr(), g.data_ptr(), qx.data_ptr(), sx.data_ptr(), rows, cols,
+            orows, ocols, float(epsilon), DTYPE_TO_CODE[x.dtype], int(bool(hi_first)))
+    return qx, sx
 
 
 def quantize_nvfp4_dynamic(x: torch.Tensor, divisor: float, pad_16x: bool = False,
@@ -275,14 +256,13 @@ def quantize_nvfp4_dynamic(x: torch.Tensor, divisor: float, pad_16x: bool = Fals
     if cols % 16:
         raise ValueError(f"K dimension must be divisible by 16 (got {cols}); pass pad_16x=True")
     qx = torch.empty((rows, cols // 2), dtype=torch.uint8, device=x.device)
-    sx = torch.empty((roundup(rows, 128), roundup(cols // 16, 4)), dtype=torch.uint8, device=x.device)
+    sx = torch.empty((roundup(rows, 128), roundup(cols // 16, 4)), dtype=torch.float8_e4m3fn, device=x.device)
     scale = torch.empty((), dtype=torch.float32, device=x.device)
     work = torch.empty(AMAX_WORKSPACE_BYTES // 4, dtype=torch.int32, device=x.device)
-    with _on_device(x):
-        _call("ckh_quantize_nvfp4_dynamic", x.data_ptr(), float(divisor), scale.data_ptr(), qx.data_ptr(),
-              sx.data_ptr(), rows, cols, orows, ocols, 0.0, DTYPE_TO_CODE[x.dtype], int(bool(hi_first)),
-              work.data_ptr(), _stream(x))
-    return qx, sx.view(torch.float8_e4m3fn), scale
+    _launch("ckh_quantize_nvfp4_dynamic", x, x.data_ptr(), float(divisor), scale.data_ptr(), qx.data_ptr(),
+            sx.data_ptr(), rows, cols, orows, ocols, 0.0, DTYPE_TO_CODE[x.dtype], int(bool(hi_first)),
+            work.data_ptr())
+    return qx, sx, scale
 
 
 def dequantize_nvfp4(qx: torch.Tensor, per_tensor_scale: torch.Tensor, block_scales: torch.Tensor,
@@ -291,15 +271,14 @@ def dequantize_nvfp4(qx: torch.Tensor, per_tensor_scale: torch.Tensor, block_sca
     rows, half = qx.shape
     cols = 2 * half
     g = _scalar_on(per_tensor_scale, qx.device, "per_tensor_scale")
-    sc = block_scales.contiguous().view(torch.uint8)
+    sc = block_scales.contiguous()
     need = roundup(rows, 128) * roundup(cols // 16, 4)
-    if cols % 16 or sc.numel() < need:
+    if cols % 16 or sc.nbytes < need:
         raise ValueError(f"dequantize_nvfp4: qx {tuple(qx.shape)} needs K % 16 == 0 and {need} scale bytes, "
-                         f"got {sc.numel()}")
+                         f"got {sc.nbytes}")
     out = torch.empty((rows, cols), dtype=output_type, device=qx.device)
-    with _on_device(qx):
-        _call("ckh_dequantize_nvfp4", qx.data_ptr(), g.data_ptr(), sc.data_ptr(), out.data_ptr(), rows, cols,
-              DTYPE_TO_CODE[output_type], int(bool(hi_first)), _stream(qx))
+    _launch("ckh_dequantize_nvfp4", qx, qx.data_ptr(), g.data_ptr(), sc.data_ptr(), out.data_ptr(), rows, cols,
+            DTYPE_TO_CODE[output_type], int(bool(hi_first)))
     return out
 
 
@@ -341,18 +320,16 @@ def scaled_mm_mxfp8(a: torch.Tensor, b: torch.Tensor, block_scale_a: torch.Tenso
     n, kb = b.shape
     if k != kb:
         raise ValueError(f"scaled_mm_mxfp8: K mismatch {k} vs {kb}")
-    sa = block_scale_a.contiguous().view(torch.uint8)
-    sb = block_scale_b.contiguous().view(torch.uint8)
+    sa, sb = block_scale_a.contiguous(), block_scale_b.contiguous()
     for name, s, rows in (("block_scale_a", sa, m), ("block_scale_b", sb, n)):
         need = roundup(rows, 128) * roundup(k // 32, 4)
-        if s.numel() < need:
-            raise ValueError(f"scaled_mm_mxfp8: {name} has {s.numel()} bytes, needs {need}")
+        if s.nbytes < need:
+            raise ValueError(f"scaled_mm_mxfp8: {name} has {s.nbytes} bytes, needs {need}")
     bias_t, bias_code = _bias_args(bias, n, a.device)
     out = torch.empty((m, n), dtype=out_dtype, device=a.device)
     ws, ws_bytes = _gemm_workspace(m, n, k, a.device)
-    with _on_device(a):
-        _call("ckh_scaled_mm_mxfp8", a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), _ptr(bias_t),
-              out.data_ptr(), m, n, k, DTYPE_TO_CODE[out_dtype], bias_code, _ptr(ws), ws_bytes, _stream(a))
+    _launch("ckh_scaled_mm_mxfp8", a, a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), _ptr(bias_t),
+            out.data_ptr(), m, n, k, DTYPE_TO_CODE[out_dtype], bias_code, _ptr(ws), ws_bytes)
     return out
 
 
@@ -369,9 +346,8 @@ def scaled_mm_fp8(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor, scale
     bias_t, bias_code = _bias_args(bias, n, a.device)
     out = torch.empty((m, n), dtype=out_dtype, device=a.device)
     ws, ws_bytes = _gemm_workspace(m, n, k, a.device)
-    with _on_device(a):
-        _call("ckh_scaled_mm_fp8", a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), _ptr(bias_t),
-              out.data_ptr(), m, n, k, DTYPE_TO_CODE[out_dtype], bias_code, _ptr(ws), ws_bytes, _stream(a))
+    _launch("ckh_scaled_mm_fp8", a, a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), _ptr(bias_t),
+            out.data_ptr(), m, n, k, DTYPE_TO_CODE[out_dtype], bias_code, _ptr(ws), ws_bytes)
     return out
 
 
@@ -393,19 +369,16 @@ def scaled_mm_nvfp4(a: torch.Tensor, b: torch.Tensor, tensor_scale_a: torch.Tens
                   _scalar_on(tensor_scale_b, a.device, "tensor_scale_b"))
     else:
         fn, scales = "ckh_scaled_mm_nvfp4", (_scalar_on(alpha, a.device, "alpha"),)
-    sa = block_scale_a.contiguous().view(torch.uint8)
-    sb = block_scale_b.contiguous().view(torch.uint8)
+    sa, sb = block_scale_a.contiguous(), block_scale_b.contiguous()
     for name, s, rows in (("block_scale_a", sa, m), ("block_scale_b", sb, n)):
         need = roundup(rows, 128) * roundup(k // 16, 4)
-        if s.numel() < need:
-            raise ValueError(f"scaled_mm_nvfp4: {name} has {s.numel()} bytes, needs {need}")
+        if s.nbytes < need:
+            raise ValueError(f"scaled_mm_nvfp4: {name} has {s.nbytes} bytes, needs {need}")
     bias_t, bias_code = _bias_args(bias, n, a.device)
     out = torch.empty((m, n), dtype=out_dtype, device=a.device)
     ws, ws_bytes = _gemm_workspace(m, n, k, a.device, "ckh_scaled_mm_nvfp4_workspace_bytes")
-    with _on_device(a):
-        _call(fn, a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), *(s.data_ptr() for s in scales),
-              _ptr(bias_t), out.data_ptr(), m, n, k, DTYPE_TO_CODE[out_dtype], bias_code, _ptr(ws), ws_bytes,
-              _stream(a))
+    _launch(fn, a, a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), *(s.data_ptr() for s in scales),
+            _ptr(bias_t), out.data_ptr(), m, n, k, DTYPE_TO_CODE[out_dtype], bias_code, _ptr(ws), ws_bytes)
     return out
 
 
@@ -428,10 +401,9 @@ def _rope_call(xq: torch.Tensor, xk: torch.Tensor | None, freqs_cis: torch.Tenso
         f = f.contiguous()
     oq = torch.empty_like(xq)
     ok = torch.empty_like(xk) if xk is not None else None
-    with _on_device(xq):
-        _call("ckh_apply_rope", xq.data_ptr(), _ptr(xk), f.data_ptr(), oq.data_ptr(), _ptr(ok), b, d1, d2, hd,
-              fb, fd1, fd2, xq.stride(0), xq.stride(1), xq.stride(2), f.stride(0), f.stride(1), f.stride(2),
-              DTYPE_TO_CODE[xq.dtype], DTYPE_TO_CODE[f.dtype], _stream(xq))
+    _launch("ckh_apply_rope", xq, xq.data_ptr(), _ptr(xk), f.data_ptr(), oq.data_ptr(), _ptr(ok), b, d1, d2, hd,
+            fb, fd1, fd2, xq.stride(0), xq.stride(1), xq.stride(2), f.stride(0), f.stride(1), f.stride(2),
+            DTYPE_TO_CODE[xq.dtype], DTYPE_TO_CODE[f.dtype])
     return oq, ok
 
 

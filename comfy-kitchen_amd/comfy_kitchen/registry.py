@@ -37,7 +37,7 @@ from typing import Any
 
 import torch
 
-from .constraints import FunctionConstraints, ValidationResult, validate_function_call
+from .constraints import FunctionConstraints, ParamConstraint, ValidationResult, validate_function_call
 from .exceptions import BackendNotFoundError, BackendNotImplementedError, NoCapableBackendError
 
 logger = logging.getLogger("comfy_kitchen.dispatch")
@@ -191,6 +191,48 @@ class BackendRegistry:
                 return f"{verdict.failed_param}: {verdict.failure_reason}"
         return None
 
+    def _accepts(self, rules: FunctionConstraints | None, kwargs: Mapping[str, Any]) -> bool:
+        """validate_function_call's verdict for a call it accepts, without its report; False
+        where it refuses or where this shortcut does not decide (the general path then does)."""
+        if rules is None:
+            return True
+        if rules.min_compute_capability is not None:
+            return False
+        if rules.required_arch is not None:
+            arch = self._hardware()[1]
+            if arch is None or not arch.startswith(tuple(rules.required_arch)):
+                return False
+        for name, limits in rules.params.items():
+            value = kwargs.get(name)
+            if value is None:
+                continue
+            if type(limits) is not ParamConstraint:
+                return False
+            dtypes = limits.dtypes
+            if not isinstance(value, torch.Tensor):
+                if dtypes is not None and value not in dtypes:
+                    return False
+                continue
+            if dtypes is not None and value.dtype not in dtypes:
+                return False
+            devices = limits.devices if limits.devices is not None else rules.default_devices
+            if not (value.is_cuda and "cuda" in devices) and not limits.check_device(value, rules.default_devices):
+                return False
+            for rule in limits.shape_rules:
+                if not rule.check(value):
+                    return False
+        return True
+
+    def _first_choice(self, func_name: str, kwargs: Mapping[str, Any] | None) -> Callable | None:
+        """The implementation get_capable_backend would choose when the first backend in the
+        priority order takes the call and nothing else has a say; None: ask the general path."""
+        if self._forced() or not self._order or not kwargs or logger.isEnabledFor(logging.DEBUG):
+            return None
+        slot = self._slots.get(self._order[0])
+        if slot is None or not slot.usable or func_name not in slot.table:
+            return None
+        return getattr(slot.module, func_name) if self._accepts(slot.table[func_name], kwargs) else None
+
     def _candidates(self) -> Iterator[tuple[str, bool]]:
         forced = self._forced()
         if forced:
@@ -214,6 +256,9 @@ class BackendRegistry:
                            kwargs: Mapping[str, Any] | None = None) -> Callable:
         """The callable serving `func_name`: from `backend` if named, else the selected one."""
         if not backend:
+            chosen = self._first_choice(func_name, kwargs)
+            if chosen is not None:
+                return chosen
             backend = self.get_capable_backend(func_name, kwargs)
             return getattr(self._slots[backend].module, func_name)
         slot = self._slots.get(backend, _Slot())

@@ -1,0 +1,120 @@
+"""Calls that skip the custom op: the registry's shortcut accepts exactly what the general
+validation accepts, and `direct` stands aside for everything that looks at or transforms an op."""
+import itertools
+
+import pytest
+import torch
+
+import comfy_kitchen as ck
+import comfy_kitchen.backends.hip as hb
+from comfy_kitchen.constraints import FunctionConstraints, MinDims, ParamConstraint, validate_function_call
+from comfy_kitchen.ops import direct
+from comfy_kitchen.registry import BackendRegistry
+
+ARCH = "gfx950:sramecc+:xnack-"
+TABLE = hb._build_constraints()
+DTYPES = [torch.float32, torch.bfloat16, torch.float16, torch.uint8, torch.int32, torch.float8_e4m3fn,
+          torch.float8_e5m2, torch.float8_e8m0fnu]
+SHAPES = [(), (1,), (4, 32), (3, 33), (2, 3, 4, 8), (0, 32), (1, 1, 2, 4, 2, 2)]
+
+
+def _registry(arch):
+    r = BackendRegistry()
+    r._identity = ((9, 5), arch)
+    return r
+
+
+def _values():
+    tensors = [torch.empty(s, dtype=d, device=dev) for s in SHAPES for d in DTYPES for dev in ("cpu", "meta")]
+    return [None, *tensors, *DTYPES, 1.0, 3, "x"]
+
+
+@pytest.mark.parametrize("arch", [ARCH, "gfx942", None])
+@pytest.mark.parametrize("func", sorted(TABLE))
+def test_shortcut_agrees_with_validation(func, arch):
+    """Each parameter over every dtype, rank, divisibility and device (alone), each function with
+    its devices as declared and widened to any."""
+    reg = _registry(arch)
+    rules = TABLE[func]
+    anywhere = FunctionConstraints(
+        params={n: ParamConstraint(p.dtypes, frozenset({"*"}), p.shape_rules) for n, p in rules.params.items()},
+        default_devices=frozenset({"*"}), required_arch=rules.required_arch)
+    accepted = 0
+    for r in (rules, anywhere):
+        for name, value in itertools.product(r.params, _values()):
+            want = validate_function_call(r, {name: value}, compute_capability=(9, 5), arch=arch).success
+            assert reg._accepts(r, {name: value}) == want, (func, name, value)
+            accepted += want
+    assert accepted > 0 or arch != ARCH
+
+
+def test_shortcut_leaves_what_it_does_not_decide():
+    class Odd(ParamConstraint):
+        def check_dtype(self, value):
+            return False
+
+    reg = _registry(ARCH)
+    x = torch.zeros(2, 2)
+    assert reg._accepts(None, {"x": x})
+    assert not reg._accepts(FunctionConstraints(params={"x": Odd()}), {"x": x})
+    assert not reg._accepts(FunctionConstraints(min_compute_capability=(8, 0)), {"x": x})
+    assert not reg._accepts(FunctionConstraints(params={"x": ParamConstraint(shape_rules=(MinDims(3),))}), {"x": x})
+
+
+def test_cpu_and_odd_arguments_take_the_custom_op():
+    x = torch.zeros(4, 32)
+    assert not direct(x) and not direct(1.0) and not direct(None)
+    with pytest.raises(Exception):
+        ck.quantize_mxfp8(x)
+
+
+@pytest.mark.gpu
+def test_direct_conditions(hip):
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x = torch.randn(64, 128, device="cuda").bfloat16()
+    assert direct(x) and direct(x, None, torch.nn.Parameter(x, requires_grad=False)) and direct(x, x.cpu())
+    grad = x.clone().requires_grad_()
+    assert not direct(grad) and not direct(x, grad)
+    with torch.no_grad():
+        assert direct(grad)
+    assert not direct(x.cpu()) and not direct(x, 1.0)
+    with Mode():
+        assert not direct(x)
+    with FakeTensorMode() as m:
+        assert not direct(m.from_tensor(x))
+    with torch.autograd.forward_ad.dual_level():
+        assert not direct(x)
+    with torch.autograd.profiler.profile():
+        assert not direct(x)
+    seen = []
+    torch.vmap(lambda v: (seen.append(direct(x)), v)[1])(x)
+    torch.jit.trace(lambda v: (seen.append(direct(v)), v + 1)[1], (x,), check_trace=False)
+    assert seen and not any(seen)
+
+
+@pytest.mark.gpu
+def test_direct_equals_custom_op(hip):
+    """The same results by either way, on another stream too, and a gradient is refused as before."""
+    x = torch.randn(70, 160, device="cuda").bfloat16()
+    op = torch.ops.comfy_kitchen
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        q, s = ck.quantize_mxfp8(x, pad_32x=True)
+    torch.cuda.current_stream().wait_stream(side)
+    oq, os = op.quantize_mxfp8(x, True)
+    assert torch.equal(q.view(torch.uint8), oq.view(torch.uint8)) and torch.equal(s.view(torch.uint8), os.view(torch.uint8))
+    assert q.dtype == oq.dtype and s.dtype == os.dtype and s.shape == os.shape
+    assert torch.equal(ck.scaled_mm_mxfp8(q, q, s, s), op.scaled_mm_mxfp8(q, q, s, s, None, 2))
+    for tensors in (ck.quantize_nvfp4_dynamic(x), ck.quantize_fp8_dynamic(x)):
+        assert all(type(t) is torch.Tensor and not t.requires_grad for t in tensors)
+    y = ck.dequantize_per_tensor_fp8(ck.quantize_per_tensor_fp8(x.clone().requires_grad_(), torch.ones(1, device="cuda")),
+                                     torch.ones(1, device="cuda"))
+    with pytest.raises(RuntimeError):
+        y.float().sum().backward()
