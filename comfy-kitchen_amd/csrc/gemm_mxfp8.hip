@@ -113,7 +113,6 @@ struct Args {
     const uint8_t* sa;  // swizzled E8M0, [roundup(M,128), ncb*4]
     const uint8_t* sb;
     const void* bias;
-    int bias_code;      // dtype code of bias
     void* out;
     int M, N, K;
     int ncb;               // scale column blocks: ceil(K/32/4)
@@ -129,6 +128,7 @@ struct Args {
     // [s * ks, min((s + 1) * ks, KT)) of tile L and writes its fp32 partial tile to part
     int splits, ks;
     float* part;
+    int bias_code;  // dtype code of bias
 };
 
 // fp32 values of one partial tile in the workspace (256 x 256)
@@ -809,28 +809,19 @@ __device__ __forceinline__ v8i staged_frag(const uint8_t* st, int r, int h, int 
     return v8i{(int)x[0], (int)x[1], (int)x[2], (int)x[3], (int)y[0], (int)y[1], (int)y[2], (int)y[3]};
 }
 
-// Offset of this lane's piece p (0, 1) of the step at k0 for a direct (unstaged) operand
-// load: bytes k0 + 32 p + 16 h of its row; past K it reads zeros.
-__device__ __forceinline__ uint32_t piece_off(uint32_t row_off, int k0, int p, int h, int K) {
-    const int k = k0 + 32 * p + 16 * h;
-    return k < K ? row_off + static_cast<uint32_t>(k) : 0x80000000u;
-}
-
-// One chunk's register-held operands: scale words and (unstaged activation) fragments.
+// One chunk's scale words.
 template <int MT, int NT>
 struct SkRegs {
     uint32_t swb[NT][kSkChunk / 2], swa[MT][kSkChunk / 2];
-    v4u al[MT][kSkChunk][2];
 };
 
 // WV: waves per workgroup, each taking every WV-th K chunk.
 // NT: 32-row weight tiles per workgroup (1 or 2); each activation fragment feeds NT MFMAs.
 // MT: 32-row activation tiles (M <= 32 MT).
-// AR: activation rows staged through LDS like the weight (8 or 16, >= M, one M-tile), or 0:
-// the activation's fragments are loaded straight into registers.
+// AR: activation rows staged through LDS like the weight (>= M).
 template <int OUT, int BIAS, bool UNIT, int WV, int NT, int MT, int AR>
 __global__ __launch_bounds__(64 * WV) void gemm_skinny_kernel(Args p) {
-    static_assert(AR == 0 || (AR % kSkRpl == 0 && AR <= 32 * MT && AR > 32 * (MT - 1)),
+    static_assert(AR % kSkRpl == 0 && AR <= 32 * MT && AR > 32 * (MT - 1),
                   "staged activation rows: within the MT tiles, a multiple of the rows per load");
     static_assert(16 % WV == 0, "each wave stores 16 / WV accumulator registers");
     constexpr int WR = 32 * NT;                   // weight rows of the workgroup
@@ -845,17 +836,11 @@ __global__ __launch_bounds__(64 * WV) void gemm_skinny_kernel(Args p) {
 
     const __amdgpu_buffer_rsrc_t rb =
         buffer_rsrc(p.b + static_cast<int64_t>(n0) * p.K, static_cast<uint32_t>(min(WR, p.N - n0)) * p.K);
-    __amdgpu_buffer_rsrc_t ra[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-        ra[t] = buffer_rsrc(p.a + static_cast<int64_t>(32 * t) * p.K,
-                            static_cast<uint32_t>(max(0, min(32, p.M - 32 * t))) * p.K);
-    // the staged activation rows (AR > 0): rows past M read as zeros
+    // the staged activation rows: rows past M read as zeros
     const __amdgpu_buffer_rsrc_t ras = buffer_rsrc(p.a, static_cast<uint32_t>(max(0, min(AR, p.M))) * p.K);
     // per-tensor mode: no scale tensors (zero-sized descriptors, never loaded)
     const __amdgpu_buffer_rsrc_t rsb = buffer_rsrc(p.sb, UNIT ? 0u : static_cast<uint32_t>(p.sb_rows) * p.ncb * 4);
     const __amdgpu_buffer_rsrc_t rsa = buffer_rsrc(p.sa, UNIT ? 0u : static_cast<uint32_t>(p.sa_rows) * p.ncb * 4);
-    const uint32_t row_off = static_cast<uint32_t>(r * p.K);
     // scale word of row r (of the 32-row group) in column block cb: swizzled offset
     // ((row/128 * ncb + cb) * 32 + row%32) * 16 + ((row%128)/32) * 4
     uint32_t sb_row[NT];
@@ -868,15 +853,14 @@ __global__ __launch_bounds__(64 * WV) void gemm_skinny_kernel(Args p) {
     const int KT = (p.K + 63) / 64;
     const int NC = (KT + kSkChunk - 1) / kSkChunk;
 
-    // issue chunk c's loads: weight (and staged activation) rows to LDS buffer `buf`, scale
-    // words and unstaged activation fragments to R
+    // issue chunk c's loads: weight and activation rows to LDS, scale words to R
     uint8_t* stb = stage + wave * WST;  // this wave's staged rows: weight, then activation
     auto issue = [&](int c, SkRegs<MT, NT>& R) {
         const int s0 = c * kSkChunk;
         // the weight is read once (nontemporal); the activation, which every workgroup
         // reads, stays cached
         stage_rows256<WR / kSkRpl, kAuxNontemporal>(rb, stb, p.K, s0 * 64, lane);
-        if constexpr (AR > 0) stage_rows256<AR / kSkRpl, 0>(ras, stb + WR * kSkRow, p.K, s0 * 64, lane);
+        stage_rows256<AR / kSkRpl, 0>(ras, stb + WR * kSkRow, p.K, s0 * 64, lane);
         if constexpr (!UNIT) {
 #pragma unroll
             for (int u = 0; u < kSkChunk / 2; ++u) {
@@ -889,16 +873,6 @@ __global__ __launch_bounds__(64 * WV) void gemm_skinny_kernel(Args p) {
                 for (int t = 0; t < MT; ++t)
                     R.swa[t][u] = __builtin_amdgcn_raw_buffer_load_b32(rsa, sa_row + t * 4 + cbo, 0, 0);
             }
-        }
-        if constexpr (AR == 0) {
-#pragma unroll
-            for (int t = 0; t < MT; ++t)
-#pragma unroll
-                for (int j = 0; j < kSkChunk; ++j)
-#pragma unroll
-                    for (int q = 0; q < 2; ++q)
-                        R.al[t][j][q] = __builtin_amdgcn_raw_buffer_load_b128(
-                            ra[t], piece_off(row_off, (s0 + j) * 64, q, h, p.K), 0, 0);
         }
     };
 
@@ -921,14 +895,9 @@ __global__ __launch_bounds__(64 * WV) void gemm_skinny_kernel(Args p) {
             v8i fa[MT];
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
-                if constexpr (AR > 0) {
-                    const int row = 32 * t + r;
-                    fa[t] = staged_frag(stb + WR * kSkRow, row < AR ? row : 0, h, j);
-                    if (row >= AR) fa[t] = v8i{};
-                } else {
-                    const v4u u = cur.al[t][j][0], w = cur.al[t][j][1];
-                    fa[t] = v8i{(int)u[0], (int)u[1], (int)u[2], (int)u[3], (int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-                }
+                const int row = 32 * t + r;
+                fa[t] = staged_frag(stb + WR * kSkRow, row < AR ? row : 0, h, j);
+                if (row >= AR) fa[t] = v8i{};
             }
 #pragma unroll
             for (int u = 0; u < NT; ++u) {
@@ -1029,6 +998,8 @@ void launch_grid(const mx::Args& p, unsigned wgs, int out_code, bool has_bias, h
 
 // Activations of at most kSkinnyMaxM rows take the skinny kernel (mxsk::gemm_skinny_kernel).
 constexpr int kSkinnyMaxM = 64;
+// From 17 rows and this N on, small tiles serve them instead (skinny_tile).
+constexpr int kSkinnySmallN = 8192;
 
 template <bool UNIT>
 int launch_skinny(const mx::Args& q, int out_code, int bias_code, bool has_bias, hipStream_t st) {
@@ -1037,34 +1008,22 @@ int launch_skinny(const mx::Args& q, int out_code, int bias_code, bool has_bias,
     p.M = q.M; p.N = q.N; p.K = q.K; p.ncb = q.ncb; p.sa_rows = q.sa_rows; p.sb_rows = q.sb_rows;
     p.tsa = q.tsa; p.tsb = q.tsb;
     // per activation size: waves per workgroup, weight tiles per workgroup, activation tiles,
-    // staged activation rows (measured on N = 18432, K = 3072: M = 1 12.7 us, M = 16 15.4 us,
-    // M = 32 20.5 us, M = 64 26.4 us, the last two with the activation fragments loaded
-    // straight into registers).  With 16 activation rows the waves per workgroup
-    // follow N: 2 waves when there are at least 256 workgroups (M = 16, N = 18432: 14.6
-    // against 15.4 us with 4), 8 when there are fewer than 128 (N = 3072, K = 12288: 16.6
-    // against 17.2 us; with 2 waves 25.9 us).  From 17 rows on, staging the activation
-    // through LDS too (32 or 64 rows) pays where the workgroups stay small enough in LDS to
-    // share CUs (same process, against the register-loaded fragments): M = 32, N = 18432
-    // 17.3 against 20.5 us (4 waves, one weight tile); N = 5120, K = 5120 10.8 against 16.5
-    // (8 waves); M = 64, N = 18432 21.7 against 26.3 (2 waves, two tiles); N = 5120,
-    // K = 13824 29.3 against 47.4 and N = 3072, K = 12288 25.4 against 42.1 (4 waves, one
-    // tile); for N from 8192 to 16383 two weight tiles with 32 staged rows (M = 24,
-    // N = 13824 17.2 against 17.8) or register-loaded fragments (M = 48: 21.0, staged 64 rows
-    // 21.0 with 4 waves, 24.4 with 2).  With 33-64 rows and N from 16384 on the choice
-    // follows how many workgroups one round holds (same process): 4 waves and two weight
-    // tiles (128 KB of LDS, one workgroup per CU) while N / 64 <= 256 (M = 64, N = 16384,
-    // K = 5120 22.6 against 25.7 us; K = 3072 16.0 against 17.8); else 2 waves and one tile
-    // (48 KB, three per CU) up to N = 24576 with K <= 4096 (M = 64, N = 18432, K = 3072 20.6
-    // against 21.6; M = 40, N = 24576 19.9 against 22.3; at K = 5120 33.8 against 33.3);
-    // else 2 waves and two tiles (N = 32768: 25.2 against 29.1 and 34.5).  17-32 rows follow the
-    // same rule (same process, against 4 waves and one tile): N = 16384, K = 5120 18.7 against
-    // 19.8 us; M = 32, N = 18432, K = 3072 16.4 against 17.3; M = 20, N = 32768 20.2 against 22.0;
-    // at K = 12288 4 waves and one tile stay (57.4 against 57.7).  With 4-8 rows and N above
-    // 16384, 2 waves rather than 8 (M = 8, N = 18432, K = 3072 13.4 against 14.5 us; N = 24576
-    // 14.9 against 15.8; M = 4 13.1 against 13.6; M = 1 and 2 and N = 16384 equal).  The NVFP4
-    // skinny kernel's form (128-byte chunks, two in flight per wave) measured slower here, where a
-    // chunk costs only a few MFMAs: M = 1 14.5 against 12.9 us, M = 16 15.9 against 15.5, M = 64
-    // 29.6 against 26.5 (same process).
+    // staged activation rows (measured on N = 18432, K = 3072: M = 1 12.7 us, M = 16 15.4 us).
+    // With 16 activation rows the waves per workgroup follow N: 2 waves when there are at least
+    // 256 workgroups (M = 16, N = 18432: 14.6 against 15.4 us with 4), 8 when there are fewer than
+    // 128 (N = 3072, K = 12288: 16.6 against 17.2 us; with 2 waves 25.9 us).  With 4-8 rows and N
+    // above 16384, 2 waves rather than 8 (M = 8, N = 18432, K = 3072 13.4 against 14.5 us; N =
+    // 24576 14.9 against 15.8; M = 4 13.1 against 13.6; M = 1 and 2 and N = 16384 equal).  From 17
+    // rows on this kernel serves what skinny_tile leaves: N below 8192, where its waves' split of K
+    // keeps more of the chip busy than small tiles would (32 x 5120 x 5120 11.6 against 16.1 us,
+    // 64 x 5120 x 12288 27.7 against 37.0); 17-32 rows with a short K (2 waves and one tile up to N
+    // = 24576: 20 x 18432 x 3072 16.4 against 17.3 with 4 waves; 2 waves and two tiles beyond: 20 x
+    // 32768 x 3072 20.2 against 22.0); and N beyond one round of 64 x 128 tiles.  There the
+    // activation is staged through LDS too, 32 or 64 rows (N = 5120, K = 5120, M = 32 10.8
+    // against 16.5 with the fragments loaded into registers; M = 64, K = 13824 29.3 against 47.4).
+    // The NVFP4 skinny kernel's form (128-byte chunks, two in flight per wave) measured slower
+    // here, where a chunk costs only a few MFMAs: M = 1 14.5 against 12.9 us, M = 16 15.9 against
+    // 15.5, M = 64 29.6 against 26.5 (same process).
 #define LAUNCH(O, B, WV, NT, MT, AR)                                                              \
     hipLaunchKernelGGL((mxsk::gemm_skinny_kernel<O, B, UNIT, WV, NT, MT, AR>),                    \
                        dim3(static_cast<unsigned>(cdiv(q.N, 32 * NT))), dim3(64 * WV), 0, st, p)
@@ -1075,16 +1034,11 @@ int launch_skinny(const mx::Args& q, int out_code, int bias_code, bool has_bias,
         else if (p.M <= 16 && p.N >= 8192) LAUNCH(O, B, 2, 1, 1, 16);  \
         else if (p.M <= 16 && p.N >= 4096) LAUNCH(O, B, 4, 1, 1, 16);  \
         else if (p.M <= 16) LAUNCH(O, B, 8, 1, 1, 16);                 \
-        else if (p.M <= 32 && p.N >= 16384 && p.N <= 16384) LAUNCH(O, B, 4, 2, 1, 32); \
-        else if (p.M <= 32 && p.N >= 16384 && p.N <= 24576 && p.K <= 4096) LAUNCH(O, B, 2, 1, 1, 32); \
-        else if (p.M <= 32 && p.N > 24576) LAUNCH(O, B, 2, 2, 1, 32);   \
-        else if (p.M <= 32 && p.N >= 16384) LAUNCH(O, B, 4, 1, 1, 32); \
-        else if (p.M <= 32 && p.N >= 8192) LAUNCH(O, B, 4, 2, 1, 32);  \
+        else if (p.M <= 32 && p.N > 24576) LAUNCH(O, B, 2, 2, 1, 32);  \
+        else if (p.M <= 32 && p.N > 16384) LAUNCH(O, B, 2, 1, 1, 32);  \
+        else if (p.M <= 32 && p.N >= kSkinnySmallN) LAUNCH(O, B, 4, 2, 1, 32); \
         else if (p.M <= 32) LAUNCH(O, B, 8, 1, 1, 32);                 \
-        else if (p.N >= 16384 && p.N <= 16384) LAUNCH(O, B, 4, 2, 2, 64); \
-        else if (p.N >= 16384 && p.N <= 24576 && p.K <= 4096) LAUNCH(O, B, 2, 1, 2, 64); \
-        else if (p.N >= 16384) LAUNCH(O, B, 2, 2, 2, 64);              \
-        else if (p.N >= 8192) LAUNCH(O, B, 4, 2, 2, 0);                \
+        else if (p.N >= kSkinnySmallN) LAUNCH(O, B, 2, 2, 2, 64);      \
         else LAUNCH(O, B, 4, 1, 2, 64);                                \
     } while (0)
 #define BY_BIAS(O)                                          \
@@ -1189,7 +1143,8 @@ void launch_split(mx::Args p, int out_code, int bias_code, bool has_bias, hipStr
 struct MidTile {
     int tm, tn;
 };
-constexpr MidTile kMidTiles[] = {{64, 64}, {128, 64}, {128, 96}, {128, 128}, {128, 160}, {128, 192}};
+constexpr MidTile kMidTiles[] = {{64, 64}, {128, 64}, {128, 96}, {128, 128}, {128, 160}, {128, 192}, {64, 128}};
+constexpr int kMidWide = 6;  // 64 x 128, for at most 64 rows only (mid_tile looks at those before it)
 
 // Index of the small tile to use, or -1: the estimated time (us) of the first that fits against
 // that of the 256 x 256 kernel.  Fitted to the same shapes:
@@ -1197,15 +1152,35 @@ constexpr MidTile kMidTiles[] = {{64, 64}, {128, 64}, {128, 96}, {128, 128}, {12
 //   split-K      14.7 + 0.575 per stage of a K range in half tiles, 1.09 in full tiles (two
 //                launches; 200 x 5120 x 13824, six ranges of 36: 35.4 measured, small tiles 50);
 //   half tiles   6.2 + 0.4 per stage of K (200 x 21504 x 512: 9.5 measured, small tiles 12.1).
+// With K not a multiple of 128 a stage's piece of a row lies in two cache lines, and lines are
+// what a CU's intake is counted in: the terms per stage of the one-launch forms take 1.45 x (84 x
+// 12624 x 9824 53.1 against 38.9, 360 x 9584 x 2400 23.6 against 17.3), 1.1 x where more than 6
+// tiles share a weight row, which then comes from L2 (691 x 1312 x 5824 16.2 against 17.5).  118 x
+// 2448 x 6304: small tiles 25.0, split-K 21.0; 460 x 3112 x 9312 43.5 and 37.5.
 int mid_tile(int M, int N, int K, const SplitPlan& sp, int cus) {
-    for (int i = 0; i < static_cast<int>(sizeof(kMidTiles) / sizeof(kMidTiles[0])); ++i) {
+    for (int i = 0; i < kMidWide; ++i) {
         const MidTile t = kMidTiles[i];
         if (cdiv(M, t.tm) * cdiv(N, t.tn) > cus) continue;
         const double rows = t.tm + t.tn;
-        const double mid = 2.0 + 0.0165 * rows + 0.00228 * rows * static_cast<double>(cdiv(K, 128));
-        const double big = sp.S > 1 ? 14.7 + (sp.nw == 2 ? 0.575 : 1.09) * sp.ks : 6.2 + 0.4 * static_cast<double>(cdiv(K, mx::BK));
+        const double lines = K % 128 == 0 ? 1.0 : cdiv(M, t.tm) <= 6 ? 1.45 : 1.1;
+        const double mid = 2.0 + 0.0165 * rows + 0.00228 * rows * lines * static_cast<double>(cdiv(K, 128));
+        const double big = sp.S > 1 ? 14.7 + (sp.nw == 2 ? 0.575 : 1.09) * sp.ks
+                                    : 6.2 + 0.4 * lines * static_cast<double>(cdiv(K, mx::BK));
         return mid < big ? i : -1;
     }
+    return -1;
+}
+
+// The small tile for at most 64 rows, or -1 for the skinny kernel: from 17 rows and N = 8192 on,
+// 64 x 64 or 64 x 128, whichever fits in one round (graph-timed, against the skinny kernel: 24 x
+// 8192 x 5120 16.3 / 17.5 us, 48 x 12288 x 3072 13.0 / 17.1, 64 x 8192 x 12288 37.7 / 46.0, 33 x
+// 18432 x 3072 18.0 / 21.0, 64 x 24576 x 5120 33.6 / 40.3; with 16 rows level).  With 17-32 rows
+// a short K leaves the ring's fill and the one workgroup per CU in view: 32 x 9000 x 512 5.5 / 5.3,
+// 17 x 21504 x 3072 18.7 / 16.5, but 32 x 16384 x 3072 12.8 / 14.3, 17 x 21504 x 5120 26.3 / 30.3.
+int skinny_tile(int M, int N, int K, int cus) {
+    if (M <= 16 || N < kSkinnySmallN) return -1;
+    if (cdiv(N, 64) <= cus) return M <= 32 && K < 1024 ? -1 : 0;
+    if (cdiv(N, 128) <= cus) return M <= 32 && K <= 4096 ? -1 : kMidWide;
     return -1;
 }
 
@@ -1234,7 +1209,8 @@ void launch_mid(const mx::Args& q, int tile, int out_code, int bias_code, bool h
         case 2: launch_mid_tile<UNIT, 128, 96, 4>(p, out_code, st); break;
         case 3: launch_mid_tile<UNIT, 128, 128, 4>(p, out_code, st); break;
         case 4: launch_mid_tile<UNIT, 128, 160, 3>(p, out_code, st); break;
-        default: launch_mid_tile<UNIT, 128, 192, 3>(p, out_code, st); break;
+        case 5: launch_mid_tile<UNIT, 128, 192, 3>(p, out_code, st); break;
+        default: launch_mid_tile<UNIT, 64, 128, 5>(p, out_code, st); break;
     }
 }
 
@@ -1247,10 +1223,15 @@ void launch_mid(const mx::Args& q, int tile, int out_code, int bias_code, bool h
 template <bool UNIT>
 int launch_gemm(mx::Args p, int out_code, int bias_code, bool has_bias, void* workspace, int64_t workspace_bytes,
                 hipStream_t st) {
-    if (p.M <= kSkinnyMaxM) return launch_skinny<UNIT>(p, out_code, bias_code, has_bias, st);
+    const int cus = device_cus();
+    if (p.M <= kSkinnyMaxM) {
+        const int tile = skinny_tile(p.M, p.N, p.K, cus);
+        if (tile < 0) return launch_skinny<UNIT>(p, out_code, bias_code, has_bias, st);
+        launch_mid<UNIT>(p, tile, out_code, bias_code, has_bias, st);
+        return check_launch(UNIT ? "scaled_mm_fp8" : "scaled_mm_mxfp8");
+    }
     SplitPlan sp = split_plan(p.M, p.N, p.K);
     if (!workspace || workspace_bytes < split_workspace_bytes(p.M, p.N, p.K)) sp.S = 1;
-    const int cus = device_cus();
     if (const int tile = mid_tile(p.M, p.N, p.K, sp, cus); tile >= 0) {
         launch_mid<UNIT>(p, tile, out_code, bias_code, has_bias, st);
         return check_launch(UNIT ? "scaled_mm_fp8" : "scaled_mm_mxfp8");

@@ -97,9 +97,7 @@ struct Args {
     const uint8_t* sa;
     const uint8_t* sb;
     const float* alpha;    // tensor scale, or the activation's
-    const float* alpha_b;  // the weight's (null: alpha is the product)
     const void* bias;
-    int bias_code;  // dtype code of bias
     void* out;
     int M, N, K;  // K in elements
     int ncb;      // scale word columns: ceil(K/16/4)
@@ -111,6 +109,8 @@ struct Args {
     // [s * ks, min((s + 1) * ks, NG)) of tile (or half tile) U and writes its fp32 partial
     int splits, ks;
     float* part;
+    int bias_code;         // dtype code of bias
+    const float* alpha_b;  // the weight's tensor scale (null: alpha is the product)
 };
 
 // fp32 values of one partial tile in the workspace (256 x 256, or two 256 x 128 halves)
@@ -1028,14 +1028,25 @@ constexpr NvMidTile kNvMidTiles[] = {{64, 64, 5.0, 0.62}, {64, 128, 6.2, 0.8}, {
 // half tiles without a split 8.5 + 2.4 per group.  It took the slower form on 12 of the 200, by
 // 20% at most (768 x 1024 x 8192, where both formats' estimates are 24.5), and the small tiles
 // gained 1.39 x over all: 256 x 13824 x 5120 50.4 -> 41.9 us, 300 x 4096 x 4096 33.5 -> 19.7,
-// 128 x 3072 x 3072 21.7 -> 12.5, 65 x 5120 x 2048 22.4 -> 10.3.
+// 128 x 3072 x 3072 21.7 -> 12.5, 65 x 5120 x 2048 22.4 -> 10.3.  Rows that do not start on a
+// cache line (K not a multiple of 256) take 6% longer (60 more shapes: 1.08 x the estimate in the
+// mean; 239 x 8824 x 4768 38.6, split-K 37.9).
+// At most 64 rows: 64 x 64 or 64 x 128 from 33 rows and N = 8192 on, K up to 8192 (graph-timed,
+// against the skinny kernel: 48 x 8192 x 3072 12.2 / 14.3 us, 64 x 12288 x 5120 17.7 / 20.8, 33 x
+// 18432 x 3072 16.3 / 21.5; with 32 rows 32 x 12288 x 3072 12.7 / 11.5, with K = 12288 33 x 8192
+// 32.5 / 30.9).
 int nv_mid_tile(int M, int N, int K, const NvSplitPlan& sp, int cus) {
+    if (M <= kNvSkinnyMaxM) {
+        if (M <= 32 || N < 8192 || K > 8192) return -1;
+        return cdiv(N, 64) <= cus ? 0 : cdiv(N, 128) <= cus ? 1 : -1;
+    }
     const double groups = static_cast<double>(cdiv(K, 256));
+    const double lines = K % 256 ? 1.06 : 1.0;
     for (int i = 0; i < static_cast<int>(sizeof(kNvMidTiles) / sizeof(kNvMidTiles[0])); ++i) {
         const NvMidTile& t = kNvMidTiles[i];
         if (cdiv(M, t.tm) * cdiv(N, t.tn) > cus) continue;
         const double big = sp.S > 1 ? 14.0 + (sp.nw == 2 ? 2.6 : 4.5) * sp.ks : 8.5 + 2.4 * groups;
-        return t.base + t.line * groups < big ? i : -1;
+        return (t.base + t.line * groups) * lines < big ? i : -1;
     }
     return -1;
 }
@@ -1188,13 +1199,13 @@ int scaled_mm_nvfp4(const void* a, const void* b, const void* sa, const void* sb
     p.tiles_m = static_cast<int>(cdiv(M, nv::BM));
     p.tiles_n = static_cast<int>(cdiv(N, nv::BN));
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    if (p.M <= kNvSkinnyMaxM) return launch_nv_skinny(p, out_code, bias_code, bias != nullptr, st);
     NvSplitPlan sp = nv_split_plan(M, N, K);
     if (!workspace || workspace_bytes < nv_split_workspace_bytes(M, N, K)) sp.S = 1;
     if (const int tile = nv_mid_tile(p.M, p.N, p.K, sp, device_cus()); tile >= 0) {
         launch_nv_mid(p, tile, out_code, bias_code, st);
         return check_launch("scaled_mm_nvfp4");
     }
+    if (p.M <= kNvSkinnyMaxM) return launch_nv_skinny(p, out_code, bias_code, bias != nullptr, st);
     if (sp.S > 1) {
         p.splits = sp.S;
         p.ks = sp.ks;

@@ -12,8 +12,9 @@ pytestmark = pytest.mark.gpu
 # fp32 output: the order of the fp32 sums; 16-bit outputs: one rounding (2^-9 and 2^-12 relative)
 REL = {torch.float32: 1e-4, torch.float16: 1e-3, torch.bfloat16: 4e-3}
 
-# (m, n, k): 64 x 64 tiles (one stage, three stages, many), then 128 x 64, 96, 128, 160, 192
-SHAPES = [(65, 33, 32), (70, 1000, 352), (200, 2001, 1152), (200, 7001, 1056), (201, 6992, 128), (300, 7001, 1120),
+# (m, n, k): at most 64 rows (64 x 64, then 64 x 128), 64 x 64 tiles (one stage, three stages,
+# many), then 64 x 128 or 128 x 64, 128 x 96, 128, 160, 192
+SHAPES = [(17, 8200, 1056), (33, 8192, 96), (64, 16384, 160), (33, 17001, 224), (65, 33, 32), (70, 1000, 352), (200, 2001, 1152), (200, 7001, 1056), (201, 6992, 128), (300, 7001, 1120),
           (300, 9003, 2080), (500, 9008, 2080), (500, 9004, 2112), (500, 11001, 4128), (512, 12288, 4096)]
 
 
@@ -44,7 +45,7 @@ def test_small_tiles(m, n, k, out_dtype, bias_dtype, hip):
 
 # (m, n, k): 64 x 64 tiles (part of a line, two lines, an odd number of them), 64 x 128, 128 x 128
 # and 128 x 192
-NV_SHAPES = [(65, 33, 32), (70, 1000, 480), (200, 2001, 1312), (200, 7001, 1056), (201, 6992, 256), (300, 9003, 2080),
+NV_SHAPES = [(33, 8200, 96), (64, 17001, 544), (65, 33, 32), (70, 1000, 480), (200, 2001, 1312), (200, 7001, 1056), (201, 6992, 256), (300, 9003, 2080),
              (500, 7000, 800), (500, 9004, 2112), (512, 12288, 1024)]
 
 
