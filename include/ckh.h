@@ -140,8 +140,9 @@ int ckh_apply_rope(const void* xq, const void* xk, const void* freqs, void* xq_o
                    int freqs_code, uintptr_t stream);
 
 /*
- * Bytes of device workspace ckh_scaled_mm_mxfp8 / ckh_scaled_mm_fp8 use at this shape to
- * split K (0: the shape does not split).  A small grid of 256 x 256 output tiles with long
+ * Bytes of device workspace ckh_scaled_mm_mxfp8 / ckh_scaled_mm_fp8 may use at this shape to
+ * split K (0: the shape does not split; a call that runs faster in one launch leaves the
+ * workspace untouched).  A small grid of 256 x 256 output tiles with long
  * K (e.g. M = 256, N = 13824, K = 5120) splits K over up to 256 workgroups, which write fp32
  * partial tiles to the workspace: grids of at most 64 tiles as 256 x 128 half tiles
  * (128 KB partials) from 32 stages of 64 along K, grids of 65-128 tiles as whole tiles
@@ -158,8 +159,8 @@ int64_t ckh_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K);
  * out [M,N] row-major of out_code (f32/f16/bf16).  K % 32 == 0.
  * workspace: NULL, or ckh_scaled_mm_workspace_bytes(M, N, K) bytes of device memory
  * (16-byte aligned) that the call may overwrite; with less than that the call does not
- * split K (same result within fp32 summation order, slower on small grids).  Calls running
- * at the same time need workspaces of their own.
+ * split K (same result within fp32 summation order, slower where it would have split).  Calls
+ * running at the same time need workspaces of their own.
  * No native counterpart in the reference (eager quantization.py:367-402 routes to
  * torch F.scaled_mm via scaled_mm_v2.py:27-53); replaces that call.
  */
@@ -214,8 +215,8 @@ int ckh_scaled_mm_nvfp4_scales(const void* a, const void* b, const void* sa, con
                                uintptr_t stream);
 
 /*
- * Bytes of device workspace ckh_scaled_mm_nvfp4 uses at this shape to split K (0: no
- * split): grids of at most 64 output tiles of 256 x 256 with K of at least 2048 (split as
+ * Bytes of device workspace ckh_scaled_mm_nvfp4 may use at this shape to split K (0: no
+ * split; as for ckh_scaled_mm_workspace_bytes): grids of at most 64 output tiles of 256 x 256 with K of at least 2048 (split as
  * 256 x 128 half tiles), and grids of 65-128 tiles with K of at least 4096 when three K
  * ranges or more fit.  No
  * counterpart in the reference (its launcher takes a cuBLASLt workspace of the caller's
