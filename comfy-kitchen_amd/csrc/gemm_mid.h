@@ -1,10 +1,12 @@
 // MXFP8 / per-tensor FP8 GEMM on small tiles, one workgroup per CU and one round, for a few
-// hundred activation rows: grids whose 256 x 256 tiles would leave CUs idle.
+// hundred activation rows (from 17 on in wide layers): grids whose 256 x 256 tiles would leave
+// CUs idle.
 //
-// What bounds it: a CU takes in about 57 GB/s of operand lines when they come from HBM and
-// about 90 GB/s from the L2 (a streaming kernel on 8 CUs measures the same, with loads to
-// registers or to LDS, at any number of loads in flight beyond 64 KB), whatever the other CUs
-// do.  A tile's time is therefore its (TM + TN) K operand bytes at that rate, about 0.5 us per
+// What bounds it: a CU takes in at most about 57 GB/s of operand lines when they come from HBM
+// (a streaming kernel on 8 CUs; 44-50 with 80 loading, 23-27 with all 256, where HBM itself is
+// the limit) and about 90 GB/s from the L2, with loads to registers or to LDS, at any number of
+// loads in flight beyond 64 KB.  Lines count, not bytes: with K not a multiple of 128 a row's
+// piece of a stage lies in two of them, and a stage takes up to 1.45 x as long.  A tile's time is therefore its (TM + TN) K operand bytes at that rate, about 0.5 us per
 // 128-byte stage of a 128 x 96 tile, and what helps is every CU busy with the smallest tile
 // that still fits the grid on the CUs at once; the matrix cores (0.2 us of those 0.5) and the
 // prefetch depth (3 to 6 stages measured equal) do not matter.  Measured against the
