@@ -92,6 +92,14 @@ __device__ __forceinline__ void wait_barrier() {
     __asm__ volatile("" ::: "memory");
 }
 
+// finish_tile's sums: K groups 0 and 1 end with them; the first column of a wave's part that
+// lane half h of group kg then holds (tiles i and quads q add 32 i + 8 q, and 4 columns follow).
+__host__ __device__ constexpr bool holds_sums(int kg) { return kg < 2; }
+template <int TN, int WN>
+__host__ __device__ constexpr int sum_column(int kg, int wn, int h) {
+    return wn * (TN / WN) + 16 * kg + 4 * h;
+}
+
 // The end of a tile, in LDS that no load writes any more (at least TM * TN * 2 KG bytes): the sums
 // of the KG K groups (of WM x WN waves, wave = WM WN kg + WM wn + wm) added, times alpha
 // (SCALE), plus the bias in lds_bias, rounded and stored.  acc: a wave's NT x MT MFMA tiles;
@@ -163,26 +171,30 @@ __device__ __forceinline__ void finish_tile(v16f (&acc)[NT][MT], uint8_t* lds, c
     if (kg == 0) recv(std::integral_constant<int, 0>{});
     else if (kg == 1) recv(std::integral_constant<int, 2>{});
 
-    const int ml = wm * (TM / WM) + r;                 // row of MFMA row tile 0
-    const int nl = wn * (TN / WN) + 16 * kg + 4 * h;   // column of MFMA column tile 0, quad 0
+    const int ml = wm * (TM / WM) + r;             // row of MFMA row tile 0
+    const int nl = sum_column<TN, WN>(kg, wn, h);  // column of MFMA column tile 0, quad 0
+    // (groups 2 and 3 hold no sums, and their nl would run past the TN columns of lds_bias)
+    const bool mine = holds_sums(kg);
+    if (mine) {
 #pragma unroll
-    for (int i = 0; i < NT; ++i)
+        for (int i = 0; i < NT; ++i)
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            float4 bv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (bias) bv = *reinterpret_cast<const float4*>(lds_bias + nl + 32 * i + 8 * q);
+            for (int q = 0; q < 2; ++q) {
+                float4 bv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (bias) bv = *reinterpret_cast<const float4*>(lds_bias + nl + 32 * i + 8 * q);
 #pragma unroll
-            for (int j = 0; j < MT; ++j) {
-                float4& o = v[i][j][q];
-                if constexpr (SCALE) o = make_float4(o.x * alpha, o.y * alpha, o.z * alpha, o.w * alpha);
-                if (bias) o = make_float4(o.x + bv.x, o.y + bv.y, o.z + bv.z, o.w + bv.w);
+                for (int j = 0; j < MT; ++j) {
+                    float4& o = v[i][j][q];
+                    if constexpr (SCALE) o = make_float4(o.x * alpha, o.y * alpha, o.z * alpha, o.w * alpha);
+                    if (bias) o = make_float4(o.x + bv.x, o.y + bv.y, o.z + bv.z, o.w + bv.w);
+                }
             }
-        }
+    }
     if constexpr (OUT == CKH_F32) {
 #pragma unroll
         for (int j = 0; j < MT; ++j) {
             const int m = m0 + ml + 32 * j;
-            if (m >= M || kg > 1) continue;
+            if (m >= M || !mine) continue;
 #pragma unroll
             for (int i = 0; i < NT; ++i)
 #pragma unroll
@@ -202,7 +214,7 @@ __device__ __forceinline__ void finish_tile(v16f (&acc)[NT][MT], uint8_t* lds, c
     } else {
         // 16-bit output: staged as TM rows in LDS, then whole rows, 16 bytes per lane
         wait_barrier<63>();  // the exchange area is read
-        if (kg < 2) {
+        if (mine) {
 #pragma unroll
             for (int j = 0; j < MT; ++j)
 #pragma unroll
