@@ -37,7 +37,9 @@ def direct(*tensors) -> bool:
     """Whether a `ck.*` call may go to the registry without the custom op around it: nothing
     looks at or transforms the op (compilation and tracing, dispatch and function modes, vmap
     and the other function transforms, forward-mode AD, the profiler), the first tensor is on
-    the GPU, and every tensor is a plain one that no gradient is asked of.  Anything else takes
+    the GPU, and every tensor is a plain one that no gradient is asked of and whose memory holds
+    its values (a lazily negated or conjugated view's does not, and a zero tensor has none: the
+    dispatcher makes them plain before the custom op's kernel sees them).  Anything else takes
     the custom op, which serves all of these.  The custom op's Python layers cost more than the
     call itself: on a 77 x 4096 tensor quantize_per_tensor_fp8 and dequantize_per_tensor_fp8
     took 20 us each from Python for 2.7 us on the GPU."""
@@ -53,6 +55,8 @@ def direct(*tensors) -> bool:
         if t is None:
             continue
         if type(t) is not _Tensor and type(t) is not _Parameter or grad and t.requires_grad:
+            return False
+        if t.is_neg() or t.is_conj() or t._is_zerotensor():
             return False
     return True
 

@@ -118,3 +118,25 @@ def test_direct_equals_custom_op(hip):
                                      torch.ones(1, device="cuda"))
     with pytest.raises(RuntimeError):
         y.float().sum().backward()
+
+
+@pytest.mark.gpu
+def test_lazy_views_take_the_custom_op(hip):
+    """A negated view's memory holds the values before the negation: as input, as scale (a complex
+    number's conjugated imaginary part is one) and as bias it gives what a plain copy gives."""
+    x = torch.randn(64, 128, device="cuda").bfloat16()
+    neg, z = torch._neg_view(x), torch.conj(torch.tensor([[1.5 - 0.25j]], device="cuda"))
+    scale = z.imag.reshape(1)
+    assert neg.is_neg() and scale.is_neg()
+    zeros = torch._efficientzerotensor((4, 128), dtype=torch.bfloat16, device="cuda")
+    assert not direct(neg) and not direct(x, scale) and not direct(zeros) and not direct(z)
+    for a, b in zip(ck.quantize_mxfp8(neg), ck.quantize_mxfp8(-x)):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    plain = torch.full((1,), 0.25, device="cuda")
+    assert torch.equal(plain, scale)
+    got, want = ck.quantize_per_tensor_fp8(x, scale), ck.quantize_per_tensor_fp8(x, plain)
+    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+    q, s = ck.quantize_mxfp8(x)
+    bias = torch.randn(64, device="cuda")
+    assert torch.equal(ck.scaled_mm_mxfp8(q, q, s, s, bias=torch._neg_view(bias)), ck.scaled_mm_mxfp8(q, q, s, s, bias=-bias))
+    assert ck.quantize_mxfp8(zeros)[0].float().abs().sum() == 0
