@@ -16,7 +16,7 @@ from .exceptions import (
     NoCapableBackendError,
 )
 from .float_utils import from_blocked, swap_nibbles, to_blocked
-from .ops import DTYPE_TO_CODE, _dispatch, direct
+from .ops import DTYPE_TO_CODE, _dispatch, direct, untouched
 from .registry import registry
 
 __version__ = "0.1.0"
@@ -58,7 +58,7 @@ def amax_scale(x: torch.Tensor, divisor: float) -> torch.Tensor:
     reduction, so dynamic quantization needs no host round trip.
     """
     divisor = float(divisor)
-    if direct(x):
+    if direct(x) and untouched("amax_scale"):
         return _dispatch("amax_scale", x=x, divisor=divisor)
     return torch.ops.comfy_kitchen.amax_scale(x, divisor)
 
@@ -67,7 +67,7 @@ def quantize_per_tensor_fp8(x: torch.Tensor, scale: torch.Tensor,
                             output_type: torch.dtype = torch.float8_e4m3fn) -> torch.Tensor:
     """FP8 quantize with one fp32 scale: fp8(clamp(x * (1/scale), +-max))."""
     code = DTYPE_TO_CODE[output_type]
-    if direct(x, scale):
+    if direct(x, scale) and untouched("quantize_fp8"):
         return _dispatch("quantize_per_tensor_fp8", x=x, scale=scale, output_type=output_type)
     return torch.ops.comfy_kitchen.quantize_fp8(x, scale, code)
 
@@ -81,7 +81,7 @@ def quantize_fp8_dynamic(x: torch.Tensor, divisor: float = 448.0,
     quantize (reference tensor/fp8.py:56-61) with the reduction fused into the quantize
     launch.  The results equal amax_scale followed by quantize_per_tensor_fp8 bit for bit."""
     divisor, code = float(divisor), DTYPE_TO_CODE[output_type]
-    if direct(x):
+    if direct(x) and untouched("quantize_fp8_dynamic"):
         return _dispatch("quantize_fp8_dynamic", x=x, divisor=divisor, output_type=output_type)
     return torch.ops.comfy_kitchen.quantize_fp8_dynamic(x, divisor, code)
 
@@ -90,7 +90,7 @@ def dequantize_per_tensor_fp8(x: torch.Tensor, scale: torch.Tensor,
                               output_type: torch.dtype = torch.bfloat16) -> torch.Tensor:
     """FP8 dequantize: x.to(output_type) * scale.to(output_type)."""
     code = DTYPE_TO_CODE[output_type]
-    if direct(x, scale):
+    if direct(x, scale) and untouched("dequantize_fp8"):
         return _dispatch("dequantize_per_tensor_fp8", x=x, scale=scale, output_type=output_type)
     return torch.ops.comfy_kitchen.dequantize_fp8(x, scale, code)
 
@@ -105,7 +105,8 @@ def stochastic_rounding_fp8(x: torch.Tensor, rng: torch.Tensor,
 def quantize_nvfp4(x: torch.Tensor, per_tensor_scale: torch.Tensor, epsilon: float = 0.0,
                    pad_16x: bool = False, hi_first: bool = True) -> tuple[torch.Tensor, torch.Tensor]:
     """NVFP4: packed E2M1 codes [M, K/2] uint8 and swizzled E4M3 block-16 scales."""
-    if type(epsilon) is float and type(pad_16x) is bool and type(hi_first) is bool and direct(x, per_tensor_scale):
+    if (type(epsilon) is float and type(pad_16x) is bool and type(hi_first) is bool
+            and direct(x, per_tensor_scale) and untouched("quantize_nvfp4")):
         return _dispatch("quantize_nvfp4", x=x, per_tensor_scale=per_tensor_scale, epsilon=epsilon,
                          pad_16x=pad_16x, hi_first=hi_first)
     return torch.ops.comfy_kitchen.quantize_nvfp4(x, per_tensor_scale, epsilon, pad_16x, hi_first)
@@ -121,7 +122,7 @@ def quantize_nvfp4_dynamic(x: torch.Tensor, divisor: float = 448.0 * 6.0, pad_16
     samples/nvfp4_linear.py:55-59) with the reduction fused into the quantize launch.
     The results equal amax_scale followed by quantize_nvfp4 bit for bit."""
     divisor = float(divisor)
-    if type(pad_16x) is bool and type(hi_first) is bool and direct(x):
+    if type(pad_16x) is bool and type(hi_first) is bool and direct(x) and untouched("quantize_nvfp4_dynamic"):
         return _dispatch("quantize_nvfp4_dynamic", x=x, divisor=divisor, pad_16x=pad_16x, hi_first=hi_first)
     return torch.ops.comfy_kitchen.quantize_nvfp4_dynamic(x, divisor, pad_16x, hi_first)
 
@@ -129,7 +130,7 @@ def quantize_nvfp4_dynamic(x: torch.Tensor, divisor: float = 448.0 * 6.0, pad_16
 def dequantize_nvfp4(qx: torch.Tensor, per_tensor_scale: torch.Tensor, block_scales: torch.Tensor,
                      output_type: torch.dtype = torch.bfloat16, hi_first: bool = True) -> torch.Tensor:
     code = DTYPE_TO_CODE[output_type]
-    if type(hi_first) is bool and direct(qx, per_tensor_scale, block_scales):
+    if type(hi_first) is bool and direct(qx, per_tensor_scale, block_scales) and untouched("dequantize_nvfp4"):
         return _dispatch("dequantize_nvfp4", qx=qx, per_tensor_scale=per_tensor_scale, block_scales=block_scales,
                          output_type=output_type, hi_first=hi_first)
     return torch.ops.comfy_kitchen.dequantize_nvfp4(qx, per_tensor_scale, block_scales, code, hi_first)
@@ -143,7 +144,8 @@ def scaled_mm_nvfp4(a: torch.Tensor, b: torch.Tensor, tensor_scale_a: torch.Tens
     """y = (a @ b.T) * (tensor_scale_a * tensor_scale_b) + bias on NVFP4 operands."""
     out_dtype = out_dtype if out_dtype is not None else torch.bfloat16
     code = DTYPE_TO_CODE[out_dtype]
-    if direct(a, b, tensor_scale_a, tensor_scale_b, block_scale_a, block_scale_b, bias, alpha):
+    if (direct(a, b, tensor_scale_a, tensor_scale_b, block_scale_a, block_scale_b, bias, alpha)
+            and untouched("scaled_mm_nvfp4")):
         return _dispatch("scaled_mm_nvfp4", a=a, b=b, tensor_scale_a=tensor_scale_a, tensor_scale_b=tensor_scale_b,
                          block_scale_a=block_scale_a, block_scale_b=block_scale_b, bias=bias, out_dtype=out_dtype,
                          alpha=alpha)
@@ -153,7 +155,7 @@ def scaled_mm_nvfp4(a: torch.Tensor, b: torch.Tensor, tensor_scale_a: torch.Tens
 
 def quantize_mxfp8(x: torch.Tensor, pad_32x: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
     """MXFP8: E4M3 codes [M, K] and swizzled E8M0 block-32 scales."""
-    if type(pad_32x) is bool and direct(x):
+    if type(pad_32x) is bool and direct(x) and untouched("quantize_mxfp8"):
         return _dispatch("quantize_mxfp8", x=x, pad_32x=pad_32x)
     return torch.ops.comfy_kitchen.quantize_mxfp8(x, pad_32x)
 
@@ -161,7 +163,7 @@ def quantize_mxfp8(x: torch.Tensor, pad_32x: bool = False) -> tuple[torch.Tensor
 def dequantize_mxfp8(qx: torch.Tensor, block_scales: torch.Tensor,
                      output_type: torch.dtype = torch.bfloat16) -> torch.Tensor:
     code = DTYPE_TO_CODE[output_type]
-    if direct(qx, block_scales):
+    if direct(qx, block_scales) and untouched("dequantize_mxfp8"):
         return _dispatch("dequantize_mxfp8", qx=qx, block_scales=block_scales, output_type=output_type)
     return torch.ops.comfy_kitchen.dequantize_mxfp8(qx, block_scales, code)
 
@@ -172,7 +174,7 @@ def scaled_mm_mxfp8(a: torch.Tensor, b: torch.Tensor, block_scale_a: torch.Tenso
     """y = a @ b.T + bias on MXFP8 operands (both K-major, E8M0 block-32 scales)."""
     out_dtype = out_dtype if out_dtype is not None else torch.bfloat16
     code = DTYPE_TO_CODE[out_dtype]
-    if direct(a, b, block_scale_a, block_scale_b, bias):
+    if direct(a, b, block_scale_a, block_scale_b, bias) and untouched("scaled_mm_mxfp8"):
         return _dispatch("scaled_mm_mxfp8", a=a, b=b, block_scale_a=block_scale_a, block_scale_b=block_scale_b,
                          bias=bias, out_dtype=out_dtype)
     return torch.ops.comfy_kitchen.scaled_mm_mxfp8(a, b, block_scale_a, block_scale_b, bias, code)
@@ -187,7 +189,7 @@ def scaled_mm_fp8(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor, scale
     """
     out_dtype = out_dtype if out_dtype is not None else torch.bfloat16
     code = DTYPE_TO_CODE[out_dtype]
-    if direct(a, b, scale_a, scale_b, bias):
+    if direct(a, b, scale_a, scale_b, bias) and untouched("scaled_mm_fp8"):
         return _dispatch("scaled_mm_fp8", a=a, b=b, scale_a=scale_a, scale_b=scale_b, bias=bias, out_dtype=out_dtype)
     return torch.ops.comfy_kitchen.scaled_mm_fp8(a, b, scale_a, scale_b, bias, code)
 
@@ -195,13 +197,13 @@ def scaled_mm_fp8(a: torch.Tensor, b: torch.Tensor, scale_a: torch.Tensor, scale
 def apply_rope(xq: torch.Tensor, xk: torch.Tensor,
                freqs_cis: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """Rotate query and key by the 2x2 matrices in freqs_cis [..., head_dim/2, 2, 2]."""
-    if direct(xq, xk, freqs_cis):
+    if direct(xq, xk, freqs_cis) and untouched("apply_rope"):
         return _dispatch("apply_rope", xq=xq, xk=xk, freqs_cis=freqs_cis)
     return torch.ops.comfy_kitchen.apply_rope(xq, xk, freqs_cis)
 
 
 def apply_rope1(x: torch.Tensor, freqs_cis: torch.Tensor) -> torch.Tensor:
-    if direct(x, freqs_cis):
+    if direct(x, freqs_cis) and untouched("apply_rope1"):
         return _dispatch("apply_rope1", x=x, freqs_cis=freqs_cis)
     return torch.ops.comfy_kitchen.apply_rope1(x, freqs_cis)
 

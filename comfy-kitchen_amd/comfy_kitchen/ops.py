@@ -31,6 +31,19 @@ def _dispatch(func_name: str, **kwargs):
 _Tensor, _Parameter = torch.Tensor, torch.nn.Parameter
 _is_compiling = torch.compiler.is_compiling
 _C = torch._C
+# Every key at which the dispatcher could find a kernel for plain GPU tensors ahead of, or in place
+# of, the custom op's own (which it holds under alias keys, so none of these is set by it)
+_KERNEL_KEYS = _C.DispatchKeySet(_C.DispatchKey.CUDA)
+for _key in ("AutocastCUDA", "AutogradCUDA", "ADInplaceOrView"):
+    _KERNEL_KEYS = _KERNEL_KEYS.add(getattr(_C.DispatchKey, _key))
+
+
+def untouched(op: str) -> bool:
+    """Whether no program has registered a kernel of its own (torch.library, an autocast rule,
+    the custom op's register_kernel) for GPU tensors on `comfy_kitchen::<op>`: one that has
+    expects `ck.*` calls to reach it.  (A kernel put in place of the op's default one under the
+    default's own alias key is not seen.)  About 0.7 us a call."""
+    return not _C._dispatch_has_kernel_for_any_dispatch_key("comfy_kitchen::" + op, _KERNEL_KEYS)
 
 
 def direct(*tensors) -> bool:

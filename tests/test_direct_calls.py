@@ -8,7 +8,7 @@ import torch
 import comfy_kitchen as ck
 import comfy_kitchen.backends.hip as hb
 from comfy_kitchen.constraints import FunctionConstraints, MinDims, ParamConstraint, validate_function_call
-from comfy_kitchen.ops import direct
+from comfy_kitchen.ops import direct, untouched
 from comfy_kitchen.registry import BackendRegistry
 
 ARCH = "gfx950:sramecc+:xnack-"
@@ -140,3 +140,38 @@ def test_lazy_views_take_the_custom_op(hip):
     bias = torch.randn(64, device="cuda")
     assert torch.equal(ck.scaled_mm_mxfp8(q, q, s, s, bias=torch._neg_view(bias)), ck.scaled_mm_mxfp8(q, q, s, s, bias=-bias))
     assert ck.quantize_mxfp8(zeros)[0].float().abs().sum() == 0
+
+
+OPS = ["amax_scale", "apply_rope", "apply_rope1", "dequantize_fp8", "dequantize_mxfp8", "dequantize_nvfp4",
+       "quantize_fp8", "quantize_fp8_dynamic", "quantize_mxfp8", "quantize_nvfp4", "quantize_nvfp4_dynamic",
+       "scaled_mm_fp8", "scaled_mm_mxfp8", "scaled_mm_nvfp4"]
+
+
+@pytest.mark.parametrize("op", OPS)
+def test_registered_kernels_are_seen(op):
+    """A kernel that a program puts on one of the ops, at any key a plain GPU tensor would meet,
+    ends the shortcut for that op, until the program takes it back."""
+    assert untouched(op)
+    for key in ("CUDA", "AutocastCUDA", "AutogradCUDA", "ADInplaceOrView"):
+        lib = torch.library.Library("comfy_kitchen", "IMPL")
+        lib.impl(op, lambda *args: None, key)
+        assert not untouched(op), key
+        lib._destroy()
+        assert untouched(op)
+
+
+@pytest.mark.gpu
+def test_registered_kernel_serves_the_call(hip):
+    x, scale = torch.randn(4, 32, device="cuda").bfloat16(), torch.ones(1, device="cuda")
+    marker = torch.zeros(4, 32, device="cuda")
+    lib = torch.library.Library("comfy_kitchen", "IMPL")
+    lib.impl("quantize_fp8", lambda x, scale, code: marker, "CUDA")
+    lib.impl("quantize_mxfp8", lambda x, pad: (marker, marker), "AutocastCUDA")
+    try:
+        assert torch.equal(ck.quantize_per_tensor_fp8(x, scale), marker)
+        assert ck.quantize_mxfp8(x)[0].dtype == torch.float8_e4m3fn  # no autocast here: the rule sleeps
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert ck.quantize_mxfp8(x)[0].dtype == torch.float32
+    finally:
+        lib._destroy()
+    assert ck.quantize_per_tensor_fp8(x, scale).dtype == torch.float8_e4m3fn
