@@ -104,8 +104,10 @@ def _call(name: str, *args) -> None:
         raise RuntimeError(f"{name}: {_lib.ckh_last_error().decode(errors='replace')}")
 
 
-_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-_current_device = getattr(torch._C, "_cuda_getDevice", None)
+# (the public forms where a torch lacks the bindings below them)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda device: torch.cuda.current_stream(device).cuda_stream)
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
 def _launch(name: str, t: torch.Tensor, *args) -> None:

@@ -29,13 +29,25 @@ def _dispatch(func_name: str, **kwargs):
 
 
 _Tensor, _Parameter = torch.Tensor, torch.nn.Parameter
-_is_compiling = torch.compiler.is_compiling
 _C = torch._C
-# Every key at which the dispatcher could find a kernel for plain GPU tensors ahead of, or in place
-# of, the custom op's own (which it holds under alias keys, so none of these is set by it)
-_KERNEL_KEYS = _C.DispatchKeySet(_C.DispatchKey.CUDA)
-for _key in ("AutocastCUDA", "AutogradCUDA", "ADInplaceOrView"):
-    _KERNEL_KEYS = _KERNEL_KEYS.add(getattr(_C.DispatchKey, _key))
+try:
+    _is_compiling = torch.compiler.is_compiling
+    _dispatch_modes, _function_modes = _C._len_torch_dispatch_stack, _C._len_torch_function_stack
+    _transforms, _tracing = _C._functorch.peek_interpreter_stack, _C._get_tracing_state
+    _profiling = _C._autograd._profiler_enabled
+    _is_zero = torch.Tensor._is_zerotensor
+    _forward_ad._current_level
+    _has_kernel = _C._dispatch_has_kernel_for_any_dispatch_key
+    # Every key at which the dispatcher could find a kernel for plain GPU tensors ahead of, or in
+    # place of, the custom op's own (which it holds under alias keys, so none of these is set by it)
+    _KERNEL_KEYS = _C.DispatchKeySet(_C.DispatchKey.CUDA)
+    for _key in ("AutocastCUDA", "AutogradCUDA", "ADInplaceOrView"):
+        _KERNEL_KEYS = _KERNEL_KEYS.add(getattr(_C.DispatchKey, _key))
+    _OBSERVABLE = True
+except (AttributeError, TypeError):
+    # A torch that lacks one of these (several are not public) gives no way to tell whether
+    # something looks at the op: every call takes the custom op then.
+    _OBSERVABLE = False
 
 
 def untouched(op: str) -> bool:
@@ -43,7 +55,7 @@ def untouched(op: str) -> bool:
     the custom op's register_kernel) for GPU tensors on `comfy_kitchen::<op>`: one that has
     expects `ck.*` calls to reach it.  (A kernel put in place of the op's default one under the
     default's own alias key is not seen.)  About 0.7 us a call."""
-    return not _C._dispatch_has_kernel_for_any_dispatch_key("comfy_kitchen::" + op, _KERNEL_KEYS)
+    return not _has_kernel("comfy_kitchen::" + op, _KERNEL_KEYS)
 
 
 def direct(*tensors) -> bool:
@@ -56,9 +68,8 @@ def direct(*tensors) -> bool:
     the custom op, which serves all of these.  The custom op's Python layers cost more than the
     call itself: on a 77 x 4096 tensor quantize_per_tensor_fp8 and dequantize_per_tensor_fp8
     took 20 us each from Python for 2.7 us on the GPU."""
-    if (_is_compiling() or _C._len_torch_dispatch_stack() or _C._len_torch_function_stack()
-            or _C._functorch.peek_interpreter_stack() is not None or _C._get_tracing_state() is not None
-            or _C._autograd._profiler_enabled() or _forward_ad._current_level >= 0):
+    if (not _OBSERVABLE or _is_compiling() or _dispatch_modes() or _function_modes() or _transforms() is not None
+            or _tracing() is not None or _profiling() or _forward_ad._current_level >= 0):
         return False
     first = tensors[0]
     if type(first) is not _Tensor and type(first) is not _Parameter or not first.is_cuda:
@@ -69,7 +80,7 @@ def direct(*tensors) -> bool:
             continue
         if type(t) is not _Tensor and type(t) is not _Parameter or grad and t.requires_grad:
             return False
-        if t.is_neg() or t.is_conj() or t._is_zerotensor():
+        if t.is_neg() or t.is_conj() or _is_zero(t):
             return False
     return True
 

@@ -1,6 +1,9 @@
 """Calls that skip the custom op: the registry's shortcut accepts exactly what the general
 validation accepts, and `direct` stands aside for everything that looks at or transforms an op."""
 import itertools
+import subprocess
+import sys
+from pathlib import Path
 
 import pytest
 import torch
@@ -11,6 +14,7 @@ from comfy_kitchen.constraints import FunctionConstraints, MinDims, ParamConstra
 from comfy_kitchen.ops import direct, untouched
 from comfy_kitchen.registry import BackendRegistry
 
+PACKAGE = Path(__file__).resolve().parent.parent / "comfy-kitchen_amd"
 ARCH = "gfx950:sramecc+:xnack-"
 TABLE = hb._build_constraints()
 DTYPES = [torch.float32, torch.bfloat16, torch.float16, torch.uint8, torch.int32, torch.float8_e4m3fn,
@@ -175,3 +179,41 @@ def test_registered_kernel_serves_the_call(hip):
     finally:
         lib._destroy()
     assert ck.quantize_per_tensor_fp8(x, scale).dtype == torch.float8_e4m3fn
+
+
+@pytest.mark.parametrize("holder,name", [("torch._C._functorch", "peek_interpreter_stack"),
+                                         ("torch._C._autograd", "_profiler_enabled"),
+                                         ("torch._C", "_get_tracing_state"),
+                                         ("torch._C", "_dispatch_has_kernel_for_any_dispatch_key"),
+                                         ("torch.autograd.forward_ad", "_current_level")])
+def test_torch_without_a_probe_takes_the_custom_op(holder, name):
+    """Where torch lacks one of the names the shortcut asks, the package imports and every call
+    takes the custom op (here: reaches the registry, which has no backend for a CPU tensor)."""
+    code = f"""
+import sys
+sys.path.insert(0, {str(PACKAGE)!r})
+import torch, torch.autograd.forward_ad
+del {holder}.{name}
+import comfy_kitchen as ck
+from comfy_kitchen.ops import direct
+x = torch.zeros(4, 32)
+assert not direct(x)
+try:
+    ck.quantize_mxfp8(x)
+except ck.NoCapableBackendError:
+    print("ok")
+"""
+    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert run.stdout.strip() == "ok", run.stderr
+
+
+@pytest.mark.gpu
+def test_no_probes_same_results(hip, monkeypatch):
+    import comfy_kitchen.ops as ops
+
+    x = torch.randn(16, 64, device="cuda").bfloat16()
+    want = ck.quantize_mxfp8(x)
+    monkeypatch.setattr(ops, "_OBSERVABLE", False)
+    assert not direct(x)
+    got = ck.quantize_mxfp8(x)
+    assert all(torch.equal(a.view(torch.uint8), b.view(torch.uint8)) for a, b in zip(got, want))
