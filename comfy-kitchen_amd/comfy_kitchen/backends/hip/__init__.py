@@ -89,7 +89,10 @@ def load_library(path: Path | str | None = None) -> ctypes.CDLL:
         raise OSError(f"{p} not found: build it with `python comfy-kitchen_amd/build.py`")
     lib = ctypes.CDLL(str(p))
     for name, (res, args) in SIGNATURES.items():
-        fn = getattr(lib, name)
+        try:
+            fn = getattr(lib, name)
+        except AttributeError:  # an older build: entry points were added without a new ABI version
+            raise OSError(f"{p}: no entry point {name}: rebuild it with `python comfy-kitchen_amd/build.py`") from None
         fn.restype, fn.argtypes = res, args
     if lib.ckh_abi_version() != ABI_VERSION:
         raise OSError(f"{p}: ABI version {lib.ckh_abi_version()} != expected {ABI_VERSION}")

@@ -2,7 +2,10 @@
 rejects bad arguments with an error code and message -- all without a GPU (argument
 validation happens before any HIP call)."""
 import ctypes
+import os
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import pytest
@@ -89,3 +92,19 @@ def test_quantize_nvfp4_dynamic_rejects_bad_arguments(lib):
     assert b"empty tensor" in lib.ckh_last_error()
     assert f(p, 2688.0, p, p, p, 16, 40, 16, 40, 0.0, 2, 1, p, 0) == 1
     assert b"multiple of 16" in lib.ckh_last_error()
+
+
+def test_library_of_an_older_build_is_reported(tmp_path):
+    """A library of this ABI version that lacks an entry point is an OSError naming it, and the
+    package imports with the backend marked unavailable for that reason."""
+    src, old = tmp_path / "old.c", tmp_path / "libckh.so"
+    names = [n for n in hb.SIGNATURES if n not in ("ckh_abi_version", "ckh_quantize_fp8_dynamic")]
+    src.write_text(f"int ckh_abi_version(void) {{ return {hb.ABI_VERSION}; }}\n"
+                   + "".join(f"int {n}(void) {{ return 0; }}\n" for n in names))
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(old), str(src)], check=True)
+    with pytest.raises(OSError, match="ckh_quantize_fp8_dynamic"):
+        hb.load_library(old)
+    code = "import comfy_kitchen as ck; print(ck.list_backends()['hip']['unavailable_reason'])"
+    env = dict(os.environ, CKH_LIBRARY=str(old), PYTHONPATH=str(HEADER.parent.parent / "comfy-kitchen_amd"))
+    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120, env=env)
+    assert "ckh_quantize_fp8_dynamic" in run.stdout, run.stderr
