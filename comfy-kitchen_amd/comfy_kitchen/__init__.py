@@ -16,7 +16,7 @@ from .exceptions import (
     NoCapableBackendError,
 )
 from .float_utils import from_blocked, swap_nibbles, to_blocked
-from .ops import DTYPE_TO_CODE, _dispatch, direct, untouched
+from .ops import DTYPE_TO_CODE, _dispatch, _quantize_fp8_dynamic, direct, untouched
 from .registry import registry
 
 __version__ = "0.1.0"
@@ -82,7 +82,7 @@ def quantize_fp8_dynamic(x: torch.Tensor, divisor: float = 448.0,
     launch.  The results equal amax_scale followed by quantize_per_tensor_fp8 bit for bit."""
     divisor, code = float(divisor), DTYPE_TO_CODE[output_type]
     if direct(x) and untouched("quantize_fp8_dynamic"):
-        return _dispatch("quantize_fp8_dynamic", x=x, divisor=divisor, output_type=output_type)
+        return _quantize_fp8_dynamic(x, divisor, output_type)
     return torch.ops.comfy_kitchen.quantize_fp8_dynamic(x, divisor, code)
 
 

@@ -108,10 +108,18 @@ def _(x, scale, output_dtype_code):
     return torch.empty_like(x, dtype=DTYPE_CODE_TO_DTYPE[output_dtype_code])
 
 
+def _quantize_fp8_dynamic(x: torch.Tensor, divisor: float, output_type: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
+    """The fused call where one backend serves it and the quantizer; else the two calls it stands
+    for, each from the backend that the program has chosen for it."""
+    if registry.serves_both("quantize_per_tensor_fp8", "quantize_fp8_dynamic", {"x": x, "output_type": output_type}):
+        return _dispatch("quantize_fp8_dynamic", x=x, divisor=divisor, output_type=output_type)
+    scale = _dispatch("amax_scale", x=x, divisor=divisor)
+    return _dispatch("quantize_per_tensor_fp8", x=x, scale=scale, output_type=output_type), scale
+
+
 @torch.library.custom_op("comfy_kitchen::quantize_fp8_dynamic", mutates_args=())
 def quantize_fp8_dynamic(x: torch.Tensor, divisor: float, output_dtype_code: int) -> tuple[torch.Tensor, torch.Tensor]:
-    return _dispatch("quantize_fp8_dynamic", x=x, divisor=divisor,
-                     output_type=DTYPE_CODE_TO_DTYPE[output_dtype_code])
+    return _quantize_fp8_dynamic(x, divisor, DTYPE_CODE_TO_DTYPE[output_dtype_code])
 
 
 @quantize_fp8_dynamic.register_fake

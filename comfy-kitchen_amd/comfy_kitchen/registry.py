@@ -223,15 +223,24 @@ class BackendRegistry:
                     return False
         return True
 
-    def _first_choice(self, func_name: str, kwargs: Mapping[str, Any] | None) -> Callable | None:
-        """The implementation get_capable_backend would choose when the first backend in the
-        priority order takes the call and nothing else has a say; None: ask the general path."""
+    def _first_choice(self, func_name: str, kwargs: Mapping[str, Any] | None) -> str | None:
+        """The backend get_capable_backend would choose when the first one in the priority
+        order takes the call and nothing else has a say; None: ask the general path."""
         if self._forced() or not self._order or not kwargs or logger.isEnabledFor(logging.DEBUG):
             return None
-        slot = self._slots.get(self._order[0])
+        name = self._order[0]
+        slot = self._slots.get(name)
         if slot is None or not slot.usable or func_name not in slot.table:
             return None
-        return getattr(slot.module, func_name) if self._accepts(slot.table[func_name], kwargs) else None
+        return name if self._accepts(slot.table[func_name], kwargs) else None
+
+    def serves_both(self, func_name: str, other: str, kwargs: Mapping[str, Any]) -> bool:
+        """Whether one backend would be chosen for both functions with these arguments."""
+        try:
+            return ((self._first_choice(func_name, kwargs) or self.get_capable_backend(func_name, kwargs))
+                    == (self._first_choice(other, kwargs) or self.get_capable_backend(other, kwargs)))
+        except NoCapableBackendError:
+            return False
 
     def _candidates(self) -> Iterator[tuple[str, bool]]:
         forced = self._forced()
@@ -256,10 +265,7 @@ class BackendRegistry:
                            kwargs: Mapping[str, Any] | None = None) -> Callable:
         """The callable serving `func_name`: from `backend` if named, else the selected one."""
         if not backend:
-            chosen = self._first_choice(func_name, kwargs)
-            if chosen is not None:
-                return chosen
-            backend = self.get_capable_backend(func_name, kwargs)
+            backend = self._first_choice(func_name, kwargs) or self.get_capable_backend(func_name, kwargs)
             return getattr(self._slots[backend].module, func_name)
         slot = self._slots.get(backend, _Slot())
         if not slot.usable:

@@ -121,3 +121,55 @@ def test_fake_shapes_under_meta():
                                                     torch.empty(128, 4, dtype=torch.float8_e8m0fnu),
                                                     torch.empty(128, 4, dtype=torch.float8_e8m0fnu), None, 2)
         assert y.shape == (8, 16) and y.dtype == torch.bfloat16
+
+
+class _OwnFp8:
+    """A program's backend: the reference's quantizer and this registry's amax_scale, no fused form."""
+
+    def __init__(self, fused=False):
+        self.calls = []
+        if fused:
+            self.quantize_fp8_dynamic = self._fused
+
+    def amax_scale(self, x, divisor):
+        self.calls.append("amax_scale")
+        return (x.abs().amax() / divisor).float()
+
+    def quantize_per_tensor_fp8(self, x, scale, output_type):
+        self.calls.append("quantize_per_tensor_fp8")
+        return (x / scale).to(output_type)
+
+    def _fused(self, x, divisor, output_type):
+        self.calls.append("quantize_fp8_dynamic")
+        scale = (x.abs().amax() / divisor).float()
+        return (x / scale).to(output_type), scale
+
+
+@pytest.mark.parametrize("fused", [False, True])
+def test_fp8_layout_uses_the_chosen_quantizer(fused):
+    """The FP8 layout's default scale: a backend that serves the quantizer is the one that
+    quantizes, whether or not it has the fused form; a backend that has only the fused form
+    further down the order does not take the call away from it."""
+    from comfy_kitchen.tensor import QuantizedTensor
+
+    own, other = _OwnFp8(fused), _OwnFp8(fused=True)
+    cpu = FunctionConstraints(default_devices=frozenset({"cpu"}))
+    order = ck.registry._order
+    names = ["amax_scale", "quantize_per_tensor_fp8"] + (["quantize_fp8_dynamic"] if fused else [])
+    ck.registry.register("own", own, {n: cpu for n in names})
+    ck.registry.register("other", other, {"quantize_fp8_dynamic": cpu})
+    try:
+        ck.registry.set_priority(["own", "other", *order])
+        x = torch.linspace(-3, 5, 64).reshape(4, 16)
+        q = QuantizedTensor.from_float(x, "TensorCoreFP8Layout")
+        assert own.calls == (["quantize_fp8_dynamic"] if fused else ["amax_scale", "quantize_per_tensor_fp8"])
+        assert other.calls == [] and float(q.params.scale) == pytest.approx(5 / 448)
+        ck.registry.set_priority(["other", *order])
+        with ck.registry.use_backend("own"):
+            own.calls.clear()
+            QuantizedTensor.from_float(x, "TensorCoreFP8Layout")
+        assert own.calls and other.calls == []
+    finally:
+        ck.registry.set_priority(list(order))
+        ck.registry._slots.pop("own")
+        ck.registry._slots.pop("other")
