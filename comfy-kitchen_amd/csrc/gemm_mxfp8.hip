@@ -52,6 +52,7 @@
 #include <utility>
 
 #include "ckh_common.h"
+#include "dispatch.h"
 #include "gemm_mid.h"
 #include "skinny.h"
 
@@ -130,9 +131,6 @@ struct Args {
     float* part;
     int bias_code;  // dtype code of bias
 };
-
-// fp32 values of one partial tile in the workspace (256 x 256)
-constexpr int kPartTile = BM * BN;
 
 // Register-staged loads of one operand for a pair of stages (s, s + 1), i.e. K bytes
 // [k0, k0 + 128) of the tile's 256 (or 128) rows.  Wave w, load j (0..7, or 0..3)
@@ -980,9 +978,6 @@ using namespace ckh;
 
 namespace {
 
-// Workgroups that can hold a 256 x 256 tile at once: one per CU.
-constexpr int kGemmSlots = 256;
-
 template <bool UNIT>
 void launch_grid(const mx::Args& p, unsigned wgs, int out_code, bool has_bias, hipStream_t st) {
 #define LAUNCH(O)                                                                                          \
@@ -996,123 +991,49 @@ void launch_grid(const mx::Args& p, unsigned wgs, int out_code, bool has_bias, h
 #undef LAUNCH
 }
 
-// Activations of at most kSkinnyMaxM rows take the skinny kernel (mxsk::gemm_skinny_kernel).
-constexpr int kSkinnyMaxM = 64;
-// From 17 rows and this N on, small tiles serve them instead (skinny_tile).
-constexpr int kSkinnySmallN = 8192;
-
 template <bool UNIT>
-int launch_skinny(const mx::Args& q, int out_code, int bias_code, bool has_bias, hipStream_t st) {
+int launch_skinny(const mx::Args& q, int form, int out_code, int bias_code, bool has_bias, hipStream_t st) {
     mxsk::Args p{};
     p.a = q.a; p.b = q.b; p.sa = q.sa; p.sb = q.sb; p.bias = q.bias; p.out = q.out;
     p.M = q.M; p.N = q.N; p.K = q.K; p.ncb = q.ncb; p.sa_rows = q.sa_rows; p.sb_rows = q.sb_rows;
     p.tsa = q.tsa; p.tsb = q.tsb;
-    // per activation size: waves per workgroup, weight tiles per workgroup, activation tiles,
-    // staged activation rows (measured on N = 18432, K = 3072: M = 1 12.7 us, M = 16 15.4 us).
-    // With 16 activation rows the waves per workgroup follow N: 2 waves when there are at least
-    // 256 workgroups (M = 16, N = 18432: 14.6 against 15.4 us with 4), 8 when there are fewer than
-    // 128 (N = 3072, K = 12288: 16.6 against 17.2 us; with 2 waves 25.9 us).  With 4-8 rows and N
-    // above 16384, 2 waves rather than 8 (M = 8, N = 18432, K = 3072 13.4 against 14.5 us; N =
-    // 24576 14.9 against 15.8; M = 4 13.1 against 13.6; M = 1 and 2 and N = 16384 equal).  From 17
-    // rows on this kernel serves what skinny_tile leaves: N below 8192, where its waves' split of K
-    // keeps more of the chip busy than small tiles would (32 x 5120 x 5120 11.6 against 16.1 us,
-    // 64 x 5120 x 12288 27.7 against 37.0); 17-32 rows with a short K (2 waves and one tile up to N
-    // = 24576: 20 x 18432 x 3072 16.4 against 17.3 with 4 waves; 2 waves and two tiles beyond: 20 x
-    // 32768 x 3072 20.2 against 22.0); and N beyond one round of 64 x 128 tiles.  There the
-    // activation is staged through LDS too, 32 or 64 rows (N = 5120, K = 5120, M = 32 10.8
-    // against 16.5 with the fragments loaded into registers; M = 64, K = 13824 29.3 against 47.4).
-    // The NVFP4 skinny kernel's form (128-byte chunks, two in flight per wave) measured slower
-    // here, where a chunk costs only a few MFMAs: M = 1 14.5 against 12.9 us, M = 16 15.9 against
-    // 15.5, M = 64 29.6 against 26.5 (same process).
-#define LAUNCH(O, B, WV, NT, MT, AR)                                                              \
-    hipLaunchKernelGGL((mxsk::gemm_skinny_kernel<O, B, UNIT, WV, NT, MT, AR>),                    \
-                       dim3(static_cast<unsigned>(cdiv(q.N, 32 * NT))), dim3(64 * WV), 0, st, p)
-#define BY_MT(O, B)                                    \
-    do {                                               \
-        if (p.M <= 8 && p.M >= 4 && p.N > 16384) LAUNCH(O, B, 2, 1, 1, 8); \
-        else if (p.M <= 8) LAUNCH(O, B, 8, 1, 1, 8);                   \
-        else if (p.M <= 16 && p.N >= 8192) LAUNCH(O, B, 2, 1, 1, 16);  \
-        else if (p.M <= 16 && p.N >= 4096) LAUNCH(O, B, 4, 1, 1, 16);  \
-        else if (p.M <= 16) LAUNCH(O, B, 8, 1, 1, 16);                 \
-        else if (p.M <= 32 && p.N > 24576) LAUNCH(O, B, 2, 2, 1, 32);  \
-        else if (p.M <= 32 && p.N > 16384) LAUNCH(O, B, 2, 1, 1, 32);  \
-        else if (p.M <= 32 && p.N >= kSkinnySmallN) LAUNCH(O, B, 4, 2, 1, 32); \
-        else if (p.M <= 32) LAUNCH(O, B, 8, 1, 1, 32);                 \
-        else if (p.N >= kSkinnySmallN) LAUNCH(O, B, 2, 2, 2, 64);      \
-        else LAUNCH(O, B, 4, 1, 2, 64);                                \
+#define LAUNCH(O, B, I)                                                                           \
+    case I:                                                                                       \
+        hipLaunchKernelGGL((mxsk::gemm_skinny_kernel<O, B, UNIT, kMxSkinny[I].waves, kMxSkinny[I].weight_tiles, \
+                                                     kMxSkinny[I].act_tiles, kMxSkinny[I].act_rows>), \
+                           dim3(static_cast<unsigned>(cdiv(q.N, 32 * kMxSkinny[I].weight_tiles))), \
+                           dim3(64 * kMxSkinny[I].waves), 0, st, p);                              \
+        break
+#define BY_FORM(O, B)        \
+    do {                     \
+        switch (form) {      \
+            LAUNCH(O, B, 0); \
+            LAUNCH(O, B, 1); \
+            LAUNCH(O, B, 2); \
+            LAUNCH(O, B, 3); \
+            LAUNCH(O, B, 4); \
+            LAUNCH(O, B, 5); \
+            LAUNCH(O, B, 6); \
+            LAUNCH(O, B, 7); \
+            LAUNCH(O, B, 8); \
+            LAUNCH(O, B, 9); \
+            LAUNCH(O, B, 10); \
+        }                    \
     } while (0)
 #define BY_BIAS(O)                                          \
     do {                                                    \
-        if (!has_bias) BY_MT(O, -1);                        \
-        else if (bias_code == CKH_F32) BY_MT(O, CKH_F32);   \
-        else if (bias_code == CKH_F16) BY_MT(O, CKH_F16);   \
-        else BY_MT(O, CKH_BF16);                            \
+        if (!has_bias) BY_FORM(O, -1);                        \
+        else if (bias_code == CKH_F32) BY_FORM(O, CKH_F32);   \
+        else if (bias_code == CKH_F16) BY_FORM(O, CKH_F16);   \
+        else BY_FORM(O, CKH_BF16);                            \
     } while (0)
     if (out_code == CKH_BF16) BY_BIAS(CKH_BF16);
     else if (out_code == CKH_F16) BY_BIAS(CKH_F16);
     else BY_BIAS(CKH_F32);
 #undef BY_BIAS
-#undef BY_MT
+#undef BY_FORM
 #undef LAUNCH
     return check_launch(UNIT ? "scaled_mm_fp8" : "scaled_mm_mxfp8");
-}
-
-// Split-K: a grid of at most half as many 256 x 256 tiles as CUs leaves most CUs idle
-// while each tile walks all of K.  Such a grid with long K instead runs S K ranges of every
-// tile (each of ks stages, a multiple of 4, at least kMinSplitStages) as S times as many
-// workgroups, at most one per CU, which write fp32 partial tiles to the caller's workspace;
-// a second launch adds them.  A partial tile (256 KB) costs about as much memory traffic
-// to write and again to read back as 8 stages of operand loads, so short K (fewer than
-// kMinSplitK stages) keeps whole-K half tiles instead.  With at most a quarter as many
-// tiles as CUs the split runs 256 x 128 half tiles, at least two K ranges each: a half
-// tile's stage costs ~53% of a full tile's (C4's last round) and its partial (128 KB) half
-// as much traffic, so for the same workgroups the partials move half the bytes.  Half
-// tiles split from kMinSplitKHalf stages on, and below kMinSplitK stages on at most
-// kShortSplitSlots workgroups (same process, against whole-K half tiles: 512 x 4096 x 3072
-// 23.0 against 28.5 us, 22.6 with 256 workgroups; 256 x 9216 x 3072 24.8 against 29.3;
-// 256 x 3072 x 3072 17.9 against 21.2; with that cap on long K too, 256 x 5120 x 13824
-// took 38.3 against 36.0 us).  Full tiles split only into three ranges or more: two
-// ranges give as many workgroups as whole-K half tiles, which need no partials (same
-// process: 256 x 32768 x 5120 57.6 against 66.6 us split, 384 x 12288 x 6144 54.0 against
-// 56.2; with three, 256 x 18432 x 8192 60.7 split against 71.2).
-// Measured, graph-timed: M = 256, N = 5120, K = 13824 40.5 us split in full tiles against
-// 110.8 us whole-K half tiles; N = 13824, K = 5120 40.1 against 46.9 us; N = 18432,
-// K = 3072 38.3 against 32.1 us (not split).  Half tiles against full tiles in the split
-// (same process): 256 x 4096 x 4096 20.9 against 27.1 us, 256 x 5120 x 13824 36.3 against
-// 40.4, 512 x 3072 x 13824 38.6 against 42.5, 256 x 13824 x 5120 38.7 against 40.6.
-constexpr int kMinSplitStages = 12;
-constexpr int kMinSplitK = 64;      // stages
-constexpr int kMinSplitKHalf = 32;  // stages, half tiles
-constexpr int kShortSplitSlots = 224;
-
-struct SplitPlan {
-    int S = 1;   // K ranges (1: no split)
-    int ks = 0;  // stages per range
-    int nw = 4;  // 4: full tiles, 2: half tiles
-};
-
-SplitPlan split_plan(int M, int N, int K) {
-    SplitPlan sp;
-    if (M <= kSkinnyMaxM) return sp;
-    const int tiles = static_cast<int>(cdiv(M, mx::BM) * cdiv(N, mx::BN));
-    const int KT = static_cast<int>(cdiv(K, mx::BK));
-    const bool half = tiles <= kGemmSlots / 4;
-    if (tiles > kGemmSlots / 2 || KT < (half ? kMinSplitKHalf : kMinSplitK)) return sp;
-    const int units = half ? 2 * tiles : tiles;
-    const int slots = half && KT < kMinSplitK ? kShortSplitSlots : kGemmSlots;
-    const int S = min(slots / units, KT / kMinSplitStages);
-    if (S < (half ? 2 : 3)) return sp;
-    sp.ks = static_cast<int>(rup(cdiv(KT, S), 4));
-    sp.S = static_cast<int>(cdiv(KT, sp.ks));
-    sp.nw = half ? 2 : 4;
-    return sp;
-}
-
-// one partial tile (or two partial half tiles) per tile and K range
-int64_t split_workspace_bytes(int M, int N, int K) {
-    const SplitPlan sp = split_plan(M, N, K);
-    if (sp.S < 2) return 0;
-    return cdiv(M, mx::BM) * cdiv(N, mx::BN) * sp.S * static_cast<int64_t>(mx::kPartTile) * 4;
 }
 
 template <bool UNIT, int NW>
@@ -1136,56 +1057,9 @@ void launch_split(mx::Args p, int out_code, int bias_code, bool has_bias, hipStr
 #undef LAUNCH
 }
 
-// Small tiles (gemm_mid.h): the first of these whose grid fits the CUs in one round.  The
-// order is by operand rows, i.e. by time: over 200 measured shapes the first that fits was
-// within 3% of the fastest that fits.  Larger tiles than these (or a second round) were slower
-// than the 256 x 256 kernel's half tiles.
-struct MidTile {
-    int tm, tn;
-};
-constexpr MidTile kMidTiles[] = {{64, 64}, {128, 64}, {128, 96}, {128, 128}, {128, 160}, {128, 192}, {64, 128}};
-constexpr int kMidWide = 6;  // 64 x 128, for at most 64 rows only (mid_tile looks at those before it)
-
-// Index of the small tile to use, or -1: the estimated time (us) of the first that fits against
-// that of the 256 x 256 kernel.  Fitted to the same shapes:
-//   small tiles  2.0 + 0.0165 rows + 0.00228 rows per 128-byte stage (rows = TM + TN);
-//   split-K      14.7 + 0.575 per stage of a K range in half tiles, 1.09 in full tiles (two
-//                launches; 200 x 5120 x 13824, six ranges of 36: 35.4 measured, small tiles 50);
-//   half tiles   6.2 + 0.4 per stage of K (200 x 21504 x 512: 9.5 measured, small tiles 12.1).
-// With K not a multiple of 128 a stage's piece of a row lies in two cache lines, and lines are
-// what a CU's intake is counted in: the terms per stage of the one-launch forms take 1.45 x (84 x
-// 12624 x 9824 53.1 against 38.9, 360 x 9584 x 2400 23.6 against 17.3), 1.1 x where more than 6
-// tiles share a weight row, which then comes from L2 (691 x 1312 x 5824 16.2 against 17.5).  118 x
-// 2448 x 6304: small tiles 25.0, split-K 21.0; 460 x 3112 x 9312 43.5 and 37.5.
-int mid_tile(int M, int N, int K, const SplitPlan& sp, int cus) {
-    for (int i = 0; i < kMidWide; ++i) {
-        const MidTile t = kMidTiles[i];
-        if (cdiv(M, t.tm) * cdiv(N, t.tn) > cus) continue;
-        const double rows = t.tm + t.tn;
-        const double lines = K % 128 == 0 ? 1.0 : cdiv(M, t.tm) <= 6 ? 1.45 : 1.1;
-        const double mid = 2.0 + 0.0165 * rows + 0.00228 * rows * lines * static_cast<double>(cdiv(K, 128));
-        const double big = sp.S > 1 ? 14.7 + (sp.nw == 2 ? 0.575 : 1.09) * sp.ks
-                                    : 6.2 + 0.4 * lines * static_cast<double>(cdiv(K, mx::BK));
-        return mid < big ? i : -1;
-    }
-    return -1;
-}
-
-// The small tile for at most 64 rows, or -1 for the skinny kernel: from 17 rows and N = 8192 on,
-// 64 x 64 or 64 x 128, whichever fits in one round (graph-timed, against the skinny kernel: 24 x
-// 8192 x 5120 16.3 / 17.5 us, 48 x 12288 x 3072 13.0 / 17.1, 64 x 8192 x 12288 37.7 / 46.0, 33 x
-// 18432 x 3072 18.0 / 21.0, 64 x 24576 x 5120 33.6 / 40.3; with 16 rows level).  With 17-32 rows
-// a short K leaves the ring's fill and the one workgroup per CU in view: 32 x 9000 x 512 5.5 / 5.3,
-// 17 x 21504 x 3072 18.7 / 16.5, but 32 x 16384 x 3072 12.8 / 14.3, 17 x 21504 x 5120 26.3 / 30.3.
-int skinny_tile(int M, int N, int K, int cus) {
-    if (M <= 16 || N < kSkinnySmallN) return -1;
-    if (cdiv(N, 64) <= cus) return M <= 32 && K < 1024 ? -1 : 0;
-    if (cdiv(N, 128) <= cus) return M <= 32 && K <= 4096 ? -1 : kMidWide;
-    return -1;
-}
-
-template <bool UNIT, int TM, int TN, int NST>
+template <bool UNIT, int TILE, int NST>
 void launch_mid_tile(const mid::Args& p, int out_code, hipStream_t st) {
+    constexpr int TM = kMxSmall[TILE].tm, TN = kMxSmall[TILE].tn;
     const dim3 grid(static_cast<unsigned>(p.tiles_m * cdiv(p.N, TN)));
 #define LAUNCH(O) hipLaunchKernelGGL((mid::gemm_mid_kernel<O, UNIT, TM, TN, NST>), grid, dim3(mid::kThreads), 0, st, p)
     if (out_code == CKH_BF16) LAUNCH(CKH_BF16);
@@ -1202,58 +1076,43 @@ void launch_mid(const mx::Args& q, int tile, int out_code, int bias_code, bool h
     p.bias_code = bias_code;
     p.M = q.M; p.N = q.N; p.K = q.K; p.ncb = q.ncb; p.sa_rows = q.sa_rows; p.sb_rows = q.sb_rows;
     p.tsa = q.tsa; p.tsb = q.tsb;
-    p.tiles_m = static_cast<int>(cdiv(p.M, kMidTiles[tile].tm));
+    p.tiles_m = static_cast<int>(cdiv(p.M, kMxSmall[tile].tm));
     switch (tile) {  // ring depth: what fits in LDS beside the staged output
-        case 0: launch_mid_tile<UNIT, 64, 64, 6>(p, out_code, st); break;
-        case 1: launch_mid_tile<UNIT, 128, 64, 5>(p, out_code, st); break;
-        case 2: launch_mid_tile<UNIT, 128, 96, 4>(p, out_code, st); break;
-        case 3: launch_mid_tile<UNIT, 128, 128, 4>(p, out_code, st); break;
-        case 4: launch_mid_tile<UNIT, 128, 160, 3>(p, out_code, st); break;
-        case 5: launch_mid_tile<UNIT, 128, 192, 3>(p, out_code, st); break;
-        default: launch_mid_tile<UNIT, 64, 128, 5>(p, out_code, st); break;
+        case 0: launch_mid_tile<UNIT, 0, 6>(p, out_code, st); break;
+        case 1: launch_mid_tile<UNIT, 1, 5>(p, out_code, st); break;
+        case 2: launch_mid_tile<UNIT, 2, 4>(p, out_code, st); break;
+        case 3: launch_mid_tile<UNIT, 3, 4>(p, out_code, st); break;
+        case 4: launch_mid_tile<UNIT, 4, 3>(p, out_code, st); break;
+        case 5: launch_mid_tile<UNIT, 5, 3>(p, out_code, st); break;
+        default: launch_mid_tile<UNIT, kMxSmallWide, 5>(p, out_code, st); break;
     }
 }
 
-// The 256 x 256 tiles run one per CU in rounds.  When the last round would be at most
-// half full (e.g. 864 tiles = 3 rounds + 96), its tiles run as twice as many 256 x 128
-// half tiles (about 55% of a full tile's time each), in the same grid.  A grid of one
-// round fills the remaining CUs with weight-prefetch workgroups (prefetch_weight).
-// Activations of at most kSkinnyMaxM rows take the skinny kernel, a few hundred rows the small
-// tiles, and small grids with long K split K when the caller gives a workspace.
+// The kernel that mx_route names.
 template <bool UNIT>
 int launch_gemm(mx::Args p, int out_code, int bias_code, bool has_bias, void* workspace, int64_t workspace_bytes,
                 hipStream_t st) {
-    const int cus = device_cus();
-    if (p.M <= kSkinnyMaxM) {
-        const int tile = skinny_tile(p.M, p.N, p.K, cus);
-        if (tile < 0) return launch_skinny<UNIT>(p, out_code, bias_code, has_bias, st);
-        launch_mid<UNIT>(p, tile, out_code, bias_code, has_bias, st);
-        return check_launch(UNIT ? "scaled_mm_fp8" : "scaled_mm_mxfp8");
+    const bool ws = workspace && workspace_bytes >= mx_split_workspace_bytes(p.M, p.N, p.K);
+    const Route r = mx_route(p.M, p.N, p.K, ws, device_cus());
+    switch (r.kind) {
+        case Route::kSkinny:
+            return launch_skinny<UNIT>(p, r.form, out_code, bias_code, has_bias, st);
+        case Route::kSmall:
+            launch_mid<UNIT>(p, r.form, out_code, bias_code, has_bias, st);
+            return check_launch(UNIT ? "scaled_mm_fp8" : "scaled_mm_mxfp8");
+        case Route::kSplit:
+            p.splits = r.split.S;
+            p.ks = r.split.ks;
+            p.part = static_cast<float*>(workspace);
+            if (r.split.nw == 2) launch_split<UNIT, 2>(p, out_code, bias_code, has_bias, st);
+            else launch_split<UNIT, 4>(p, out_code, bias_code, has_bias, st);
+            return check_launch(UNIT ? "scaled_mm_fp8" : "scaled_mm_mxfp8");
+        default: break;
     }
-    SplitPlan sp = split_plan(p.M, p.N, p.K);
-    if (!workspace || workspace_bytes < split_workspace_bytes(p.M, p.N, p.K)) sp.S = 1;
-    if (const int tile = mid_tile(p.M, p.N, p.K, sp, cus); tile >= 0) {
-        launch_mid<UNIT>(p, tile, out_code, bias_code, has_bias, st);
-        return check_launch(UNIT ? "scaled_mm_fp8" : "scaled_mm_mxfp8");
-    }
-    if (sp.S > 1) {
-        p.splits = sp.S;
-        p.ks = sp.ks;
-        p.part = static_cast<float*>(workspace);
-        if (sp.nw == 2) launch_split<UNIT, 2>(p, out_code, bias_code, has_bias, st);
-        else launch_split<UNIT, 4>(p, out_code, bias_code, has_bias, st);
-        return check_launch(UNIT ? "scaled_mm_fp8" : "scaled_mm_mxfp8");
-    }
-    const int tiles = p.tiles_m * p.tiles_n;
-    // (a grid of at most half as many tiles as CUs with no workspace for split-K runs all
-    // of its tiles as half tiles: 256 x 18432 x 3072 measured 31.9 against 41.3 us)
-    const int tail = tiles > kGemmSlots ? tiles % kGemmSlots : tiles;
-    p.n_half = (tail > 0 && tail <= kGemmSlots / 2) ? tail : 0;
-    p.n_full = tiles - p.n_half;
+    p.n_full = r.n_full;
+    p.n_half = r.n_half;
+    p.n_pref = r.n_pref;
     const int wgs = p.n_full + 2 * p.n_half;
-    // (the CUs the device has, which a partitioned GPU reduces: prefetch workgroups that
-    // found no idle CU would run after the tiles, for nothing)
-    p.n_pref = wgs < cus ? cus - wgs : 0;
     p.bias_code = bias_code;
     launch_grid<UNIT>(p, static_cast<unsigned>(wgs + p.n_pref), out_code, has_bias, st);
     return check_launch(UNIT ? "scaled_mm_fp8" : "scaled_mm_mxfp8");
@@ -1277,7 +1136,7 @@ mx::Args base_args(const void* a, const void* b, const void* bias, void* out, in
 
 extern "C" int64_t ckh_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || N <= 0 || K <= 0 || M >= (1ll << 30) || N >= (1ll << 30) || K >= (1ll << 24)) return 0;
-    return split_workspace_bytes(static_cast<int>(M), static_cast<int>(N), static_cast<int>(K));
+    return mx_split_workspace_bytes(static_cast<int>(M), static_cast<int>(N), static_cast<int>(K));
 }
 
 extern "C" int ckh_scaled_mm_mxfp8(const void* a, const void* b, const void* sa, const void* sb, const void* bias,

@@ -46,6 +46,7 @@
 #include <utility>
 
 #include "ckh_common.h"
+#include "dispatch.h"
 #include "gemm_mid_nv.h"
 #include "quant_math.h"
 #include "skinny.h"
@@ -112,9 +113,6 @@ struct Args {
     int bias_code;         // dtype code of bias
     const float* alpha_b;  // the weight's tensor scale (null: alpha is the product)
 };
-
-// fp32 values of one partial tile in the workspace (256 x 256, or two 256 x 128 halves)
-constexpr int kPartTile = BM * BN;
 
 // Direct-to-LDS loads of one operand's group.  Wave w, load j (0..7) covers rows
 // R = 64 w + 8 j .. +7 (1 KB of LDS; 32 w + 8 j, j = 0..3, for a 128-row half tile);
@@ -953,106 +951,9 @@ using namespace ckh;
 
 namespace {
 
-// Activations of at most kNvSkinnyMaxM rows take the skinny kernel (nvsk::gemm_skinny_kernel).
-constexpr int kNvSkinnyMaxM = 64;
-
-// Split-K: a grid of at most 128 tiles (half the CUs) with at least kNvMinSplitK groups of
-// 256 elements runs S K ranges of every tile (each of ks groups, the last one fewer, at
-// least kNvMinSplitGroups) as S times as many workgroups, at most 256, which write fp32
-// partial tiles to the caller's workspace; a second launch adds them.  A group costs about
-// 4 us of MFMA time per tile and a partial tile's round trip about as much as one group.
-// Ranges of an odd number of groups end mid-pair (measured against ranges rounded up to an
-// even count, same process: M = 256, N = 13824, K = 5120, four ranges of 5 instead of 6, 6,
-// 6, 2: 48.7 against 53.8 us; M = 300, N = 2000, K = 4160 35.0 against 39.6; M = 2048, N =
-// 4096, K = 5376 84.6 against 90.1).  Minimum range lengths of 2, 3, 6 and 8 groups
-// measured no better than 4 over six shapes (2: 300 x 2000 x 4160 30.9 against 34.4 us but
-// 256 x 3072 x 12288 36.5 against 35.4; 8: up to 40% slower).  Grids of at most
-// kNvHalfSplitTiles tiles split their 256 x 128 column halves instead (twice the units,
-// half the ranges: less partial traffic per unit of work), also in ranges of at least
-// kNvMinSplitGroups (3 measured 2-4% faster on three shapes but 16% slower on 512 x 3072 x
-// 3072; 2 slower on four of five).  Grids of 65-128 tiles split whole tiles only into three
-// ranges or more and from kNvMinSplitKFull groups on; otherwise they run as one round of
-// whole-K half tiles, which write no partials (same process, split against half tiles: two
-// ranges, 256 x 32768 x 5120 86.0 against 73.8 us, 2048 x 4096 x 5376 86.6 against 74.4,
-// 384 x 12288 x 6144 74.3 against 71.8; three ranges of 4 groups, 256 x 18432 x 3072 44.6
-// against 39.8; three of 11 and 7, 256 x 18432 x 8192 77.4 against 90.9 and 512 x 8704 x
-// 5120 55.7 against 59.5).
-constexpr int kNvSlots = 256;
-constexpr int kNvMinSplitK = 8;
-constexpr int kNvMinSplitKFull = 16;
-constexpr int kNvMinSplitGroups = 4;
-constexpr int kNvHalfSplitTiles = 64;
-// A last round of at most this many tiles runs them as half tiles (see ckh_scaled_mm_nvfp4).
-constexpr int kNvHalfTail = kNvSlots / 2;
-
-struct NvSplitPlan {
-    int S = 1;   // K ranges (1: no split)
-    int ks = 0;  // groups per range
-    int nw = 4;  // 4: full tiles, 2: half tiles
-};
-
-NvSplitPlan nv_split_plan(int64_t M, int64_t N, int64_t K) {
-    NvSplitPlan sp;
-    if (M <= kNvSkinnyMaxM) return sp;
-    const int tiles = static_cast<int>(cdiv(M, nv::BM) * cdiv(N, nv::BN));
-    const int NG = static_cast<int>(cdiv(K / 2, nv::GKB));
-    const bool half = tiles <= kNvHalfSplitTiles;
-    if (tiles > kNvSlots / 2 || NG < (half ? kNvMinSplitK : kNvMinSplitKFull)) return sp;
-    const int units = half ? 2 * tiles : tiles;
-    const int S = min(kNvSlots / units, NG / kNvMinSplitGroups);
-    if (S < (half ? 2 : 3)) return sp;
-    sp.ks = static_cast<int>(cdiv(NG, S));
-    sp.S = static_cast<int>(cdiv(NG, sp.ks));
-    sp.nw = half ? 2 : 4;
-    return sp;
-}
-
-// one partial tile (or two partial half tiles) per tile and K range
-int64_t nv_split_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    const NvSplitPlan sp = nv_split_plan(M, N, K);
-    if (sp.S < 2) return 0;
-    return cdiv(M, nv::BM) * cdiv(N, nv::BN) * sp.S * static_cast<int64_t>(nv::kPartTile) * 4;
-}
-
-// Small tiles (gemm_mid_nv.h): the first of these whose grid fits the CUs in one round, which
-// was the fastest of those that fit on all of 200 measured shapes of 65-1333 rows.  Time (us):
-// base + line per 256 elements of K.
-struct NvMidTile {
-    int tm, tn;
-    double base, line;
-};
-constexpr NvMidTile kNvMidTiles[] = {{64, 64, 5.0, 0.62}, {64, 128, 6.2, 0.8}, {128, 128, 8.5, 1.25}, {128, 192, 11.0, 1.75}};
-
-// Index of the small tile to use, or -1: that estimate against the 256 x 256 kernel's, fitted to
-// the same shapes: split-K 14 + 2.6 per group of a K range in half tiles (4.5 in whole tiles),
-// half tiles without a split 8.5 + 2.4 per group.  It took the slower form on 12 of the 200, by
-// 20% at most (768 x 1024 x 8192, where both formats' estimates are 24.5), and the small tiles
-// gained 1.39 x over all: 256 x 13824 x 5120 50.4 -> 41.9 us, 300 x 4096 x 4096 33.5 -> 19.7,
-// 128 x 3072 x 3072 21.7 -> 12.5, 65 x 5120 x 2048 22.4 -> 10.3.  Rows that do not start on a
-// cache line (K not a multiple of 256) take 6% longer (60 more shapes: 1.08 x the estimate in the
-// mean; 239 x 8824 x 4768 38.6, split-K 37.9).
-// At most 64 rows: 64 x 64 or 64 x 128 from 33 rows and N = 8192 on, K up to 8192 (graph-timed,
-// against the skinny kernel: 48 x 8192 x 3072 12.2 / 14.3 us, 64 x 12288 x 5120 17.7 / 20.8, 33 x
-// 18432 x 3072 16.3 / 21.5; with 32 rows 32 x 12288 x 3072 12.7 / 11.5, with K = 12288 33 x 8192
-// 32.5 / 30.9).
-int nv_mid_tile(int M, int N, int K, const NvSplitPlan& sp, int cus) {
-    if (M <= kNvSkinnyMaxM) {
-        if (M <= 32 || N < 8192 || K > 8192) return -1;
-        return cdiv(N, 64) <= cus ? 0 : cdiv(N, 128) <= cus ? 1 : -1;
-    }
-    const double groups = static_cast<double>(cdiv(K, 256));
-    const double lines = K % 256 ? 1.06 : 1.0;
-    for (int i = 0; i < static_cast<int>(sizeof(kNvMidTiles) / sizeof(kNvMidTiles[0])); ++i) {
-        const NvMidTile& t = kNvMidTiles[i];
-        if (cdiv(M, t.tm) * cdiv(N, t.tn) > cus) continue;
-        const double big = sp.S > 1 ? 14.0 + (sp.nw == 2 ? 2.6 : 4.5) * sp.ks : 8.5 + 2.4 * groups;
-        return (t.base + t.line * groups) * lines < big ? i : -1;
-    }
-    return -1;
-}
-
-template <int TM, int TN, int KG, int NST>
+template <int TILE, int KG, int NST>
 void launch_nv_mid_tile(const midnv::Args& p, int out_code, hipStream_t st) {
+    constexpr int TM = kNvSmall[TILE].tm, TN = kNvSmall[TILE].tn;
     const dim3 grid(static_cast<unsigned>(p.tiles_m * cdiv(p.N, TN)));
 #define LAUNCH(O) hipLaunchKernelGGL((midnv::gemm_mid_nv_kernel<O, TM, TN, KG, NST>), grid, dim3(mid::kThreads), 0, st, p)
     if (out_code == CKH_BF16) LAUNCH(CKH_BF16);
@@ -1066,15 +967,15 @@ void launch_nv_mid(const nv::Args& q, int tile, int out_code, int bias_code, hip
     p.a = q.a; p.b = q.b; p.sa = q.sa; p.sb = q.sb; p.alpha = q.alpha; p.alpha_b = q.alpha_b; p.bias = q.bias; p.out = q.out;
     p.bias_code = bias_code;
     p.M = q.M; p.N = q.N; p.K = q.K; p.ncb = q.ncb; p.sa_rows = q.sa_rows; p.sb_rows = q.sb_rows;
-    p.tiles_m = static_cast<int>(cdiv(p.M, kNvMidTiles[tile].tm));
+    p.tiles_m = static_cast<int>(cdiv(p.M, kNvSmall[tile].tm));
     // K groups: the more, the larger a wave's part of the tile and the fewer operand decodes per
     // MFMA (64 x 128 with 4 groups, 64 x 64 a wave: 15.7 us on 128 x 3072 x 3072; with 2 groups,
     // 32 x 64 a wave, 18.1; with 8, which add up three times in the epilogue, 18.7)
     switch (tile) {
-        case 0: launch_nv_mid_tile<64, 64, 4, 6>(p, out_code, st); break;
-        case 1: launch_nv_mid_tile<64, 128, 4, 5>(p, out_code, st); break;
-        case 2: launch_nv_mid_tile<128, 128, 4, 4>(p, out_code, st); break;
-        default: launch_nv_mid_tile<128, 192, 2, 3>(p, out_code, st); break;
+        case 0: launch_nv_mid_tile<0, 4, 6>(p, out_code, st); break;
+        case 1: launch_nv_mid_tile<1, 4, 5>(p, out_code, st); break;
+        case 2: launch_nv_mid_tile<2, 4, 4>(p, out_code, st); break;
+        default: launch_nv_mid_tile<3, 2, 3>(p, out_code, st); break;
     }
 }
 
@@ -1099,58 +1000,48 @@ void launch_nv_split(const nv::Args& p, int out_code, int bias_code, bool has_bi
 #undef LAUNCH
 }
 
-int launch_nv_skinny(const nv::Args& q, int out_code, int bias_code, bool has_bias, hipStream_t st) {
+int launch_nv_skinny(const nv::Args& q, int form, int out_code, int bias_code, bool has_bias, hipStream_t st) {
     nvsk::Args p{};
     p.a = q.a; p.b = q.b; p.sa = q.sa; p.sb = q.sb; p.alpha = q.alpha; p.alpha_b = q.alpha_b; p.bias = q.bias; p.out = q.out;
     p.M = q.M; p.N = q.N; p.K = q.K; p.ncb = q.ncb; p.sa_rows = q.sa_rows; p.sb_rows = q.sb_rows;
-    // Per activation size: waves per workgroup, weight tiles per workgroup, activation tiles,
-    // activation rows decoded to LDS, chunks in flight per wave.  Measured (graph-timed, K = 5120,
-    // N = 13824): M = 1 12.5 us, M = 8 13.0 us, M = 16 16.0 us; 8 waves, 3 chunks in flight, or
-    // activation fragments decoded in registers were 10-20% slower at M <= 8.  With fewer than
-    // 256 workgroups (N < 8192) 8 waves per workgroup pay instead (same process, against 4):
-    // M = 16, N = 5120, K = 13824 18.8 against 22.1 us; M = 16, N = 3072, K = 12288 17.0
-    // against 20.0; M = 1, N = 5120, K = 5120 8.1 against 8.8 (for the staged 32-row
-    // activation 8 waves measured 9-11% slower).  For M > 16 two
-    // weight tiles per workgroup halve the activation decoding per weight byte, which pays
-    // while N gives enough workgroups (M = 64: N = 13824 19.4 against 24.8 us with one tile;
-    // N = 5120, K = 13824 27.5 against 32.4 us with two).  With one tile (N < 8192) the
-    // activation codes are staged in LDS by whole-line loads rather than loaded by each lane
-    // (M = 32, N = 5120, K = 5120 10.0 against 10.4 us; M = 64, N = 3072, K = 12288 22.3
-    // against 24.7; M = 64, N = 5120, K = 13824 25.1 against 26.6); with two tiles that
-    // measured no better (19.6 against 19.5 us at M = 64, N = 13824).
-    const bool two = q.N >= 8192;
-#define LAUNCH(O, B, WV, NT, MT, AR, D, AS)                                                       \
-    do {                                                                                          \
-        if constexpr (WV == 8)                                                                    \
-            hipLaunchKernelGGL((nvsk::gemm_skinny_kernel8<O, B, NT, MT, AR, D, AS>),              \
-                               dim3(static_cast<unsigned>(cdiv(q.N, 32 * NT))), dim3(512), 0, st, p); \
-        else                                                                                      \
-            hipLaunchKernelGGL((nvsk::gemm_skinny_kernel<O, B, WV, NT, MT, AR, D, AS>),           \
-                               dim3(static_cast<unsigned>(cdiv(q.N, 32 * NT))), dim3(64 * WV), 0, st, p); \
-    } while (0)
-#define BY_MT(O, B)                                                \
-    do {                                                           \
-        if (p.M <= 8 && two) LAUNCH(O, B, 4, 1, 1, 8, 2, 0);       \
-        else if (p.M <= 8) LAUNCH(O, B, 8, 1, 1, 8, 2, 0);         \
-        else if (p.M <= 16 && two) LAUNCH(O, B, 4, 1, 1, 16, 2, 0); \
-        else if (p.M <= 16) LAUNCH(O, B, 8, 1, 1, 16, 2, 0);       \
-        else if (p.M <= 32 && two) LAUNCH(O, B, 4, 2, 1, 0, 2, 0); \
-        else if (p.M <= 32) LAUNCH(O, B, 4, 1, 1, 0, 2, 32);       \
-        else if (two) LAUNCH(O, B, 4, 2, 2, 0, 2, 0);              \
-        else LAUNCH(O, B, 4, 1, 2, 0, 2, 64);                      \
+#define LAUNCH(O, B, I)                                                                            \
+    case I:                                                                                        \
+        if constexpr (kNvSkinny[I].waves == 8)                                                     \
+            hipLaunchKernelGGL((nvsk::gemm_skinny_kernel8<O, B, kNvSkinny[I].weight_tiles, kNvSkinny[I].act_tiles, \
+                                                          kNvSkinny[I].act_rows, 2, kNvSkinny[I].code_rows>), \
+                               dim3(static_cast<unsigned>(cdiv(q.N, 32 * kNvSkinny[I].weight_tiles))), dim3(512), 0, st, p); \
+        else                                                                                       \
+            hipLaunchKernelGGL((nvsk::gemm_skinny_kernel<O, B, kNvSkinny[I].waves, kNvSkinny[I].weight_tiles, \
+                                                         kNvSkinny[I].act_tiles, kNvSkinny[I].act_rows, 2, \
+                                                         kNvSkinny[I].code_rows>),                 \
+                               dim3(static_cast<unsigned>(cdiv(q.N, 32 * kNvSkinny[I].weight_tiles))), \
+                               dim3(64 * kNvSkinny[I].waves), 0, st, p);                           \
+        break
+#define BY_FORM(O, B)        \
+    do {                     \
+        switch (form) {      \
+            LAUNCH(O, B, 0); \
+            LAUNCH(O, B, 1); \
+            LAUNCH(O, B, 2); \
+            LAUNCH(O, B, 3); \
+            LAUNCH(O, B, 4); \
+            LAUNCH(O, B, 5); \
+            LAUNCH(O, B, 6); \
+            LAUNCH(O, B, 7); \
+        }                    \
     } while (0)
 #define BY_BIAS(O)                                          \
     do {                                                    \
-        if (!has_bias) BY_MT(O, -1);                        \
-        else if (bias_code == CKH_F32) BY_MT(O, CKH_F32);   \
-        else if (bias_code == CKH_F16) BY_MT(O, CKH_F16);   \
-        else BY_MT(O, CKH_BF16);                            \
+        if (!has_bias) BY_FORM(O, -1);                        \
+        else if (bias_code == CKH_F32) BY_FORM(O, CKH_F32);   \
+        else if (bias_code == CKH_F16) BY_FORM(O, CKH_F16);   \
+        else BY_FORM(O, CKH_BF16);                            \
     } while (0)
     if (out_code == CKH_BF16) BY_BIAS(CKH_BF16);
     else if (out_code == CKH_F16) BY_BIAS(CKH_F16);
     else BY_BIAS(CKH_F32);
 #undef BY_BIAS
-#undef BY_MT
+#undef BY_FORM
 #undef LAUNCH
     return check_launch("scaled_mm_nvfp4");
 }
@@ -1199,28 +1090,25 @@ int scaled_mm_nvfp4(const void* a, const void* b, const void* sa, const void* sb
     p.tiles_m = static_cast<int>(cdiv(M, nv::BM));
     p.tiles_n = static_cast<int>(cdiv(N, nv::BN));
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    NvSplitPlan sp = nv_split_plan(M, N, K);
-    if (!workspace || workspace_bytes < nv_split_workspace_bytes(M, N, K)) sp.S = 1;
-    if (const int tile = nv_mid_tile(p.M, p.N, p.K, sp, device_cus()); tile >= 0) {
-        launch_nv_mid(p, tile, out_code, bias_code, st);
-        return check_launch("scaled_mm_nvfp4");
+    const bool ws = workspace && workspace_bytes >= nv_split_workspace_bytes(M, N, K);
+    const Route r = nv_route(p.M, p.N, p.K, ws, device_cus());
+    switch (r.kind) {
+        case Route::kSkinny:
+            return launch_nv_skinny(p, r.form, out_code, bias_code, bias != nullptr, st);
+        case Route::kSmall:
+            launch_nv_mid(p, r.form, out_code, bias_code, st);
+            return check_launch("scaled_mm_nvfp4");
+        case Route::kSplit:
+            p.splits = r.split.S;
+            p.ks = r.split.ks;
+            p.part = static_cast<float*>(workspace);
+            if (r.split.nw == 2) launch_nv_split<2>(p, out_code, bias_code, bias != nullptr, st);
+            else launch_nv_split<4>(p, out_code, bias_code, bias != nullptr, st);
+            return check_launch("scaled_mm_nvfp4");
+        default: break;
     }
-    if (p.M <= kNvSkinnyMaxM) return launch_nv_skinny(p, out_code, bias_code, bias != nullptr, st);
-    if (sp.S > 1) {
-        p.splits = sp.S;
-        p.ks = sp.ks;
-        p.part = static_cast<float*>(workspace);
-        if (sp.nw == 2) launch_nv_split<2>(p, out_code, bias_code, bias != nullptr, st);
-        else launch_nv_split<4>(p, out_code, bias_code, bias != nullptr, st);
-        return check_launch("scaled_mm_nvfp4");
-    }
-    // The tiles run one per CU in rounds.  When the last round would be at most half full,
-    // its tiles run as twice as many 256 x 128 half tiles in the same grid (a grid of one
-    // round with no split-K workspace runs all of its tiles so).
-    const int tiles = p.tiles_m * p.tiles_n;
-    const int tail = tiles > kNvSlots ? tiles % kNvSlots : tiles;
-    p.n_half = (tail > 0 && tail <= kNvHalfTail) ? tail : 0;
-    p.n_full = tiles - p.n_half;
+    p.n_full = r.n_full;
+    p.n_half = r.n_half;
     dim3 grid(static_cast<unsigned>(p.n_full + 2 * p.n_half));
     p.bias_code = bias_code;
 #define LAUNCH(O)                                                                                       \

@@ -1,7 +1,9 @@
-// Host-side facts about the small-tile GEMMs, from the kernels' own headers.  TEST CODE ONLY:
-// built into tests/hw/libckh_hwcheck.so; nothing here runs on a GPU.
+// Host-side facts about the GEMMs, from the kernels' own headers: the kernel that a call's sizes
+// select, and the small tiles' bias columns.  TEST CODE ONLY: built into
+// tests/hw/libckh_hwcheck.so; nothing here runs on a GPU.
 #include <algorithm>
 
+#include "dispatch.h"
 #include "gemm_mid.h"
 #include "gemm_mid_nv.h"
 
@@ -52,4 +54,33 @@ extern "C" int ckh_tile_bias_end(int nv, int tm, int tn) {
 #undef MX
 #undef NV
     return 0;
+}
+
+// The kernel that serves a GEMM call on a device of `cus` CUs: fills out[0..5] and returns
+//   0 skinny     waves, weight tiles, activation tiles, staged or decoded activation rows, code rows
+//   1 small tile rows, columns
+//   2 split-K    ranges, stages (MXFP8, FP8) or groups (NVFP4) per range, 4 whole / 2 half tiles
+//   3 tiles      whole tiles, tiles run as two halves, weight-prefetch workgroups
+extern "C" int ckh_route(int nv, int64_t M, int64_t N, int64_t K, int workspace, int cus, int* out) {
+    const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
+    const Route r = nv ? nv_route(m, n, k, workspace != 0, cus) : mx_route(m, n, k, workspace != 0, cus);
+    std::fill(out, out + 6, 0);
+    if (r.kind == Route::kSkinny) {
+        const SkinnyForm f = nv ? kNvSkinny[r.form] : kMxSkinny[r.form];
+        out[0] = f.waves, out[1] = f.weight_tiles, out[2] = f.act_tiles, out[3] = f.act_rows, out[4] = f.code_rows;
+    } else if (r.kind == Route::kSmall) {
+        out[0] = nv ? kNvSmall[r.form].tm : kMxSmall[r.form].tm;
+        out[1] = nv ? kNvSmall[r.form].tn : kMxSmall[r.form].tn;
+    } else if (r.kind == Route::kSplit) {
+        out[0] = r.split.S, out[1] = r.split.ks, out[2] = r.split.nw;
+    } else {
+        out[0] = r.n_full, out[1] = r.n_half, out[2] = r.n_pref;
+    }
+    return r.kind;
+}
+
+// Number of skinny forms of a format.
+extern "C" int ckh_skinny_forms(int nv) {
+    return nv ? static_cast<int>(sizeof(kNvSkinny) / sizeof(kNvSkinny[0]))
+              : static_cast<int>(sizeof(kMxSkinny) / sizeof(kMxSkinny[0]));
 }
