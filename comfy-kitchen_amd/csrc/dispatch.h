@@ -43,30 +43,36 @@ struct Route {
 };
 
 // ------------------------------------------------------------------ MXFP8, per-tensor FP8
-// The skinny form by activation size (N = 18432, K = 3072: M = 1 12.7 us, M = 16 15.4 us).  With 16 activation rows the waves per workgroup follow N: 2 waves when there are at least
-// 256 workgroups (M = 16, N = 18432: 14.6 against 15.4 us with 4), 8 when there are fewer than
-// 128 (N = 3072, K = 12288: 16.6 against 17.2 us; with 2 waves 25.9 us).  With 4-8 rows and N
-// above 16384, 2 waves rather than 8 (M = 8, N = 18432, K = 3072 13.4 against 14.5 us; N =
-// 24576 14.9 against 15.8; M = 4 13.1 against 13.6; M = 1 and 2 and N = 16384 equal).  From 17
-// rows on this kernel serves what mx_few_rows_tile leaves: N below 8192, where its waves' split of K
-// keeps more of the chip busy than small tiles would (32 x 5120 x 5120 11.6 against 16.1 us,
-// 64 x 5120 x 12288 27.7 against 37.0); 17-32 rows with a short K (2 waves and one tile up to N
-// = 24576: 20 x 18432 x 3072 16.4 against 17.3 with 4 waves; 2 waves and two tiles beyond: 20 x
-// 32768 x 3072 20.2 against 22.0); and N beyond one round of 64 x 128 tiles.  There the
-// activation is staged through LDS too, 32 or 64 rows (N = 5120, K = 5120, M = 32 10.8
-// against 16.5 with the fragments loaded into registers; M = 64, K = 13824 29.3 against 47.4).
+// The skinny form by activation size (N = 18432, K = 3072: M = 1 12.7 us, M = 16 15.4 us).  With
+// 16 activation rows the waves per workgroup follow N: 2 waves when there are at least 256
+// workgroups (M = 16, N = 18432: 14.6 against 15.4 us with 4), 8 when there are fewer than 128
+// (N = 3072, K = 12288: 16.6 against 17.2 us; with 2 waves 25.9 us).  With 4-8 rows and N above
+// 16384, 2 waves rather than 8 (M = 8, N = 18432, K = 3072 13.4 against 14.5 us; N = 24576 14.9
+// against 15.8; M = 4 13.1 against 13.6; M = 1 and 2 and N = 16384 equal).  From 17 rows on this
+// kernel serves what mx_few_rows_tile leaves: N below 8192, where its waves' split of K keeps
+// more of the chip busy than small tiles would (32 x 5120 x 5120 11.6 against 16.1 us, 64 x 5120
+// x 12288 27.7 against 37.0); short K; 17-32 rows of a narrow layer; and N beyond one round of 64
+// x 128 tiles.  There the activation is staged through LDS too, 32 or 64 rows (N = 5120, K =
+// 5120, M = 32 10.8 against 16.5 us with the fragments loaded into registers; M = 64, K = 13824
+// 29.3 against 47.4), and the choice follows how many workgroups one round holds: 17-32 rows 4
+// waves and two weight tiles up to N = 16384 (K = 5120 18.7 against 19.8 us with one tile); then
+// one tile with 2 waves (20 x 18432 x 3072 16.4 against 17.3 with 4) or, from K = 4096 on, 4 (32
+// x 18432 x 12288 57.4 against 57.7 with 2 waves and two tiles); 2 waves and two tiles beyond N =
+// 24576 (20 x 32768 x 3072 20.2 against 22.0); 33-64 rows 2 waves and one tile (three workgroups
+// of 48 KB per CU) up to N = 24576 (64 x 18432 x 3072 20.6 against 21.6 with two tiles), two
+// tiles beyond (64 x 32768 x 3072 25.2 against 29.1).
 // The NVFP4 skinny kernel's form (128-byte chunks, two in flight per wave) measured slower
 // here, where a chunk costs only a few MFMAs: M = 1 14.5 against 12.9 us, M = 16 15.9 against
 // 15.5, M = 64 29.6 against 26.5 (same process).
-constexpr SkinnyForm kMxSkinny[] = {{8, 1, 1, 8},  {2, 1, 1, 8},  {8, 1, 1, 16}, {4, 1, 1, 16},
-                                    {2, 1, 1, 16}, {8, 1, 1, 32}, {4, 2, 1, 32}, {2, 1, 1, 32},
-                                    {2, 2, 1, 32}, {4, 1, 2, 64}, {2, 2, 2, 64}};
+constexpr SkinnyForm kMxSkinny[] = {{8, 1, 1, 8},  {2, 1, 1, 8},  {8, 1, 1, 16}, {4, 1, 1, 16}, {2, 1, 1, 16},
+                                    {8, 1, 1, 32}, {4, 2, 1, 32}, {2, 1, 1, 32}, {2, 2, 1, 32}, {4, 1, 1, 32},
+                                    {4, 1, 2, 64}, {2, 2, 2, 64}, {2, 1, 2, 64}};
 
-inline int mx_skinny_form(int M, int N) {
+inline int mx_skinny_form(int M, int N, int K) {
     if (M <= 8) return M >= 4 && N > 16384 ? 1 : 0;
     if (M <= 16) return N >= 8192 ? 4 : N >= 4096 ? 3 : 2;
-    if (M <= 32) return N > 24576 ? 8 : N > 16384 ? 7 : N >= kSkinnySmallN ? 6 : 5;
-    return N >= kSkinnySmallN ? 10 : 9;
+    if (M <= 32) return N > 24576 ? 8 : N > 16384 ? (K <= 4096 ? 7 : 9) : N >= kSkinnySmallN ? 6 : 5;
+    return N < kSkinnySmallN ? 10 : N > 24576 ? 11 : 12;
 }
 
 // Split-K: a grid of at most half as many 256 x 256 tiles as CUs leaves most CUs idle
@@ -154,16 +160,26 @@ inline int mx_small_tile(int M, int N, int K, const SplitPlan& sp, int cus) {
 }
 
 // The small tile for at most 64 rows, or -1 for the skinny kernel: from 17 rows and N = 8192 on,
-// 64 x 64 or 64 x 128, whichever fits in one round (graph-timed, against the skinny kernel: 24 x
-// 8192 x 5120 16.3 / 17.5 us, 48 x 12288 x 3072 13.0 / 17.1, 64 x 8192 x 12288 37.7 / 46.0, 33 x
-// 18432 x 3072 18.0 / 21.0, 64 x 24576 x 5120 33.6 / 40.3; with 16 rows level).  With 17-32 rows
-// a short K leaves the ring's fill and the one workgroup per CU in view: 32 x 9000 x 512 5.5 / 5.3,
-// 17 x 21504 x 3072 18.7 / 16.5, but 32 x 16384 x 3072 12.8 / 14.3, 17 x 21504 x 5120 26.3 / 30.3.
+// 64 x 64 or 64 x 128, whichever fits in one round, where K is long enough to make up for the ring's
+// fill and the one workgroup per CU.  Measured against the skinny kernel on 3,600 shapes, graph-timed
+// both with every call's weight read anew and with one weight that stays in the caches (small tile /
+// skinny, us, anew; the same kept):
+//   33-64 rows  64 x 64 at any K: 64 x 8192 x 12288 37.7 / 46.0; the mean of all 0.91; 0.72 kept.
+//               64 x 128 from K = 1280 on (640 above N = 24576): 52 x 19808 x 512 7.4 / 5.9; 6.5 / 5.2,
+//               57 x 17328 x 1024 9.6 / 8.1; 8.2 / 7.6, 64 x 24576 x 5120 33.6 / 40.3.
+//   17-32 rows  they gain only where the weight is in the caches, so they stay where they are level
+//               otherwise (in the mean 1.00; 0.82 kept): 64 x 64 above N = 10240 from K = 3072 on (25 x
+//               8688 x 1024 6.8 / 5.2; 5.9 / 4.2, 32 x 9688 x 2624 11.6 / 10.6; 8.4 / 6.6); 64 x 128
+//               above K = 4096, up to N = 24576 only with whole lines (K a multiple of 128; 29 x 20408 x
+//               6880 42.1 / 36.7; 26.7 / 35.7).
+// With 16 rows they are level.
 inline int mx_few_rows_tile(int M, int N, int K, int cus) {
     if (M <= 16 || N < kSkinnySmallN) return -1;
-    if (cdiv(N, 64) <= cus) return M <= 32 && K < 1024 ? -1 : 0;
-    if (cdiv(N, 128) <= cus) return M <= 32 && K <= 4096 ? -1 : kMxSmallWide;
-    return -1;
+    const bool few = M <= 32;
+    if (cdiv(N, 64) <= cus) return few && (N <= 10240 || K < 3072) ? -1 : 0;
+    if (cdiv(N, 128) > cus) return -1;
+    if (few) return K <= 4096 || (K % 128 && N <= 24576) ? -1 : kMxSmallWide;
+    return K < (N <= 24576 ? 1280 : 640) ? -1 : kMxSmallWide;
 }
 
 // The 256 x 256 tiles run one per CU in rounds.  When the last round would be at most
@@ -188,7 +204,7 @@ inline Route mx_route(int M, int N, int K, bool workspace, int cus) {
     if (M <= kSkinnyMaxM) {
         r.form = mx_few_rows_tile(M, N, K, cus);
         r.kind = r.form >= 0 ? Route::kSmall : Route::kSkinny;
-        if (r.form < 0) r.form = mx_skinny_form(M, N);
+        if (r.form < 0) r.form = mx_skinny_form(M, N, K);
         return r;
     }
     r.split = mx_split_plan(M, N, K);

@@ -1004,21 +1004,23 @@ int launch_skinny(const mx::Args& q, int form, int out_code, int bias_code, bool
                            dim3(static_cast<unsigned>(cdiv(q.N, 32 * kMxSkinny[I].weight_tiles))), \
                            dim3(64 * kMxSkinny[I].waves), 0, st, p);                              \
         break
-#define BY_FORM(O, B)        \
-    do {                     \
-        switch (form) {      \
-            LAUNCH(O, B, 0); \
-            LAUNCH(O, B, 1); \
-            LAUNCH(O, B, 2); \
-            LAUNCH(O, B, 3); \
-            LAUNCH(O, B, 4); \
-            LAUNCH(O, B, 5); \
-            LAUNCH(O, B, 6); \
-            LAUNCH(O, B, 7); \
-            LAUNCH(O, B, 8); \
-            LAUNCH(O, B, 9); \
+#define BY_FORM(O, B)         \
+    do {                      \
+        switch (form) {       \
+            LAUNCH(O, B, 0);  \
+            LAUNCH(O, B, 1);  \
+            LAUNCH(O, B, 2);  \
+            LAUNCH(O, B, 3);  \
+            LAUNCH(O, B, 4);  \
+            LAUNCH(O, B, 5);  \
+            LAUNCH(O, B, 6);  \
+            LAUNCH(O, B, 7);  \
+            LAUNCH(O, B, 8);  \
+            LAUNCH(O, B, 9);  \
             LAUNCH(O, B, 10); \
-        }                    \
+            LAUNCH(O, B, 11); \
+            LAUNCH(O, B, 12); \
+        }                     \
     } while (0)
 #define BY_BIAS(O)                                          \
     do {                                                    \

@@ -20,3 +20,22 @@ def test_every_skinny_form_is_reached():
         seen = {route(fmt, m, n, k) for m in (1, 4, 8, 12, 16, 17, 24, 32, 33, 48, 64)
                 for n in (64, 4096, 8192, 16384, 16392, 24576, 24584, 32768, 40000) for k in (512, 1024, 4096, 4128, 12288)}
         assert len({r for r in seen if r[0] == "skinny"}) == library().ckh_skinny_forms(nv)
+
+
+@pytest.mark.parametrize("m,n,k,want", [
+    (25, 8688, 1024, (4, 2, 1, 32)), (32, 9688, 2624, (4, 2, 1, 32)), (24, 10240, 5120, (4, 2, 1, 32)),
+    (32, 16384, 2048, (4, 2, 1, 32)), (18, 16392, 4096, (2, 1, 1, 32)), (29, 20408, 6880, (4, 1, 1, 32)),
+    (17, 24576, 4128, (4, 1, 1, 32)), (32, 30000, 4096, (2, 2, 1, 32)), (52, 19808, 512, (2, 1, 2, 64)),
+    (33, 16392, 1248, (2, 1, 2, 64)), (64, 24576, 1024, (2, 1, 2, 64)), (64, 32768, 512, (2, 2, 2, 64)),
+    (40, 40000, 3072, (2, 2, 2, 64))])
+def test_few_rows_short_k_or_narrow_take_the_skinny_kernel(m, n, k, want):
+    """Where the small tiles measured slower than the skinny kernel, in the form that measured best."""
+    assert route("mx", m, n, k)[:5] == ("skinny", *want)
+
+
+@pytest.mark.parametrize("m,n,k,want", [
+    (32, 16384, 3072, (64, 64)), (17, 10248, 5120, (64, 64)), (17, 24576, 4224, (64, 128)),
+    (20, 32768, 4128, (64, 128)), (64, 8192, 512, (64, 64)), (33, 16384, 32, (64, 64)),
+    (48, 18432, 1280, (64, 128)), (64, 32768, 640, (64, 128))])
+def test_few_rows_small_tiles(m, n, k, want):
+    assert route("mx", m, n, k) == ("small", *want)
