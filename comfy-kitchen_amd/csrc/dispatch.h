@@ -309,13 +309,14 @@ constexpr NvSmallTile kNvSmall[] = {{64, 64, 5.0, 0.62}, {64, 128, 6.2, 0.8}, {1
 // 128 x 3072 x 3072 21.7 -> 12.5, 65 x 5120 x 2048 22.4 -> 10.3.  Rows that do not start on a
 // cache line (K not a multiple of 256) take 6% longer (60 more shapes: 1.08 x the estimate in the
 // mean; 239 x 8824 x 4768 38.6, split-K 37.9).
-// At most 64 rows: 64 x 64 or 64 x 128 from 33 rows and N = 8192 on, K up to 8192 (graph-timed,
-// against the skinny kernel: 48 x 8192 x 3072 12.2 / 14.3 us, 64 x 12288 x 5120 17.7 / 20.8, 33 x
-// 18432 x 3072 16.3 / 21.5; with 32 rows 32 x 12288 x 3072 12.7 / 11.5, with K = 12288 33 x 8192
-// 32.5 / 30.9).
+// At most 64 rows: 64 x 64 or 64 x 128 from 33 rows and N = 8192 on, K up to 8192, and from K = 1024
+// on where rows do not start on a cache line (graph-timed, against the skinny kernel: 48 x 8192 x 3072
+// 12.2 / 14.3 us, 64 x 12288 x 5120 17.7 / 20.8, 33 x 18432 x 3072 16.3 / 21.5; with 32 rows 32 x 12288
+// x 3072 12.7 / 11.5, with K = 12288 33 x 8192 32.5 / 30.9; 50 x 9232 x 928 8.7 / 7.1 and, over 190
+// such shapes, 1.06 with the weight read anew and 1.00 with it in the caches).
 inline int nv_small_tile(int M, int N, int K, const SplitPlan& sp, int cus) {
     if (M <= kSkinnyMaxM) {
-        if (M <= 32 || N < 8192 || K > 8192) return -1;
+        if (M <= 32 || N < 8192 || K > 8192 || (K % 256 && K < 1024)) return -1;
         return cdiv(N, 64) <= cus ? 0 : cdiv(N, 128) <= cus ? 1 : -1;
     }
     const double groups = static_cast<double>(cdiv(K, 256));

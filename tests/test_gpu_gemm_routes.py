@@ -56,3 +56,22 @@ def test_mxfp8_and_fp8(m, n, k, want, hip):
     ta, tb = torch.full((1,), 0.37, device="cuda"), torch.full((1,), 0.021, device="cuda")
     product = (qx.float() @ qw.float().t()) * (ta * tb)
     _check(lambda b, o: ck.scaled_mm_fp8(qx, qw, ta, tb, bias=b, out_dtype=o), product, bias, m, n)
+
+
+NV = [  # 33-64 rows with two weight tiles per workgroup: short ragged K, long K, N past one round of small tiles
+    (50, 9233, 928, ("skinny", 4, 2, 2, 0, 0)), (33, 8193, 96, ("skinny", 4, 2, 2, 0, 0)),
+    (64, 8205, 8224, ("skinny", 4, 2, 2, 0, 0)), (40, 32771, 544, ("skinny", 4, 2, 2, 0, 0)),
+]
+
+
+@pytest.mark.parametrize("m,n,k,want", NV)
+def test_nvfp4(m, n, k, want, hip):
+    assert route("nv", m, n, k) == want
+    x, w, bias = _inputs(m, n, k)
+    qx, sx, gx = ck.quantize_nvfp4_dynamic(x)
+    qw, sw, gw = ck.quantize_nvfp4_dynamic(w)
+    product = ck.dequantize_nvfp4(qx, gx, sx, torch.float32) @ ck.dequantize_nvfp4(qw, gw, sw, torch.float32).t()
+    scaled = _check(lambda b, o: ck.scaled_mm_nvfp4(qx, qw, gx, gw, sx, sw, bias=b, out_dtype=o), product, bias, m, n)
+    # two tensor scales give the bits that their fp32 product, passed as alpha, gives
+    alpha = ck.scaled_mm_nvfp4(qx, qw, gx, gw, sx, sw, alpha=gx * gw, out_dtype=torch.float32)
+    assert torch.equal(scaled, alpha)

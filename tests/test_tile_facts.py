@@ -39,3 +39,12 @@ def test_few_rows_short_k_or_narrow_take_the_skinny_kernel(m, n, k, want):
     (48, 18432, 1280, (64, 128)), (64, 32768, 640, (64, 128))])
 def test_few_rows_small_tiles(m, n, k, want):
     assert route("mx", m, n, k) == ("small", *want)
+
+
+@pytest.mark.parametrize("m,n,k,want", [
+    (50, 9232, 928, ("skinny", 4, 2, 2, 0, 0)), (64, 30000, 992, ("skinny", 4, 2, 2, 0, 0)),
+    (33, 8192, 32, ("skinny", 4, 2, 2, 0, 0)), (33, 8192, 768, ("small", 64, 64)), (40, 8200, 1056, ("small", 64, 64)),
+    (64, 17001, 1024, ("small", 64, 128)), (32, 9000, 1024, ("skinny", 4, 2, 1, 0, 0))])
+def test_nvfp4_few_rows(m, n, k, want):
+    """Short rows that do not start on a cache line measured slower in small tiles."""
+    assert route("nv", m, n, k) == want
