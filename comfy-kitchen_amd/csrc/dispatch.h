@@ -142,15 +142,19 @@ constexpr int kMxSmallWide = 6;  // 64 x 128, for at most 64 rows only (mx_small
 //   half tiles   6.2 + 0.4 per stage of K (200 x 21504 x 512: 9.5 measured, small tiles 12.1).
 // With K not a multiple of 128 a stage's piece of a row lies in two cache lines, and lines are
 // what a CU's intake is counted in: the terms per stage of the one-launch forms take 1.45 x (84 x
-// 12624 x 9824 53.1 against 38.9, 360 x 9584 x 2400 23.6 against 17.3), 1.1 x where more than 6
-// tiles share a weight row, which then comes from L2 (691 x 1312 x 5824 16.2 against 17.5).  118 x
-// 2448 x 6304: small tiles 25.0, split-K 21.0; 460 x 3112 x 9312 43.5 and 37.5.
+// 12624 x 9824 53.1 against 38.9, 360 x 9584 x 2400 23.6 against 17.3), 1.33 x where more than 6
+// tiles share a weight row, part of which then comes from L2 (691 x 1312 x 5824 16.2 against 17.5,
+// 1024 x 4368 x 13728 103 against 81 split with the weight read anew, 80 against 72 with it in the
+// caches; 1.1 x chose the small tiles there).  118 x 2448 x 6304: small tiles 25.0, split-K 21.0; 460
+// x 3112 x 9312 43.5 and 37.5.  Over 4,200 shapes of 65-1400 rows the small tiles it chooses take
+// 0.57 of the time; 1% of the choices are more than 5% slower, at most 20%, where the two
+// estimates are close.
 inline int mx_small_tile(int M, int N, int K, const SplitPlan& sp, int cus) {
     for (int i = 0; i < kMxSmallWide; ++i) {
         const SmallTile t = kMxSmall[i];
         if (cdiv(M, t.tm) * cdiv(N, t.tn) > cus) continue;
         const double rows = t.tm + t.tn;
-        const double lines = K % 128 == 0 ? 1.0 : cdiv(M, t.tm) <= 6 ? 1.45 : 1.1;
+        const double lines = K % 128 == 0 ? 1.0 : cdiv(M, t.tm) <= 6 ? 1.45 : 1.33;
         const double mid = 2.0 + 0.0165 * rows + 0.00228 * rows * lines * static_cast<double>(cdiv(K, 128));
         const double big = sp.S > 1 ? 14.7 + (sp.nw == 2 ? 0.575 : 1.09) * sp.ks
                                     : 6.2 + 0.4 * lines * static_cast<double>(cdiv(K, 64));

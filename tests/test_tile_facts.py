@@ -48,3 +48,12 @@ def test_few_rows_small_tiles(m, n, k, want):
 def test_nvfp4_few_rows(m, n, k, want):
     """Short rows that do not start on a cache line measured slower in small tiles."""
     assert route("nv", m, n, k) == want
+
+
+@pytest.mark.parametrize("m,n,k,want", [
+    (1024, 4368, 13728, ("split", 3, 72, 4)), (848, 560, 7072, ("split", 7, 16, 2)),
+    (691, 1312, 5824, ("small", 64, 64)), (1024, 4336, 4096, ("small", 128, 160))])
+def test_ragged_rows_shared_by_many_tiles(m, n, k, want):
+    """Rows that do not start on a cache line cost small tiles more, also with over six of them
+    along m: long K splits there, as it measured faster."""
+    assert route("mx", m, n, k) == want
