@@ -303,16 +303,16 @@ struct NvSmallTile {
     int tm, tn;
     double base, line;
 };
-constexpr NvSmallTile kNvSmall[] = {{64, 64, 5.0, 0.62}, {64, 128, 6.2, 0.8}, {128, 128, 8.5, 1.25}, {128, 192, 11.0, 1.75}};
+constexpr NvSmallTile kNvSmall[] = {{64, 64, 5.0, 0.66}, {64, 128, 6.2, 0.8}, {128, 128, 8.5, 1.25}, {128, 192, 11.0, 1.75}};
 
 // Index of the small tile to use, or -1: that estimate against the 256 x 256 kernel's, fitted to
 // the same shapes: split-K 14 + 2.6 per group of a K range in half tiles (4.5 in whole tiles),
-// half tiles without a split 8.5 + 2.4 per group.  It took the slower form on 12 of the 200, by
-// 20% at most (768 x 1024 x 8192, where both formats' estimates are 24.5), and the small tiles
-// gained 1.39 x over all: 256 x 13824 x 5120 50.4 -> 41.9 us, 300 x 4096 x 4096 33.5 -> 19.7,
-// 128 x 3072 x 3072 21.7 -> 12.5, 65 x 5120 x 2048 22.4 -> 10.3.  Rows that do not start on a
-// cache line (K not a multiple of 256) take 6% longer (60 more shapes: 1.08 x the estimate in the
-// mean; 239 x 8824 x 4768 38.6, split-K 37.9).
+// half tiles without a split 8.5 + 2.4 per group.  Over 2,780 more shapes of 65-1400 rows the small
+// tiles took 0.55 of the time and one of 2,250 choices was more than 3% slower (0.62 per line of 64 x
+// 64 tiles chose them for long K too: 200 x 792 x 8704 24.2 against 22.1 us split).  256 x 13824 x
+// 5120 50.4 -> 41.9 us, 300 x 4096 x 4096 33.5 -> 19.7, 128 x 3072 x 3072 21.7 -> 12.5, 65 x 5120 x
+// 2048 22.4 -> 10.3.  Rows that do not start on a cache line (K not a multiple of 256) take 6% longer
+// (60 more shapes: 1.08 x the estimate in the mean; 239 x 8824 x 4768 38.6, split-K 37.9).
 // At most 64 rows: 64 x 64 or 64 x 128 from 33 rows and N = 8192 on, K up to 8192, and from K = 1024
 // on where rows do not start on a cache line (graph-timed, against the skinny kernel: 48 x 8192 x 3072
 // 12.2 / 14.3 us, 64 x 12288 x 5120 17.7 / 20.8, 33 x 18432 x 3072 16.3 / 21.5; with 32 rows 32 x 12288

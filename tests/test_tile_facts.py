@@ -57,3 +57,9 @@ def test_ragged_rows_shared_by_many_tiles(m, n, k, want):
     """Rows that do not start on a cache line cost small tiles more, also with over six of them
     along m: long K splits there, as it measured faster."""
     assert route("mx", m, n, k) == want
+
+
+@pytest.mark.parametrize("m,n,k,want", [
+    (200, 792, 8704, ("split", 7, 5, 2)), (146, 576, 7040, ("split", 7, 4, 2)), (200, 792, 4096, ("small", 64, 64))])
+def test_nvfp4_narrow_layers_with_long_k_split(m, n, k, want):
+    assert route("nv", m, n, k) == want
