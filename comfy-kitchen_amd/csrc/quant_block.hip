@@ -12,6 +12,7 @@
 //   MXFP8: 32-element blocks, 4 lanes per block, 16 lanes per unit.
 //   NVFP4: 16-element blocks, 2 lanes per block,  8 lanes per unit.
 #include "ckh_common.h"
+#include "dispatch.h"
 #include "quant_math.h"
 
 namespace ckh {
@@ -272,7 +273,8 @@ __global__ __launch_bounds__(kThreads) void quantize_nvfp4_kernel(const void* __
 
 // ------------------------------------------------------- NVFP4, 16-bit fast path
 // For bf16/f16 inputs with no column padding, cols % 64 == 0, 16-byte aligned, < 2^31
-// elements; rows from orows to rows (pad_16x) are zeros that are not read.  One lane per 16-element block, four lanes per unit (one scale word), two
+// elements; rows from orows to rows (pad_16x) are zeros that are not read (with a given scale, see
+// nv_quantize_fast_rows).  One lane per 16-element block, four lanes per unit (one scale word), two
 // units per thread.  A lane's block is two 16-byte chunks that another lane's loads
 // share (nv_pair_exchange), so that each load instruction reads one contiguous KB
 // rather than every other 16 bytes of 2 KB (which measured 6% slower).  The IEEE
@@ -860,7 +862,7 @@ extern "C" int ckh_quantize_nvfp4(const void* x, const void* global_scale, void*
     uint8_t* q = static_cast<uint8_t*>(qx);
     uint32_t* s = static_cast<uint32_t*>(scales);
     const bool hf = hi_first != 0;
-    if (nvfp4_fast_applies(x, qx, scales, rows, cols, orig_cols, in_code)) {
+    if (nvfp4_fast_applies(x, qx, scales, rows, cols, orig_cols, in_code) && nv_quantize_fast_rows(rows, orig_rows, cols)) {
         launch_nvfp4_fast<0>(x, g, q, s, rows, orig_rows, cols, in_code, hf, nullptr, 0u, 0.0f, nullptr, st);
         return check_launch("quantize_nvfp4");
     }

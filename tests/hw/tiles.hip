@@ -84,3 +84,8 @@ extern "C" int ckh_skinny_forms(int nv) {
     return nv ? static_cast<int>(sizeof(kNvSkinny) / sizeof(kNvSkinny[0]))
               : static_cast<int>(sizeof(kMxSkinny) / sizeof(kMxSkinny[0]));
 }
+
+// Whether the NVFP4 quantizer with a given scale may take its fast path for this row padding.
+extern "C" int ckh_nv_quantize_fast_rows(int64_t rows, int64_t orig_rows, int64_t cols) {
+    return nv_quantize_fast_rows(rows, orig_rows, cols);
+}

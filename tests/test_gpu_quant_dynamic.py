@@ -75,3 +75,13 @@ def test_mxfp8_rows_padded(m, k, dtype, hip):
     q, s = ck.quantize_mxfp8(x, pad_32x=True)
     rq, rs = ref.quantize_mxfp8(x.cpu(), pad_32x=True)
     assert torch.equal(bits(q), bits(rq)) and torch.equal(bits(s), bits(rs))
+
+
+@pytest.mark.parametrize("hi_first", [True, False])
+@pytest.mark.parametrize("m", [1022, 1025])  # either side of the size from which the fast path serves them
+def test_nvfp4_rows_padded_given_scale(m, hi_first, hip):
+    x = _x(m * 3072, torch.bfloat16).reshape(m, 3072)
+    g = ck.amax_scale(x, 2688.0)
+    q, s = ck.quantize_nvfp4(x, g, pad_16x=True, hi_first=hi_first)
+    rq, rs = ref.quantize_nvfp4(x.cpu(), g.cpu(), pad_16x=True, hi_first=hi_first)
+    assert torch.equal(q.cpu(), rq) and torch.equal(bits(s), bits(rs))

@@ -1,5 +1,7 @@
 """GEMM kernels: facts that hold by construction, computed on the host from the kernels' own
 headers (tests/hw/tiles.hip)."""
+import ctypes
+
 import pytest
 
 from routes import library, route
@@ -63,3 +65,12 @@ def test_ragged_rows_shared_by_many_tiles(m, n, k, want):
     (200, 792, 8704, ("split", 7, 5, 2)), (146, 576, 7040, ("split", 7, 4, 2)), (200, 792, 4096, ("small", 64, 64))])
 def test_nvfp4_narrow_layers_with_long_k_split(m, n, k, want):
     assert route("nv", m, n, k) == want
+
+
+@pytest.mark.parametrize("rows,cols,fast", [(230, 1856, False), (1, 3072, False), (1023, 3072, False), (1025, 3072, True),
+                                            (16, 64, True), (240, 1856, True)])
+def test_nvfp4_quantize_of_padded_rows(rows, cols, fast):
+    """Small inputs padded in rows take the general kernel, which measured faster there."""
+    f = library().ckh_nv_quantize_fast_rows
+    f.argtypes = [ctypes.c_int64] * 3
+    assert f(-(-rows // 16) * 16, rows, cols) == fast
