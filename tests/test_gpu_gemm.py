@@ -11,6 +11,7 @@ import torch
 
 import comfy_kitchen as ck
 from oracle import eager_ref as ref
+from routes import route
 
 pytestmark = pytest.mark.gpu
 
@@ -44,11 +45,12 @@ def test_scaled_mm_mxfp8_vs_oracle(m, n, k, out_dtype, hip):
 
 
 def test_scaled_mm_one_round_grid_with_weight_prefetch(hip):
-    """256 x 18432 x 3072 runs as 144 half tiles, and the other 112 CUs run workgroups that
+    """256 x 25600 x 1024 runs as 200 half tiles, and the other 56 CUs run workgroups that
     read the weight ahead of the tiles (they write nothing): MXFP8 and per-tensor FP8
     against the oracle on the first and last 1024 output columns (swizzled scale rows of
     whole 128-row blocks slice like the weight)."""
-    m, n, k = 256, 18432, 3072
+    m, n, k = 256, 25600, 1024
+    assert route("mx", m, n, k) == ("tiles", 0, 100, 56)
     qx, sx, qw, sw = mx_operands(m, n, k, seed=77)
     got = ck.scaled_mm_mxfp8(qx.cuda(), qw.cuda(), sx.cuda(), sw.cuda(), out_dtype=torch.bfloat16).cpu()
     ta, tb = torch.tensor([0.5]), torch.tensor([3e-3])
@@ -89,6 +91,7 @@ def test_scaled_mm_mxfp8_half_tile_tail(out_dtype, with_bias, hip):
     """289 tiles of 256 x 256: 256 run as full tiles, the last 33 as 66 half-width tiles
     (partial ones at the right edge, one wholly past N)."""
     m, n, k = 4352, 4196, 128
+    assert route("mx", m, n, k) == ("tiles", 256, 33, 0)
     qx, sx, qw, sw = mx_operands(m, n, k, seed=21)
     bias = (torch.randn(n) * 2).float() if with_bias else None
     want = ref.scaled_mm_mxfp8_ref(qx, qw, sx, sw, bias=bias, out_dtype=torch.float32)
@@ -135,10 +138,11 @@ def test_scaled_mm_mxfp8_config4_full(hip):
                                    (28, 20000, 4160), (6, 18440, 288), (4, 24576, 3104)])
 def test_scaled_mm_mxfp8_skinny(m, n, k, out_dtype, hip):
     """At most 64 activation rows take the skinny kernel (a workgroup per 32 or 64 weight
-    rows, K split over its waves; configurations by M, boundaries 8 / 16 / 32 / 64, and from
-    9 rows on by N, boundaries 4096 / 8192 / 16384: waves per workgroup, weight tiles, and
-    32 or 64 activation rows staged in LDS or loaded as fragments): rows past M, columns
-    past N, K % 64 == 32, K past one chunk round and long K."""
+    rows, K split over its waves; configurations by M, boundaries 8 / 16 / 32 / 64, and by N,
+    boundaries 4096 / 8192 / 16384 / 24576: waves per workgroup, weight tiles, activation rows
+    staged in LDS) or, from 17 rows of wide layers with long K on, small tiles: rows past M,
+    columns past N, K % 64 == 32, K past one chunk round and long K."""
+    assert route("mx", m, n, k)[0] == "skinny" or m >= 17 and n >= 8192
     qx, sx, qw, sw = mx_operands(m, n, k, seed=m * 13 + n + k)
     want = ref.scaled_mm_mxfp8_ref(qx, qw, sx, sw, out_dtype=torch.float32)
     got = ck.scaled_mm_mxfp8(qx.cuda(), qw.cuda(), sx.cuda(), sw.cuda(), out_dtype=out_dtype)
@@ -180,15 +184,37 @@ def _mx_abi(qx, qw, sx, sw, out_dtype, ws):
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("m,n,k", [(256, 4096, 4096), (300, 2000, 4160), (129, 520, 4128), (65, 18432, 4096),
-                                   (512, 3072, 13824), (200, 2000, 2080)])
-def test_scaled_mm_mxfp8_split_k(m, n, k, out_dtype, hip):
-    """Grids of at most 128 tiles split K over more workgroups into a workspace, and a second
-    launch adds the partial tiles (fixed order) and runs the epilogue: against the oracle,
-    and against the same call with no workspace (whole-K half tiles), which differs only in
-    fp32 summation order.  Covers a last K range shorter than the others (and than one
-    group of 4 stages), K % 64 == 32, rows past M and columns past N."""
+                                   (200, 2000, 2080)])
+def test_scaled_mm_mxfp8_small_tiles_instead_of_split_k(m, n, k, out_dtype, hip):
+    """Shapes for which a workspace is offered and small tiles are faster: the same result with
+    and without it, against the oracle."""
     import comfy_kitchen.backends.hip as hb
 
+    assert route("mx", m, n, k)[0] == route("mx", m, n, k, workspace=False)[0] == "small"
+    nbytes = hb._lib.ckh_scaled_mm_workspace_bytes(m, n, k)
+    qx, sx, qw, sw = mx_operands(m, n, k, seed=m + 5 * n + k)
+    want = ref.scaled_mm_mxfp8_ref(qx, qw, sx, sw, out_dtype=torch.float32)
+    qx, sx, qw, sw = qx.cuda(), sx.cuda(), qw.cuda(), sw.cuda()
+    got = _mx_abi(qx, qw, sx, sw, out_dtype, torch.empty(nbytes, dtype=torch.uint8, device="cuda"))
+    assert rel_l2(got, want) <= REL_L2[out_dtype]
+    assert torch.equal(got, _mx_abi(qx, qw, sx, sw, out_dtype, None))
+    assert torch.equal(got, ck.scaled_mm_mxfp8(qx, qw, sx, sw, out_dtype=out_dtype))
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("m,n,k,form", [(300, 1001, 10016, (10, 16, 2)), (129, 520, 8224, (9, 16, 2)),
+                                        (65, 129, 6432, (7, 16, 2)), (512, 3072, 13824, (5, 44, 2)),
+                                        (1600, 2500, 7584, (3, 40, 4))])
+def test_scaled_mm_mxfp8_split_k(m, n, k, form, out_dtype, hip):
+    """Grids of at most 128 tiles with long K split it over more workgroups into a workspace
+    (as half tiles up to 64 tiles, else whole ones), and a second launch adds the partial tiles
+    (fixed order) and runs the epilogue: against the oracle, and against the same call with
+    no workspace (small tiles), which differs only in fp32 summation order.  Covers a last K
+    range shorter than the others (and than one group of 4 stages), K % 64 == 32, rows past M
+    and columns past N."""
+    import comfy_kitchen.backends.hip as hb
+
+    assert route("mx", m, n, k) == ("split", *form) and route("mx", m, n, k, workspace=False)[0] == "small"
     nbytes = hb._lib.ckh_scaled_mm_workspace_bytes(m, n, k)
     assert nbytes > 0
     qx, sx, qw, sw = mx_operands(m, n, k, seed=m + 5 * n + k)
@@ -204,10 +230,11 @@ def test_scaled_mm_mxfp8_split_k(m, n, k, out_dtype, hip):
     assert torch.equal(ck.scaled_mm_mxfp8(qx, qw, sx, sw, out_dtype=out_dtype), got)  # the wrapper splits too
 
 
-@pytest.mark.parametrize("bias_dtype", [torch.bfloat16, torch.float32])
-def test_scaled_mm_split_k_bias_and_per_tensor(bias_dtype, hip):
-    """The split-K reduce kernel's epilogue: bias, and the per-tensor FP8 mode."""
-    m, n, k = 200, 1000, 4096
+@pytest.mark.parametrize("bias_dtype", [torch.bfloat16, torch.float32, torch.float16])
+@pytest.mark.parametrize("m,n,k,halves", [(200, 1001, 10240, 2), (1600, 2500, 7584, 4)])
+def test_scaled_mm_split_k_bias_and_per_tensor(m, n, k, halves, bias_dtype, hip):
+    """The split-K reduce kernel's epilogue (half and whole tiles): bias, and the per-tensor FP8 mode."""
+    assert route("mx", m, n, k)[0] == "split" and route("mx", m, n, k)[3] == halves
     qx, sx, qw, sw = mx_operands(m, n, k, seed=31)
     bias = (torch.randn(n) * 2).to(bias_dtype)
     want = ref.scaled_mm_mxfp8_ref(qx, qw, sx, sw, bias=bias, out_dtype=torch.float32)
@@ -302,8 +329,8 @@ def test_scaled_mm_nvfp4_hi_first_invariance(m, hip):
                                    (2, 33, 32), (48, 13824, 128), (3, 160, 1536), (20, 8200, 256), (40, 8192, 96),
                                    (12, 40, 4096), (64, 3000, 5152), (17, 8100, 2080)])
 def test_scaled_mm_nvfp4_skinny(m, n, k, out_dtype, hip):
-    """At most 64 activation rows take the skinny NVFP4 kernel (a workgroup per 32 or 64
-    weight rows, K split over its waves in chunks of 256 elements, two chunks in flight per
+    """At most 64 activation rows take the skinny NVFP4 kernel (or, from 33 rows of wide layers
+    on, small tiles; a workgroup per 32 or 64 weight rows, K split over its waves in chunks of 256 elements, two chunks in flight per
     wave; configurations by M (boundaries 8 / 16 / 32 / 64) and, past 16 rows, by N (two weight
     tiles from N = 8192)): rows past M, columns past N, K % 64 == 32 (a half-used scale word),
     fewer chunks than waves, K past one chunk round and long K."""
@@ -318,11 +345,12 @@ def test_scaled_mm_nvfp4_skinny(m, n, k, out_dtype, hip):
 @pytest.mark.parametrize("n", [96, 8200])
 @pytest.mark.parametrize("m", [1, 8, 16, 24, 32, 48, 64])
 def test_scaled_mm_nvfp4_skinny_chunks_per_wave(m, n, k, hip):
-    """Every skinny configuration (by M, and one or two weight tiles by N) with 1, 5, 9 and
-    10 chunks of 256 elements, i.e. 4 waves holding 0 to 3 chunks each: the paths from the
+    """The skinny configurations (by M, and one or two weight tiles by N; from 33 rows with two
+    weight tiles only 224 columns, the rest are small tiles) with 1, 5, 9 and 10 chunks of 256 elements, i.e. 4 waves holding 0 to 3 chunks each: the paths from the
     prologue straight to the last step, through one loop iteration, and through the loop
     and the last step.  Each step's wait must cover its own chunk's LDS rows on every one of
     them (the staged activation rows included)."""
+    assert route("nv", m, n, k)[0] == ("small" if m > 32 and n == 8200 and k > 224 else "skinny")
     qx, sx, gx, qw, sw, gw = nv_operands(m, n, k, seed=m * 31 + n + k)
     want = ref.scaled_mm_nvfp4_ref(qx, qw, gx, gw, sx, sw, out_dtype=torch.float32)
     got = ck.scaled_mm_nvfp4(qx.cuda(), qw.cuda(), gx.cuda(), gw.cuda(), sx.cuda(), sw.cuda(),
@@ -359,17 +387,22 @@ def _nv_abi(qx, qw, gx, gw, sx, sw, out_dtype, ws, bias=None):
 
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("m,n,k", [(256, 4096, 2048), (300, 2000, 4160), (129, 520, 5152), (65, 13824, 2048),
-                                   (300, 8500, 4096)])
-def test_scaled_mm_nvfp4_split_k(m, n, k, out_dtype, hip):
-    """Small NVFP4 tile grids split K into a workspace, as half tiles (at most 64 tiles) or
-    whole tiles (300 x 8500: 68 tiles, 3 ranges) (ranges of ks 256-element groups, odd
+@pytest.mark.parametrize("m,n,k,form", [(300, 1001, 10016, (10, 4, 2)), (129, 520, 8224, (7, 5, 2)),
+                                        (65, 129, 6976, (7, 4, 2)), (300, 2000, 9248, (8, 5, 2)),
+                                        (1600, 2500, 4128, (3, 6, 4)), (256, 4096, 2048, None),
+                                        (300, 2000, 4160, None), (129, 520, 5152, None), (65, 13824, 2048, None),
+                                        (300, 8500, 4096, None)])
+def test_scaled_mm_nvfp4_split_k(m, n, k, form, out_dtype, hip):
+    """Small NVFP4 tile grids with long K split it into a workspace, as half tiles (at most 64
+    tiles) or whole tiles (1600 x 2500: 70 tiles, 3 ranges) (ranges of ks 256-element groups, odd
     counts and odd starts included, and a last range shorter than the others, down to one
     group; K % 256 != 0, rows past M, columns past N), against the oracle and against the
-    unsplit call (fp32 summation order only; an odd group count there too); the reduce
-    kernel applies alpha and bias."""
+    unsplit call (small tiles: fp32 summation order only); the reduce kernel applies alpha and
+    bias.  form None: a workspace is offered, but the small tiles are faster and leave it."""
     import comfy_kitchen.backends.hip as hb
 
+    assert route("nv", m, n, k, workspace=False)[0] == "small"
+    assert route("nv", m, n, k) == ("split", *form) if form else route("nv", m, n, k)[0] == "small"
     nbytes = hb._lib.ckh_scaled_mm_nvfp4_workspace_bytes(m, n, k)
     assert nbytes > 0
     qx, sx, gx, qw, sw, gw = nv_operands(m, n, k, seed=m + 7 * n + k)
@@ -405,8 +438,9 @@ def test_scaled_mm_nvfp4_workspace_bytes(hip):
 def test_scaled_mm_nvfp4_half_tile_tail(out_dtype, with_bias, hip):
     """289 tiles of 256 x 256: 256 run as full tiles, the last 33 as 66 half-width tiles
     (partial ones at the right edge, one wholly past N); and a one-round grid without a
-    workspace, all of it half tiles."""
+    split, all of it half tiles."""
     m, n, k = 4352, 4196, 320
+    assert route("nv", m, n, k) == ("tiles", 256, 33, 0)
     qx, sx, gx, qw, sw, gw = nv_operands(m, n, k, seed=23)
     bias = (torch.randn(n) * 0.1).float() if with_bias else None
     want = ref.scaled_mm_nvfp4_ref(qx, qw, gx, gw, sx, sw, bias=bias, out_dtype=torch.float32)
@@ -417,15 +451,16 @@ def test_scaled_mm_nvfp4_half_tile_tail(out_dtype, with_bias, hip):
     # The tiles are taken in groups of 6 tile rows, each group column by column: tiles
     # 256..288 lie in the last group (tile rows 12..16) at tile columns 10..16.
     assert rel_l2(got[12 * 256:, 10 * 256:], want[12 * 256:, 10 * 256:]) <= REL_L2[out_dtype]
-    # 3 x 5 tiles, no split (K = 1024: 4 groups), as 30 half tiles
-    qx, sx, gx, qw, sw, gw = nv_operands(700, 1100, 1024, seed=24)
+    # 3 x 36 tiles, no split (K = 320: 2 groups) and too wide for small tiles, as 216 half tiles
+    assert route("nv", 700, 9000, 320, workspace=False) == ("tiles", 0, 108, 0)
+    qx, sx, gx, qw, sw, gw = nv_operands(700, 9000, 320, seed=24)
     want = ref.scaled_mm_nvfp4_ref(qx, qw, gx, gw, sx, sw, out_dtype=torch.float32)
     got = _nv_abi(qx.cuda(), qw.cuda(), gx.cuda(), gw.cuda(), sx.cuda(), sw.cuda(), out_dtype, None)
     assert rel_l2(got, want) <= REL_L2[out_dtype]
 
 
 def test_scaled_mm_nvfp4_skinny_matches_tile_rows(hip):
-    """Rows of a 65-row product (tile kernel) against the same rows computed alone (skinny
+    """Rows of a 65-row product (small tiles) against the same rows computed alone (skinny
     kernel): both sum exact fp16 products in fp32 MFMAs, so they agree to fp32 rounding."""
     qx, sx, gx, qw, sw, gw = nv_operands(65, 512, 2048, seed=44)
     full = ck.scaled_mm_nvfp4(qx.cuda(), qw.cuda(), gx.cuda(), gw.cuda(), sx.cuda(), sw.cuda(), out_dtype=torch.float32)

@@ -42,6 +42,11 @@ MX = [  # 17-64 rows: the skinny forms that the small tiles leave
     (29, 20401, 4128, ("skinny", 4, 1, 1, 32, 0)), (32, 24579, 96, ("skinny", 2, 2, 1, 32, 0)),
     (52, 16403, 544, ("skinny", 2, 1, 2, 64, 0)), (33, 24576, 1216, ("skinny", 2, 1, 2, 64, 0)),
     (64, 32771, 160, ("skinny", 2, 2, 2, 64, 0)), (40, 33001, 672, ("skinny", 2, 2, 2, 64, 0)),
+    # split-K in half and in whole tiles; whole tiles, the last round whole or in halves; one round
+    # of half tiles with weight-prefetch workgroups beside it
+    (300, 1001, 10016, ("split", 10, 16, 2)), (512, 3073, 13824, ("split", 4, 56, 2)),
+    (130, 17001, 6432, ("split", 3, 36, 4)), (4400, 5541, 96, ("tiles", 396, 0, 0)),
+    (4352, 4099, 160, ("tiles", 256, 33, 0)), (700, 9003, 224, ("tiles", 0, 108, 40)),
 ]
 
 
@@ -53,7 +58,9 @@ def test_mxfp8_and_fp8(m, n, k, want, hip):
     qw, sw = ck.quantize_mxfp8(w)
     product = ck.dequantize_mxfp8(qx, sx, torch.float32) @ ck.dequantize_mxfp8(qw, sw, torch.float32).t()
     _check(lambda b, o: ck.scaled_mm_mxfp8(qx, qw, sx, sw, bias=b, out_dtype=o), product, bias, m, n)
-    ta, tb = torch.full((1,), 0.37, device="cuda"), torch.full((1,), 0.021, device="cuda")
+    # (codes of about 150 in the root mean square: sums of about 150^2 sqrt(K) = 2.6e6 at K = 13824, and
+    # six times that, times 7.8e-4, is 1.2e4, inside f16's 65504)
+    ta, tb = torch.full((1,), 0.37, device="cuda"), torch.full((1,), 0.0021, device="cuda")
     product = (qx.float() @ qw.float().t()) * (ta * tb)
     _check(lambda b, o: ck.scaled_mm_fp8(qx, qw, ta, tb, bias=b, out_dtype=o), product, bias, m, n)
 
@@ -61,6 +68,13 @@ def test_mxfp8_and_fp8(m, n, k, want, hip):
 NV = [  # 33-64 rows with two weight tiles per workgroup: short ragged K, long K, N past one round of small tiles
     (50, 9233, 928, ("skinny", 4, 2, 2, 0, 0)), (33, 8193, 96, ("skinny", 4, 2, 2, 0, 0)),
     (64, 8205, 8224, ("skinny", 4, 2, 2, 0, 0)), (40, 32771, 544, ("skinny", 4, 2, 2, 0, 0)),
+    # the same with 1, 5, 9 and 10 chunks of 256 elements: its 4 waves hold 0 to 3 each
+    (64, 32800, 224, ("skinny", 4, 2, 2, 0, 0)), (48, 32800, 1280, ("skinny", 4, 2, 2, 0, 0)),
+    (64, 32801, 2304, ("skinny", 4, 2, 2, 0, 0)), (64, 32800, 2336, ("skinny", 4, 2, 2, 0, 0)),
+    # split-K in half and in whole tiles; tiles as for MXFP8
+    (300, 1001, 10016, ("split", 10, 4, 2)), (130, 17001, 6432, ("split", 3, 9, 4)),
+    (4400, 5541, 96, ("tiles", 396, 0, 0)), (4352, 4099, 160, ("tiles", 256, 33, 0)),
+    (700, 9003, 224, ("tiles", 0, 108, 0)),
 ]
 
 

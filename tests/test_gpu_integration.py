@@ -11,6 +11,7 @@ import torch
 import torch.nn.functional as F
 
 from comfy_kitchen.tensor import QuantizedTensor
+from routes import route
 
 pytestmark = pytest.mark.gpu
 
@@ -38,22 +39,18 @@ def _input(seed, rows=64, cols=256):
     return torch.randn(rows, cols, device="cuda", generator=g).bfloat16()
 
 
-# (rows, in_features, hidden, out_features): 64 rows run the skinny GEMM kernels; 256 rows
-# against K = 4096 and 512 outputs split K over a workspace (two launches per GEMM)
-SHAPES = [(64, 256, 512, 128), (256, 4096, 512, 128)]
+# (rows, in_features, hidden, out_features): 64 rows run the skinny GEMM kernels, 256 rows small
+# tiles, and 256 rows against K = 10240 and 512 outputs split K over a workspace (two launches)
+SHAPES = [(64, 256, 512, 128), (256, 4096, 512, 128), (256, 10240, 512, 128)]
 
 
-@pytest.mark.parametrize("shape", SHAPES, ids=["skinny", "split_k"])
+@pytest.mark.parametrize("shape", SHAPES, ids=["skinny", "small_tiles", "split_k"])
 @pytest.mark.parametrize("layout", LAYOUTS)
 def test_graph_capture_replay(layout, shape, hip):
     rows, fin, hidden, fout = shape
     model = TwoLayer(layout, in_features=fin, hidden=hidden, out_features=fout)
-    if shape[0] == 256:
-        import comfy_kitchen.backends.hip as hb
-
-        fn = ("ckh_scaled_mm_nvfp4_workspace_bytes" if layout == "TensorCoreNVFP4Layout"
-              else "ckh_scaled_mm_workspace_bytes")
-        assert getattr(hb._lib, fn)(rows, hidden, fin) > 0  # the first GEMM splits K
+    fmt = "nv" if layout == "TensorCoreNVFP4Layout" else "mx"
+    assert route(fmt, rows, hidden, fin)[0] == {(64, 256): "skinny", (256, 4096): "small", (256, 10240): "split"}[rows, fin]
     x = _input(1, rows, fin)
     with torch.no_grad():
         want = model(x)
