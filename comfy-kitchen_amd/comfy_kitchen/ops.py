@@ -37,25 +37,37 @@ try:
     _profiling = _C._autograd._profiler_enabled
     _is_zero = torch.Tensor._is_zerotensor
     _forward_ad._current_level
-    _has_kernel = _C._dispatch_has_kernel_for_any_dispatch_key
-    # Every key at which the dispatcher could find a kernel for plain GPU tensors ahead of, or in
-    # place of, the custom op's own (which it holds under alias keys, so none of these is set by it)
-    _KERNEL_KEYS = _C.DispatchKeySet(_C.DispatchKey.CUDA)
-    for _key in ("AutocastCUDA", "AutogradCUDA", "ADInplaceOrView"):
-        _KERNEL_KEYS = _KERNEL_KEYS.add(getattr(_C.DispatchKey, _key))
+    _registered = torch.library._impls  # "namespace/op/key" of every kernel registered from Python
+    _registered.isdisjoint
     _OBSERVABLE = True
-except (AttributeError, TypeError):
+except AttributeError:
     # A torch that lacks one of these (several are not public) gives no way to tell whether
     # something looks at the op: every call takes the custom op then.
     _OBSERVABLE = False
+
+# Every key at which the dispatcher could find a kernel for plain GPU tensors ahead of, or in place
+# of, the custom op's own (which it holds under alias keys, so none of these is set by it).
+_KERNEL_KEYS = ("CUDA", "AutocastCUDA", "AutogradCUDA", "ADInplaceOrView")
+
+
+class _Kernels(dict):
+    """op name -> the entries that a program's own kernels for it make in torch's list."""
+
+    def __missing__(self, op: str) -> frozenset:
+        entries = self[op] = frozenset(f"comfy_kitchen/{op}/{key}" for key in _KERNEL_KEYS)
+        return entries
+
+
+_kernels = _Kernels()
 
 
 def untouched(op: str) -> bool:
     """Whether no program has registered a kernel of its own (torch.library, an autocast rule,
     the custom op's register_kernel) for GPU tensors on `comfy_kitchen::<op>`: one that has
-    expects `ck.*` calls to reach it.  (A kernel put in place of the op's default one under the
-    default's own alias key is not seen.)  About 0.7 us a call."""
-    return not _has_kernel("comfy_kitchen::" + op, _KERNEL_KEYS)
+    expects `ck.*` calls to reach it.  (Not seen: a kernel registered in C++, and one put in
+    place of the op's default under the default's own alias key.)  About 0.15 us a call; asking
+    the dispatcher itself took 0.7."""
+    return _registered.isdisjoint(_kernels[op])
 
 
 def direct(*tensors) -> bool:
@@ -63,8 +75,9 @@ def direct(*tensors) -> bool:
     looks at or transforms the op (compilation and tracing, dispatch and function modes, vmap
     and the other function transforms, forward-mode AD, the profiler), the first tensor is on
     the GPU, and every tensor is a plain one that no gradient is asked of and whose memory holds
-    its values (a lazily negated or conjugated view's does not, and a zero tensor has none: the
-    dispatcher makes them plain before the custom op's kernel sees them).  Anything else takes
+    its values (a lazily negated view's does not, and a zero tensor has none: the dispatcher makes
+    them plain before the custom op's kernel sees them; complex tensors, which alone can be lazily
+    conjugated, no backend function takes).  Anything else takes
     the custom op, which serves all of these.  The custom op's Python layers cost more than the
     call itself: on a 77 x 4096 tensor quantize_per_tensor_fp8 and dequantize_per_tensor_fp8
     took 20 us each from Python for 2.7 us on the GPU."""
@@ -80,7 +93,7 @@ def direct(*tensors) -> bool:
             continue
         if type(t) is not _Tensor and type(t) is not _Parameter or grad and t.requires_grad:
             return False
-        if t.is_neg() or t.is_conj() or _is_zero(t):
+        if t.is_neg() or _is_zero(t):
             return False
     return True
 
@@ -111,8 +124,10 @@ def _(x, scale, output_dtype_code):
 def _quantize_fp8_dynamic(x: torch.Tensor, divisor: float, output_type: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
     """The fused call where one backend serves it and the quantizer; else the two calls it stands
     for, each from the backend that the program has chosen for it."""
-    if registry.serves_both("quantize_per_tensor_fp8", "quantize_fp8_dynamic", {"x": x, "output_type": output_type}):
-        return _dispatch("quantize_fp8_dynamic", x=x, divisor=divisor, output_type=output_type)
+    fused = registry.shared_implementation("quantize_fp8_dynamic", "quantize_per_tensor_fp8",
+                                           {"x": x, "output_type": output_type})
+    if fused is not None:
+        return fused(x=x, divisor=divisor, output_type=output_type)
     scale = _dispatch("amax_scale", x=x, divisor=divisor)
     return _dispatch("quantize_per_tensor_fp8", x=x, scale=scale, output_type=output_type), scale
 

@@ -234,13 +234,16 @@ class BackendRegistry:
             return None
         return name if self._accepts(slot.table[func_name], kwargs) else None
 
-    def serves_both(self, func_name: str, other: str, kwargs: Mapping[str, Any]) -> bool:
-        """Whether one backend would be chosen for both functions with these arguments."""
+    def shared_implementation(self, func_name: str, other: str, kwargs: Mapping[str, Any]) -> Callable | None:
+        """The callable serving `func_name` if the same backend would be chosen for `other` with
+        these arguments, else None."""
         try:
-            return ((self._first_choice(func_name, kwargs) or self.get_capable_backend(func_name, kwargs))
-                    == (self._first_choice(other, kwargs) or self.get_capable_backend(other, kwargs)))
+            name = self._first_choice(func_name, kwargs) or self.get_capable_backend(func_name, kwargs)
+            if name != (self._first_choice(other, kwargs) or self.get_capable_backend(other, kwargs)):
+                return None
         except NoCapableBackendError:
-            return False
+            return None
+        return getattr(self._slots[name].module, func_name)
 
     def _candidates(self) -> Iterator[tuple[str, bool]]:
         forced = self._forced()

@@ -133,7 +133,7 @@ def test_lazy_views_take_the_custom_op(hip):
     scale = z.imag.reshape(1)
     assert neg.is_neg() and scale.is_neg()
     zeros = torch._efficientzerotensor((4, 128), dtype=torch.bfloat16, device="cuda")
-    assert not direct(neg) and not direct(x, scale) and not direct(zeros) and not direct(z)
+    assert not direct(neg) and not direct(x, scale) and not direct(zeros)
     for a, b in zip(ck.quantize_mxfp8(neg), ck.quantize_mxfp8(-x)):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
     plain = torch.full((1,), 0.25, device="cuda")
@@ -164,6 +164,24 @@ def test_registered_kernels_are_seen(op):
         assert untouched(op)
 
 
+def test_custom_op_registrations_are_seen():
+    """register_kernel and register_autocast last as long as the process, so in one of its own."""
+    code = f"""
+import sys
+sys.path.insert(0, {str(PACKAGE)!r})
+import torch
+import comfy_kitchen.ops as ops
+assert ops.untouched("quantize_fp8") and ops.untouched("quantize_mxfp8") and ops.untouched("apply_rope1")
+ops.quantize_fp8.register_kernel("cuda")(lambda x, scale, code: x)
+torch.library.register_kernel("comfy_kitchen::apply_rope1", "cuda", lambda x, f: x)
+ops.quantize_mxfp8.register_autocast("cuda", torch.float32)
+assert not ops.untouched("quantize_fp8") and not ops.untouched("quantize_mxfp8") and not ops.untouched("apply_rope1")
+print("ok")
+"""
+    run = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert run.stdout.strip() == "ok", run.stderr
+
+
 @pytest.mark.gpu
 def test_registered_kernel_serves_the_call(hip):
     x, scale = torch.randn(4, 32, device="cuda").bfloat16(), torch.ones(1, device="cuda")
@@ -184,7 +202,6 @@ def test_registered_kernel_serves_the_call(hip):
 @pytest.mark.parametrize("holder,name", [("torch._C._functorch", "peek_interpreter_stack"),
                                          ("torch._C._autograd", "_profiler_enabled"),
                                          ("torch._C", "_get_tracing_state"),
-                                         ("torch._C", "_dispatch_has_kernel_for_any_dispatch_key"),
                                          ("torch.autograd.forward_ad", "_current_level")])
 def test_torch_without_a_probe_takes_the_custom_op(holder, name):
     """Where torch lacks one of the names the shortcut asks, the package imports and every call
