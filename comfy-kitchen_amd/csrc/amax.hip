@@ -29,10 +29,11 @@ namespace am {
 
 constexpr int kThreads = 256;
 constexpr int kUnroll = 16;                // 16-byte loads in flight per thread, large tensors
-// Below kSpreadBlocks workgroups' worth of work at kUnroll loads a thread, the tensor is
-// spread thinner, kUnrollSmall loads a thread: 256 x 3072 bf16 ran on 24 workgroups in 9.5 us
-// and 256 x 5120 on 40 in 9.7 us, waiting out the loads' issue on a few CUs; spread, the
-// NVFP4 dynamic quantize of 256 x 5120 takes 6 us less.
+// A tensor of at most kSpreadBlocks workgroups' worth of work at kUnrollSmall loads a thread (4 MB)
+// is spread thinner than kUnroll: 256 x 3072 bf16 ran on 24 workgroups in 9.5 us and 256 x 5120 on
+// 40 in 9.7 us, waiting out the loads' issue on a few CUs; spread, the NVFP4 dynamic quantize of
+// 256 x 5120 takes 6 us less.  (Just above 4 MB the grid falls from 512 workgroups to 65; a tensor
+// there takes what it took before, 6.2 us at 6 MB.)
 constexpr int kUnrollSmall = 2;
 constexpr int kSpreadBlocks = 512;
 constexpr int kMaxBlocks = CKH_AMAX_WORKSPACE_BYTES / 4;  // one partial word per workgroup

@@ -320,8 +320,8 @@ __device__ __forceinline__ float tensor_scale(const float* a, const float* b) { 
 // (raw bits; zeros past N, for a bias never read out of range) before the tile's operand
 // loads are issued and writes it after them, so neither waits for the other; the caller's
 // next barrier publishes it.  Read column by column from memory in the epilogue, the bias's
-// 2-byte loads cost 48 of 207 us on 4608 x 12288 x 3072 (MXFP8) and about 100 of 912 us on
-// 8192 x 13824 x 5120 (NVFP4).
+// 2-byte loads cost 65 of 216 us on 4608 x 12288 x 3072 (MXFP8; 6 of 154 now) and 120 of 945 us on
+// 8192 x 13824 x 5120 (NVFP4; 7 of 830 now).
 __device__ __forceinline__ uint32_t load_bias_bits(const void* bias, int code, int n, int N) {
     if (n >= N) return 0u;
     return code == CKH_F32 ? static_cast<const uint32_t*>(bias)[n] : static_cast<const uint16_t*>(bias)[n];

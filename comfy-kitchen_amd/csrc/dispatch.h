@@ -168,9 +168,10 @@ inline int mx_small_tile(int M, int N, int K, const SplitPlan& sp, int cus) {
 // fill and the one workgroup per CU.  Measured against the skinny kernel on 3,600 shapes, graph-timed
 // both with every call's weight read anew and with one weight that stays in the caches (small tile /
 // skinny, us, anew; the same kept):
-//   33-64 rows  64 x 64 at any K: 64 x 8192 x 12288 37.7 / 46.0; the mean of all 0.91; 0.72 kept.
-//               64 x 128 from K = 1280 on (640 above N = 24576): 52 x 19808 x 512 7.4 / 5.9; 6.5 / 5.2,
-//               57 x 17328 x 1024 9.6 / 8.1; 8.2 / 7.6, 64 x 24576 x 5120 33.6 / 40.3.
+//   33-64 rows  64 x 64 at any K: 64 x 8192 x 12288 40.5 / 43.5; 25.2 / 42.8, 48 x 12288 x 3072 13.1 /
+//               15.2; 10.1 / 14.1; the mean of all 0.91; 0.72.  64 x 128 from K = 1280 on (640 above N =
+//               24576): 52 x 19808 x 512 7.4 / 5.9; 6.5 / 5.2, 57 x 17328 x 1024 9.6 / 8.1; 8.2 / 7.6,
+//               64 x 24576 x 5120 33.6 / 37.6; 24.0 / 36.8.
 //   17-32 rows  they gain only where the weight is in the caches, so they stay where they are level
 //               otherwise (in the mean 1.00; 0.82 kept): 64 x 64 above N = 10240 from K = 3072 on (25 x
 //               8688 x 1024 6.8 / 5.2; 5.9 / 4.2, 32 x 9688 x 2624 11.6 / 10.6; 8.4 / 6.6); 64 x 128
@@ -309,15 +310,15 @@ constexpr NvSmallTile kNvSmall[] = {{64, 64, 5.0, 0.66}, {64, 128, 6.2, 0.8}, {1
 // the same shapes: split-K 14 + 2.6 per group of a K range in half tiles (4.5 in whole tiles),
 // half tiles without a split 8.5 + 2.4 per group.  Over 2,780 more shapes of 65-1400 rows the small
 // tiles took 0.55 of the time and one of 2,250 choices was more than 3% slower (0.62 per line of 64 x
-// 64 tiles chose them for long K too: 200 x 792 x 8704 24.2 against 22.1 us split).  256 x 13824 x
-// 5120 50.4 -> 41.9 us, 300 x 4096 x 4096 33.5 -> 19.7, 128 x 3072 x 3072 21.7 -> 12.5, 65 x 5120 x
-// 2048 22.4 -> 10.3.  Rows that do not start on a cache line (K not a multiple of 256) take 6% longer
+// 64 tiles chose them for long K too: 200 x 792 x 8704 24.2 against 22.1 us split).  Weight read anew,
+// 256 x 13824 x 5120 49.0 -> 39.4 us, 300 x 4096 x 4096 32.7 -> 18.5, 128 x 3072 x 3072 20.7 -> 12.1, 65 x
+// 5120 x 2048 21.2 -> 9.8.  Rows that do not start on a cache line (K not a multiple of 256) take 6% longer
 // (60 more shapes: 1.08 x the estimate in the mean; 239 x 8824 x 4768 38.6, split-K 37.9).
 // At most 64 rows: 64 x 64 or 64 x 128 from 33 rows and N = 8192 on, K up to 8192, and from K = 1024
-// on where rows do not start on a cache line (graph-timed, against the skinny kernel: 48 x 8192 x 3072
-// 12.2 / 14.3 us, 64 x 12288 x 5120 17.7 / 20.8, 33 x 18432 x 3072 16.3 / 21.5; with 32 rows 32 x 12288
-// x 3072 12.7 / 11.5, with K = 12288 33 x 8192 32.5 / 30.9; 50 x 9232 x 928 8.7 / 7.1 and, over 190
-// such shapes, 1.06 with the weight read anew and 1.00 with it in the caches).
+// on where rows do not start on a cache line (graph-timed against the skinny kernel, weight read anew: 64
+// x 24576 x 5120 26.0 / 33.3 us, 33 x 18432 x 3072 16.9 / 20.9, 64 x 12288 x 5120 18.3 / 18.7, 48 x 8192 x
+// 3072 12.8 / 12.1; 0.91 in the mean of 1,400 shapes; with 32 rows 32 x 12288 x 3072 12.7 / 11.5, with K =
+// 12288 33 x 8192 32.5 / 30.9; 50 x 9232 x 928 8.7 / 7.1 and 1.06 over 190 such shapes).
 inline int nv_small_tile(int M, int N, int K, const SplitPlan& sp, int cus) {
     if (M <= kSkinnyMaxM) {
         if (M <= 32 || N < 8192 || K > 8192 || (K % 256 && K < 1024)) return -1;

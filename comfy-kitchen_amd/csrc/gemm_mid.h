@@ -2,17 +2,22 @@
 // hundred activation rows (from 17 on in wide layers): grids whose 256 x 256 tiles would leave
 // CUs idle.
 //
-// What bounds it: a CU takes in at most about 57 GB/s of operand lines when they come from HBM
-// (a streaming kernel on 8 CUs; 44-50 with 80 loading, 23-27 with all 256, where HBM itself is
-// the limit) and about 90 GB/s from the L2, with loads to registers or to LDS, at any number of
-// loads in flight beyond 64 KB.  Lines count, not bytes: with K not a multiple of 128 a row's
-// piece of a stage lies in two of them, and a stage takes up to 1.45 x as long.  A tile's time is therefore its (TM + TN) K operand bytes at that rate, about 0.5 us per
-// 128-byte stage of a 128 x 96 tile, and what helps is every CU busy with the smallest tile
-// that still fits the grid on the CUs at once; the matrix cores (0.2 us of those 0.5) and the
-// prefetch depth (3 to 6 stages measured equal) do not matter.  Measured against the
-// 256 x 256 kernel's half tiles and split-K over 200 shapes of 65-1333 rows (graph-timed,
-// rotated operands): 1.3 x faster on average, e.g. 256 x 9216 x 3072 19.4 against 25.5 us,
-// 512 x 5120 x 5120 28.0 / 32.2, 1024 x 3072 x 3072 19.1 / 29.0, 256 x 3072 x 3072 10.8 / 19.2.
+// What bounds it: the rate at which a CU takes in its operand lines.  512 x 5120 x 5120 MXFP8 on 216
+// tiles of 128 x 96: 1.18 MB a CU in 24.7 us, 48 GB/s, with the weight in the memory-side cache, and
+// in 30.0 us, 39 GB/s, with it read from HBM; 79% of the lines hit the L2 either way, and the matrix
+// cores are busy 27% and 20% of the time (counters).  A kernel that only loads reached 57 GB/s per CU
+// from HBM with 8 CUs loading, 44-50 with 80 and 23-27 with all 256, where HBM itself is the limit,
+// and about 90 from the L2, with loads to registers or to LDS, at any number of loads in flight
+// beyond 64 KB.  Lines count, not bytes: with K not a multiple of 128 a row's piece of a stage lies
+// in two of them, and a stage takes up to 1.45 x as long.  So a tile's time follows its (TM + TN) K
+// operand bytes, about 0.5 us per 128-byte stage of a 128 x 96 tile, and what helps is every CU busy
+// with the smallest tile that still fits the grid on the CUs at once; the matrix cores (0.2 us of
+// those 0.5) and the prefetch depth (3 to 6 stages measured equal) do not matter.
+//
+// Against the 256 x 256 kernel's half tiles and split-K (graph-timed MXFP8, us; one weight that stays in
+// the caches, then weights read anew): 256 x 9216 x 3072 16.2 / 22.5, 20.5 / 24.1; 512 x 5120 x 5120 23.4
+// / 28.8, 29.8 / 30.4; 1024 x 3072 x 3072 16.8 / 25.2, 16.7 / 25.3; 256 x 3072 x 3072 9.1 / 17.5, 9.5 /
+// 17.6.  Six layers of 512 x 5120 x 5120 in turn, whose 157 MB the caches partly hold, run level.
 //
 // A 512-thread workgroup computes a TM x TN tile.  K advances one 128-byte line per row and
 // stage; the two K groups of four waves each take one of a stage's two 64-wide MFMA steps, so
@@ -294,7 +299,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mid_kernel(Args p) {
     const uint32_t voff = static_cast<uint32_t>((wave * 8 + (lane >> 3)) * p.K + cb);
     const uint32_t rowstep = 64u * p.K;
     // scale words: 512-byte chunk (128-row block, stage) of the swizzled tensor, two blocks
-    // per operand (the second only for 256-row tiles); wave w loads quarter w % 4 of the
+    // per operand (a 96-, 160- or 192-wide tile's weight rows can straddle two); wave w loads quarter w % 4 of the
     // activation's (w < 4) or the weight's 1 KB
     const int sq = (wave & 3) * 64 + lane;  // word of the operand's two blocks
     const __amdgpu_buffer_rsrc_t rs = wave < 4 ? rsa : rsb;

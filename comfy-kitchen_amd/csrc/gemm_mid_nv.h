@@ -13,7 +13,9 @@
 // and 16-wide substep.  More K groups of fewer waves give each wave a larger part of the tile
 // and so fewer decodes per MFMA: 128 x 128 with 2 groups (64 x 64 a wave) spends 8 decode
 // instructions per MFMA and took 46.1 us on 256 x 13824 x 5120, with 4 groups (128 x 64 a wave)
-// 6 and 41.9 us; with all codes zero, i.e. without the power limit, 35.4.
+// 6 and 41.9 us; with all codes zero, i.e. without the power limit, 35.4.  (On another card, with the
+// weight kept in the caches / read anew: 37.0 / 39.4, the 256 x 256 kernel's split-K 45.2 / 49.0; the
+// matrix cores are busy 46% of the time.)
 #pragma once
 
 #include "gemm_mid.h"
