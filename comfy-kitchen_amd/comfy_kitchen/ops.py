@@ -35,7 +35,7 @@ try:
     _dispatch_modes, _function_modes = _C._len_torch_dispatch_stack, _C._len_torch_function_stack
     _transforms, _tracing = _C._functorch.peek_interpreter_stack, _C._get_tracing_state
     _profiling = _C._autograd._profiler_enabled
-    _is_zero = torch.Tensor._is_zerotensor
+    torch.Tensor._is_zerotensor
     _forward_ad._current_level
     _registered = torch.library._impls  # "namespace/op/key" of every kernel registered from Python
     _registered.isdisjoint
@@ -84,18 +84,16 @@ def direct(*tensors) -> bool:
     if (not _OBSERVABLE or _is_compiling() or _dispatch_modes() or _function_modes() or _transforms() is not None
             or _tracing() is not None or _profiling() or _forward_ad._current_level >= 0):
         return False
-    first = tensors[0]
-    if type(first) is not _Tensor and type(first) is not _Parameter or not first.is_cuda:
-        return False
     grad = torch.is_grad_enabled()
     for t in tensors:
-        if t is None:
-            continue
-        if type(t) is not _Tensor and type(t) is not _Parameter or grad and t.requires_grad:
+        kind = type(t)
+        if kind is _Tensor or kind is _Parameter:
+            if grad and t.requires_grad or t.is_neg() or t._is_zerotensor():
+                return False
+        elif t is not None:
             return False
-        if t.is_neg() or _is_zero(t):
-            return False
-    return True
+    first = tensors[0]
+    return first is not None and first.is_cuda
 
 
 # --------------------------------------------------------------- per-tensor FP8

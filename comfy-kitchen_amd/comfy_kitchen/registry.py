@@ -235,15 +235,17 @@ class BackendRegistry:
         return name if self._accepts(slot.table[func_name], kwargs) else None
 
     def shared_implementation(self, func_name: str, other: str, kwargs: Mapping[str, Any]) -> Callable | None:
-        """The callable serving `func_name` if the same backend would be chosen for `other` with
-        these arguments, else None."""
+        """The callable serving `func_name` if the backend chosen for it with these arguments
+        serves `other` too, and no backend that comes before it does; else None."""
+        name = self._first_choice(func_name, kwargs)
+        if name is not None:  # first in the order: nothing comes before it
+            slot = self._slots[name]
+            return getattr(slot.module, func_name) if other in slot.table else None
         try:
-            name = self._first_choice(func_name, kwargs) or self.get_capable_backend(func_name, kwargs)
-            if name != (self._first_choice(other, kwargs) or self.get_capable_backend(other, kwargs)):
-                return None
+            name = self.get_capable_backend(func_name, kwargs)
+            return getattr(self._slots[name].module, func_name) if name == self.get_capable_backend(other, kwargs) else None
         except NoCapableBackendError:
             return None
-        return getattr(self._slots[name].module, func_name)
 
     def _candidates(self) -> Iterator[tuple[str, bool]]:
         forced = self._forced()

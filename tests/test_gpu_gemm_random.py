@@ -1,11 +1,12 @@
 """Seeded random GEMM shapes against the CPU oracle, both block formats.
 
-The GEMM launchers choose among many forms by M, N and K: skinny kernels (waves, weight
-tiles and staged activation rows by M and N), small tiles of seven shapes for up to some 1,300
-rows, whole tiles, half tiles for a last or only round, weight-prefetch workgroups on idle CUs, and split-K in full or half tiles with
-ranges of any length.  Each case draws a shape from ranges that straddle those choices, so
-the suite crosses their boundaries in combinations the hand-picked shapes do not; a few
-larger grids with short K cover the whole-tile rounds and their last rounds.
+The GEMM launchers choose among many forms by M, N and K: skinny kernels (waves, weight tiles
+and staged activation rows by M and N), small tiles of seven shapes for up to some 1,300 rows,
+whole tiles, half tiles for a last or only round, weight-prefetch workgroups on idle CUs, and
+split-K in full or half tiles with ranges of any length. Each case draws a shape from ranges
+that straddle those choices, so the suite crosses their boundaries in combinations the hand-
+picked shapes do not; a few larger grids with short K cover the whole-tile rounds and their last
+rounds.
 """
 import random
 
